@@ -103,8 +103,8 @@ struct BatchWs {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<unsigned char> key;          // descriptor bytes the graph was captured for
-    std::map<std::string, int> tuned;        // group shape signature -> waves per workgroup
-    int groups = 0, nodes = 0, replayed = 0, nw = 0, blocks = 0;
+    std::map<std::string, int> tuned;        // group shape signature -> particles per work item
+    int groups = 0, nodes = 0, replayed = 0, cp = 0, blocks = 0;
     float cand_ms[3] = {0.0f, 0.0f, 0.0f};
     void drop_graph() {
         if (exec) (void)hipGraphExecDestroy(exec);
@@ -712,24 +712,25 @@ struct BatchSlice {
 struct BatchGroup {
     std::vector<BatchSlice> sl;
     size_t spec = 0, norm = 0, rec = 0;      // workspace elements used
-    int nw = 4, blocks = 0;
+    int cp = 1, blocks = 0;                  // particles per work item, persistent workgroups
     size_t job_off = 0, item_off = 0, q_off = 0;
     int n_items = 0;
 };
 
-// Items (slice, particle, reference block, 0) of a group for `nw` waves per
-// workgroup; particle i of the group goes to XCD queue i % 8 with all its
-// blocks.  `limit[k]` caps the particles taken from slice k (sampling).
-void build_queue(const std::vector<BatchSub> &subs, const BatchGroup &gr, int nw,
+// Items (slice, first particle, reference group, particles) of a group, runs of `cp`
+// particles; a run's reference groups go to one XCD queue.  `limit[k]` caps the
+// particles taken from slice k (sampling).
+void build_queue(const std::vector<BatchSub> &subs, const BatchGroup &gr, int cp,
                  const std::vector<int> *limit, std::vector<int4> &items, int qbeg[9]) {
     std::vector<int4> q[8];
     int running = 0;
     for (size_t k = 0; k < gr.sl.size(); ++k) {
         const BatchSlice &sl = gr.sl[k];
-        const int G = (subs[sl.sub].N + 3) / 4, GB = (G + nw - 1) / nw;
+        const int ng = (subs[sl.sub].N + isac::kMrefRefs - 1) / isac::kMrefRefs;
         const int n = limit ? std::min(sl.n, (*limit)[k]) : sl.n;
-        for (int i = 0; i < n; ++i, ++running)
-            for (int b = 0; b < GB; ++b) q[running & 7].push_back(make_int4((int)k, i, b, 0));
+        for (int i = 0; i < n; i += cp, ++running)
+            for (int b = 0; b < ng; ++b)
+                q[running & 7].push_back(make_int4((int)k, i, b, std::min(cp, n - i)));
     }
     items.clear();
     for (int x = 0; x < 8; ++x) {
@@ -739,8 +740,7 @@ void build_queue(const std::vector<BatchSub> &subs, const BatchGroup &gr, int nw
     qbeg[8] = (int)items.size();
 }
 
-std::vector<isac::MrefJob> group_jobs(const std::vector<BatchSub> &subs, const BatchGroup &gr,
-                                      int nw) {
+std::vector<isac::MrefJob> group_jobs(const std::vector<BatchSub> &subs, const BatchGroup &gr) {
     BatchWs &b = ws.batch;
     std::vector<isac::MrefJob> jobs;
     for (const BatchSlice &sl : gr.sl) {
@@ -748,9 +748,15 @@ std::vector<isac::MrefJob> group_jobs(const std::vector<BatchSub> &subs, const B
         jobs.push_back(isac::mref_job(b.spec.as<float2>() + sl.spec_off,
                                       b.norm.as<float2>() + sl.norm_off,
                                       b.rspec.as<float2>() + u.rs_off, b.rsum0.as<float>() + u.rn_off,
-                                      b.rec.as<PeakRec>() + sl.rec_off, sl.n, u.S, u.R, u.N, nw));
+                                      b.rec.as<PeakRec>() + sl.rec_off, sl.n, u.S, u.R, u.N));
     }
     return jobs;
+}
+
+int group_min_ring(const std::vector<BatchSub> &subs, const BatchGroup &gr) {
+    int r = isac::kMaxRings;
+    for (const BatchSlice &sl : gr.sl) r = std::min(r, subs[sl.sub].R);
+    return r;
 }
 
 ShiftView subset_acc(const BatchSub &u, int p0) {
@@ -770,9 +776,10 @@ int batch_polar(const std::vector<BatchSub> &subs, const BatchSlice &sl, int n, 
     return 0;
 }
 
-// Chooses waves per workgroup (1, 2 or 4) for a group by timing the persistent
+// Chooses the particles per work item (1, 2 or 4) for a group by timing the persistent
 // kernel on a sample of the group's particles (about four rounds of resident
-// wavefronts); the winner is cached by the group's shape signature.
+// workgroups with four particles each); the winner is cached by the group's shape
+// signature.
 int tune_group(const std::vector<BatchSub> &subs, BatchGroup &gr, int n_cu, bool report,
                hipStream_t st) {
     BatchWs &b = ws.batch;
@@ -782,23 +789,21 @@ int tune_group(const std::vector<BatchSub> &subs, BatchGroup &gr, int n_cu, bool
         sig += std::to_string(u.R) + "," + std::to_string(u.S) + "," + std::to_string(u.N) + ";";
     }
     const int cand[3] = {1, 2, 4};
-    int bpc[3];
-    for (int c = 0; c < 3; ++c) bpc[c] = isac::mref_queue_blocks_per_cu(cand[c]);
-    auto grid_for = [&](int c) { return std::max(8, (bpc[c] * n_cu + 7) / 8 * 8); };
+    const int bpc = isac::mref_queue_blocks_per_cu();
+    gr.blocks = std::max(8, (bpc * n_cu + 7) / 8 * 8);
     auto it = b.tuned.find(sig);
     if (it != b.tuned.end()) {
-        gr.nw = it->second;
-        gr.blocks = grid_for(gr.nw == 1 ? 0 : gr.nw == 2 ? 1 : 2);
+        gr.cp = it->second;
         return 0;
     }
-    // sample: particles from every slice in proportion, ~4 rounds of resident waves
-    long long wave_items = 0;
-    for (const BatchSlice &sl : gr.sl) wave_items += (long long)sl.n * ((subs[sl.sub].N + 3) / 4);
-    const long long want = 4LL * 8 * n_cu;
+    // sample: particles from every slice in proportion
+    long long pairs = 0;   // (particle, reference group) pairs
+    for (const BatchSlice &sl : gr.sl)
+        pairs += (long long)sl.n * ((subs[sl.sub].N + isac::kMrefRefs - 1) / isac::kMrefRefs);
+    const long long want = 4LL * 4 * gr.blocks;
     std::vector<int> limit;
     for (const BatchSlice &sl : gr.sl) {
-        const long long m = wave_items > want ? ((long long)sl.n * want + wave_items - 1) / wave_items
-                                              : sl.n;
+        const long long m = pairs > want ? ((long long)sl.n * want + pairs - 1) / pairs : sl.n;
         limit.push_back((int)std::max<long long>(1, std::min<long long>(m, sl.n)));
     }
     for (size_t k = 0; k < gr.sl.size(); ++k)
@@ -811,8 +816,7 @@ int tune_group(const std::vector<BatchSub> &subs, BatchGroup &gr, int n_cu, bool
     float ms_c[3] = {0.0f, 0.0f, 0.0f};
     int rc = 0;
     for (int c = 0; c < 3 && !rc; ++c) {
-        if (bpc[c] <= 0) continue;
-        std::vector<isac::MrefJob> jobs = group_jobs(subs, gr, cand[c]);
+        std::vector<isac::MrefJob> jobs = group_jobs(subs, gr);
         std::vector<int4> items;
         int qb[9];
         build_queue(subs, gr, cand[c], &limit, items, qb);
@@ -829,8 +833,8 @@ int tune_group(const std::vector<BatchSub> &subs, BatchGroup &gr, int n_cu, bool
         for (int rep = 0; rep < 2 && !rc; ++rep) {
             (void)hipEventRecord(e0, st);
             if (isac::launch_ccf_mref_queue(b.jobs.as<isac::MrefJob>(), b.items.as<int4>(),
-                                            b.qbeg.as<int>(), b.counters.as<int>(), cand[c],
-                                            grid_for(c), ws.twiddle.as<float2>(), st) != hipSuccess)
+                                            b.qbeg.as<int>(), b.counters.as<int>(), gr.blocks,
+                                            group_min_ring(subs, gr), ws.twiddle.as<float2>(), st) != hipSuccess)
                 rc = kErrHip;
             (void)hipEventRecord(e1, st);
             if (hipEventSynchronize(e1) != hipSuccess) rc = kErrHip;
@@ -847,8 +851,7 @@ int tune_group(const std::vector<BatchSub> &subs, BatchGroup &gr, int n_cu, bool
         set_error(kErrHip, "batched tuning launch failed");
         return rc;
     }
-    gr.nw = best;
-    gr.blocks = grid_for(best == 1 ? 0 : best == 2 ? 1 : 2);
+    gr.cp = best;
     b.tuned[sig] = best;
     if (report) std::copy(ms_c, ms_c + 3, b.cand_ms);
     return 0;
@@ -983,7 +986,8 @@ int batch_record(const std::vector<BatchSub> &subs, const std::vector<BatchGroup
         HIP_OK(isac::launch_ccf_mref_queue(b.jobs.as<isac::MrefJob>() + gr.job_off,
                                            b.items.as<int4>() + gr.item_off,
                                            b.qbeg.as<int>() + gr.q_off, b.counters.as<int>() + 8 * gi,
-                                           gr.nw, gr.blocks, ws.twiddle.as<float2>(), st));
+                                           gr.blocks, group_min_ring(subs, gr),
+                                           ws.twiddle.as<float2>(), st));
         for (const BatchSlice &sl : gr.sl) {
             const BatchSub &u = subs[sl.sub];
             HIP_OK(isac::launch_decode_mref(b.rec.as<PeakRec>() + sl.rec_off, sl.n, u.N,
@@ -1032,17 +1036,17 @@ int run_batched_graph(const IsacMrefSubset *d, unsigned n, hipStream_t st) {
     }
     for (size_t gi = 0; gi < groups.size(); ++gi)
         if (int e = tune_group(subs, groups[gi], n_cu, gi == 0, ws.stream)) return e;
-    b.nw = groups[0].nw;
+    b.cp = groups[0].cp;
     b.blocks = groups[0].blocks;
     // work-queue tables of every group
     std::vector<isac::MrefJob> jobs;
     std::vector<int4> items;
     std::vector<int> qbeg;
     for (BatchGroup &gr : groups) {
-        std::vector<isac::MrefJob> j = group_jobs(subs, gr, gr.nw);
+        std::vector<isac::MrefJob> j = group_jobs(subs, gr);
         std::vector<int4> it;
         int qb[9];
-        build_queue(subs, gr, gr.nw, nullptr, it, qb);
+        build_queue(subs, gr, gr.cp, nullptr, it, qb);
         gr.job_off = jobs.size();
         gr.item_off = items.size();
         gr.q_off = qbeg.size();
@@ -1793,7 +1797,7 @@ void isac_batched_report(int *n_groups, int *n_nodes, int *replayed, int *nw, in
     if (n_groups) *n_groups = b.groups;
     if (n_nodes) *n_nodes = b.nodes;
     if (replayed) *replayed = b.replayed;
-    if (nw) *nw = b.nw;
+    if (nw) *nw = b.cp;
     if (blocks) *blocks = b.blocks;
     if (cand_ms3) std::copy(b.cand_ms, b.cand_ms + 3, cand_ms3);
 }

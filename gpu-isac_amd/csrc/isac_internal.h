@@ -11,10 +11,14 @@ namespace isac {
 constexpr int kRingLen = 256;   // samples per ring (fixed by every caller)
 constexpr int kSlots = 128;     // packed spectrum slots per ring: slot 0 = (X[0], X[128])
 
-// Position of spectrum slot k in a ring row of kSlots float2: slots k and k + 64
-// are adjacent, so a lane that owns slots l and l + 64 reads both with one
-// 16-byte access (float4 l of the row).
-__host__ __device__ constexpr int slot_pos(int k) { return 2 * (k & 63) + (k >> 6); }
+// A ring row is 256 floats in the operand order of the FP32 matrix instruction
+// (v_mfma_f32_16x16x1, four 16 x 16 blocks): slot k's real part sits at float
+// slot_re(k), its imaginary part 4 floats on.  One lane's 16-byte load then holds one
+// part of the four slots u + 16 (4 mh + j), j = 0..3 (the operands of four
+// instructions), and the four slots of an instruction, u = 4 uq .. 4 uq + 3, are one
+// 128-byte line.
+constexpr int kPartOff = 4;
+__host__ __device__ constexpr int slot_re(int k) { return (k >> 6) * 128 + (k & 15) * 8 + ((k >> 4) & 3); }
 constexpr int kMaxImgDim = 128; // image staged whole in LDS by the polar kernel
 constexpr int kMaxRings = 127;  // rings must fit inside a 256-sample ring FFT budget
 
@@ -69,23 +73,27 @@ struct MrefJob {
     const float2 *rspec;    // [N][R][kSlots] normalised, ring-weighted reference spectra
     const float *rsum0;     // [N]
     PeakRec *rec;           // [n_img][N], or [lists][K] in the candidate form
-    int n_img, S, R, N, G, GB;   // G reference groups of 4, GB workgroups per particle
-    const int *cand = nullptr;   // candidate form: [lists][K] reference ids
+    int n_img, S, R, N;
+    const int *cand = nullptr;   // candidate form: [lists][K] reference ids, K <= kMrefRefs
     const int *pidx = nullptr;   // candidate form: spectra row of each list, or null
     int K = 0;
 };
 
-MrefJob mref_job(const float2 *spec, const float2 *norm, const float2 *rspec, const float *rsum0,
-                 PeakRec *rec, int n_img, int n_shift, int n_ring, int n_ref, int nw);
+constexpr int kMrefRefs = 8;     // references of one search workgroup
+constexpr int kMrefWaves = 16;   // wavefronts of one search workgroup
 
-// Persistent multi-reference kernel over many jobs: items (job, particle, block)
-// in 8 per-XCD queues [qbeg[q], qbeg[q+1]); counters (8 ints) are reset by a
-// kernel first (no memset node, safe inside captured graphs).
-// nw (waves per workgroup) is 1, 2 or 4; blocks should be a multiple of 8.
+MrefJob mref_job(const float2 *spec, const float2 *norm, const float2 *rspec, const float *rsum0,
+                 PeakRec *rec, int n_img, int n_shift, int n_ring, int n_ref);
+
+// Persistent multi-reference kernel over many jobs: items (job, first particle,
+// reference group, particle count) in 8 per-XCD queues [qbeg[q], qbeg[q+1]);
+// counters (8 ints) are reset by a kernel first (no memset node, safe inside
+// captured graphs).  blocks should be a multiple of 8; min_ring = the smallest ring
+// count of the jobs.
 hipError_t launch_ccf_mref_queue(const MrefJob *jobs, const int4 *items, const int *qbeg,
-                                 int *counters, int nw, int blocks, const float2 *twiddle,
+                                 int *counters, int blocks, int min_ring, const float2 *twiddle,
                                  hipStream_t st);
-int mref_queue_blocks_per_cu(int nw);   // occupancy of the queue kernel (0 on error)
+int mref_queue_blocks_per_cu();   // occupancy of the queue kernel (0 on error)
 
 // Polar spectra of the shifts marked in smask[img] only (n_shift <= 64).
 hipError_t launch_polar_spectra_masked(const float *imgs, int n_img, int img_dim, ShiftView acc,

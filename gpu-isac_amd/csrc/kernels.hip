@@ -18,6 +18,7 @@
 #include <climits>
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 namespace isac {
 namespace {
@@ -150,24 +151,34 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
     return (xcd < r) ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
-// Slots lane and lane + 64 of one ring row (adjacent in memory, slot_pos): one
-// 16-byte load.
-__device__ __forceinline__ void load_slots(const float2 *row, int lane, float2 &lo, float2 &hi) {
-    const float4 v = reinterpret_cast<const float4 *>(row)[lane];
-    lo = make_float2(v.x, v.y);
-    hi = make_float2(v.z, v.w);
+// Stores a wavefront's slots lane (lo) and lane + 64 (hi) of one ring row in the
+// operand order of slot_re: a 4 x 4 transpose between the four 16-lane rows and the
+// four parts (2 + 2 lane-row swaps), then one 16-byte store per lane.
+__device__ __forceinline__ void swap32(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void store_ring(float2 *row, int lane, float2 lo, float2 hi) {
+    float r0 = lo.x, r1 = lo.y, r2 = hi.x, r3 = hi.y;
+    swap32(r0, r2);
+    swap32(r1, r3);
+    swap16(r0, r1);
+    swap16(r2, r3);
+    // lane row 0 / 1: real / imaginary parts of slots u + 16 j, 2 / 3: of slots 64 on
+    const int g = lane >> 4, u = lane & 15;
+    reinterpret_cast<float4 *>(row)[(g >> 1) * 32 + u * 2 + (g & 1)] = make_float4(r0, r1, r2, r3);
 }
 
-__device__ __forceinline__ void wave_argmax(float &v, int &t) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(v, off, kWave);
-        const int ot = __shfl_xor(t, off, kWave);
-        if (ov > v || (ov == v && ot < t)) {
-            v = ov;
-            t = ot;
-        }
-    }
+// One slot of a ring row.
+__device__ __forceinline__ float2 load_slot(const float2 *row, int k) {
+    const float *q = reinterpret_cast<const float *>(row) + slot_re(k);
+    return make_float2(q[0], q[kPartOff]);
 }
 
 // ------------------------------------------------------------------ stage A
@@ -267,10 +278,9 @@ __global__ __launch_bounds__(256) void k_polar_spectra(
                     al = f2(zl.x, v[2].x);
                     bl = f2(zl.y, v[2].y);
                 }
-                // slots lane and lane + 64 are adjacent (slot_pos): one 16-byte store per ring
-                float4 *oa = reinterpret_cast<float4 *>(spec + (((size_t)p * S + sg[g]) * (size_t)R + i) * kSlots);
-                oa[lane] = make_float4(al.x, al.y, ah.x, ah.y);
-                if (hb) oa[kSlots / 2 + lane] = make_float4(bl.x, bl.y, bh.x, bh.y);
+                float2 *oa = spec + (((size_t)p * S + sg[g]) * (size_t)R + i) * kSlots;
+                store_ring(oa, lane, al, ah);
+                if (hb) store_ring(oa + kSlots, lane, bl, bh);
             }
         }
 #pragma unroll
@@ -584,8 +594,8 @@ __global__ __launch_bounds__(128) void k_ref_finalize(float2 *__restrict__ rspec
     const float2 nm = rnorm[n];
     double acc0 = 0.0;
     for (int i = 0; i < R; ++i) {
-        float2 *px = rspec + ((size_t)n * R + i) * kSlots + slot_pos(k);
-        float2 x = *px;
+        float *px = reinterpret_cast<float *>(rspec + ((size_t)n * R + i) * kSlots) + slot_re(k);
+        float2 x = f2(px[0], px[kPartOff]);
         const float gw = nm.y * (float)(i + 1);
         if (k == 0) {
             x.x = (x.x - nm.x) * gw;
@@ -595,143 +605,316 @@ __global__ __launch_bounds__(128) void k_ref_finalize(float2 *__restrict__ rspec
             x.x *= gw;
             x.y *= gw;
         }
-        *px = x;
+        px[0] = x.x;
+        px[kPartOff] = x.y;
     }
     if (k == 0) rsum0[n] = (float)acc0;
 }
 
 // ------------------------------------------------------------------ stage B
-// Psi stage of one (shift row, reference) pair.  Q / P hold the four real ring
-// products P1..P4 (sr*rr, si*ri, si*rr, sr*ri summed over rings with the ring
-// weight folded into the reference) of spectrum slots `lane` and `lane+64`:
-// C0 = R conj S = (P1+P2, P4-P3), C1 = conj(R S) = (P1-P2, -(P3+P4)).  The pair
-// becomes one 256-point inverse FFT of Z = C0 + i C1 (Hermitian-extended), so
-// z[t] = c0[t] + i c1[t] holds the psi CCF of both mirrors.  The running
-// first-max over (mirror, shift, psi) of this reference (bv, bf) and the seven
-// samples around it (nb, LDS) are updated; the 6-step wave argmax only runs
-// when some lane beats the running maximum (rows arrive in increasing shift
-// order, so an equal value can never displace the earlier maximum).
-//
-// MASKED: only samples whose bit (m * 4 + q) is set in `allow` (lane's samples
-// lane + 64 q of mirror m) take part in the maximum; the seven neighbours stay
-// the unmasked CCF values.
-template <bool SINGLE, bool MASKED = false>
-__device__ __forceinline__ void psi_update(const float (&Q)[4], const float (&P)[4], float2 nm,
-                                           float rs0, int s, int lane, float2 *b0, float2 *b1,
-                                           const float2 *tw, float *zb, float (*nb)[8],
-                                           float (&bv)[2], int (&bf)[2], unsigned allow = 0xffu) {
-    const int pl = (64 - lane) & 63;
-    const float gs = nm.y;
-    float A = P[0] + P[1], B = P[3] - P[2], Cc = P[0] - P[1], Dd = -(P[2] + P[3]);
-    const float2 zhi = f2(gs * (A - Dd), gs * (B + Cc));
-    const float2 yhi = f2(gs * (A + Dd), gs * (Cc - B));
-    A = Q[0] + Q[1];
-    B = Q[3] - Q[2];
-    Cc = Q[0] - Q[1];
-    Dd = -(Q[2] + Q[3]);
-    float2 zlo = f2(gs * (A - Dd), gs * (B + Cc));
-    const float2 ylo = f2(gs * (A + Dd), gs * (Cc - B));
-    float2 nyq = f2(0.0f, 0.0f);
-    if (lane == 0) {  // packed slot 0: DC (with the mean correction) and Nyquist
-        const float c0 = gs * (Q[0] - nm.x * rs0);
-        const float cn = gs * Q[1];
-        zlo = f2(c0, c0);
-        nyq = f2(cn, cn);
-    }
-    const float2 syhi = shfl2(yhi, pl), sylo = shfl2(ylo, pl);
-    float2 v[4];
-    v[0] = zlo;
-    v[1] = zhi;
-    v[2] = lane ? syhi : nyq;
-    v[3] = lane ? sylo : yhi;
-    fft256_wave<true>(v, b0, b1, tw, lane);
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        float bvl = m ? v[0].y : v[0].x;
-        if (MASKED && !((allow >> (m * 4)) & 1u)) bvl = -INFINITY;
-        int bt = lane;
-#pragma unroll
-        for (int q = 1; q < 4; ++q) {
-            float x = m ? v[q].y : v[q].x;
-            if (MASKED && !((allow >> (m * 4 + q)) & 1u)) x = -INFINITY;
-            if (x > bvl) {
-                bvl = x;
-                bt = lane + 64 * q;
-            }
-        }
-        const bool sentinel = SINGLE && m == 0 && s == 0 && bf[0] == 0 && bv[0] == 0.0f;
-        if (!__any(bvl > bv[m]) && !sentinel) continue;
-        wave_argmax(bvl, bt);
-        const int flat = s * kRingLen + bt;
-        const bool upd = bvl > bv[m] || (bvl == bv[m] && flat < bf[m]);
-        if (upd || sentinel) {
-            const int tc = upd ? bt : 0;
-            if (upd) {
-                bv[m] = bvl;
-                bf[m] = flat;
-            }
-            wave_lds_sync();
-#pragma unroll
-            for (int q = 0; q < 4; ++q) zb[lane + 64 * q] = m ? v[q].y : v[q].x;
-            wave_lds_sync();
-            if (lane < 7) nb[m][lane] = zb[(tc + lane - 3) & 255];
-            wave_lds_sync();
-        }
+// Psi transform: 256-point inverse FFTs, four per wavefront (16 lanes each, 16 points
+// per lane).  The four radix-4 stages run in pairs inside a lane, so one exchange
+// through LDS is left (a form with a transform spread over 64 lanes had three, and 36
+// LDS instructions per transform against 12 here); the arithmetic of a stage (inputs,
+// twiddles, operation order) is that of the Stockham stages above.
+constexpr int kFftLd = 273;       // float2 per transform in LDS (odd mod 32: no bank conflicts
+                                  // between transforms; 17 x 16 + 1 hold the padded exchange)
+constexpr int kMirOff = 136;      // Z[k], k < 128, at k; Z[256 - k] at kMirOff + k (k = 1..128)
+constexpr int kIfftTw = 15 * 16;  // lane twiddles of the last two stages
+
+// entry q - 1: stage 3, e^{-2 pi i 4 q u / 256}; entry 3 + 3 q3 + q - 1: stage 4,
+// e^{-2 pi i q (u + 16 q3) / 256}
+__device__ __forceinline__ void fill_ifft_twiddles(float2 *tw, const float2 *twg, int tid, int nthreads) {
+    for (int i = tid; i < kIfftTw; i += nthreads) {
+        const int e = i >> 4, u = i & 15;
+        tw[i] = e < 3 ? twg[4 * (e + 1) * u] : twg[((e - 3) % 3 + 1) * (u + 16 * ((e - 3) / 3))];
     }
 }
 
-__device__ __forceinline__ void write_rec(PeakRec *o, const float (&bv)[2], const int (&bf)[2],
-                                          const float (*nb)[8], int lane) {
-    const int m = (bv[1] > bv[0]) ? 1 : 0;
-    const int f = (bf[m] == INT_MAX) ? 0 : bf[m];   // never updated (all values NaN)
+// v conj(w), with the operation order of cmul under INV
+__device__ __forceinline__ float2 cmulc(float2 v, float2 w) {
+    return f2(fmaf(v.x, w.x, v.y * w.y), fmaf(v.y, w.x, -(v.x * w.y)));
+}
+
+// cos, sin of -2 pi m / 256 for the m = 16 q k of the second stage (the table's values)
+__device__ __forceinline__ constexpr float2 stage2_tw(int m) {
+    return m == 16    ? float2{0.92387953251128674f, -0.38268343236508977f}
+           : m == 32  ? float2{0.70710678118654757f, -0.70710678118654757f}
+           : m == 48  ? float2{0.38268343236508984f, -0.92387953251128674f}
+           : m == 64  ? float2{6.123233995736766e-17f, -1.0f}
+           : m == 96  ? float2{-0.70710678118654746f, -0.70710678118654757f}
+                      : float2{-0.92387953251128685f, 0.38268343236508967f};   // m == 144
+}
+
+// First two stages.  In: x[m] = Z[u + 16 m], Z[64..127] (m = 4..7) without the row's
+// scale gs, which the first butterflies apply in one rounding.  Out: x[4 k + q] is
+// point 17 u + k + 4 q of the exchange.
+__device__ __forceinline__ void ifft256_head(float2 (&x)[16], float gs) {
+#pragma unroll
+    for (int q2 = 0; q2 < 4; ++q2) {   // stage 1, butterfly u + 16 q2
+        const float2 v0 = x[q2], v1 = x[q2 + 4], v2 = x[q2 + 8], v3 = x[q2 + 12];
+        const float2 a0 = f2(v0.x + v2.x, v0.y + v2.y), a1 = f2(v0.x - v2.x, v0.y - v2.y);
+        const float2 a2 = f2(fmaf(gs, v1.x, v3.x), fmaf(gs, v1.y, v3.y));
+        const float2 a3 = f2(fmaf(gs, v1.x, -v3.x), fmaf(gs, v1.y, -v3.y));
+        x[q2] = f2(a0.x + a2.x, a0.y + a2.y);
+        x[q2 + 4] = f2(a1.x - a3.y, a1.y + a3.x);
+        x[q2 + 8] = f2(a0.x - a2.x, a0.y - a2.y);
+        x[q2 + 12] = f2(a1.x + a3.y, a1.y - a3.x);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {      // stage 2, butterfly 4 u + k
+        float2 v[4] = {x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
+        if (k > 0) {
+#pragma unroll
+            for (int q = 1; q < 4; ++q) v[q] = cmulc(v[q], stage2_tw(16 * q * k));
+        }
+        radix4<true>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[4 * k + q] = v[q];
+    }
+}
+
+__device__ __forceinline__ void ifft256_put(const float2 (&x)[16], float2 *xb, int u) {
+    float2 *xw = xb + 17 * u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xw[k + 4 * q] = x[4 * k + q];
+}
+
+__device__ __forceinline__ void ifft256_get(float2 (&x)[16], const float2 *xb, int u) {
+    const float2 *xr = xb + u;
+#pragma unroll
+    for (int a = 0; a < 16; ++a) x[a] = xr[17 * a];
+}
+
+// Last two stages.  Out: x[m] = z[u + 16 m].
+__device__ __forceinline__ void ifft256_tail(float2 (&x)[16], const float2 *tw, int u) {
+    float2 w3[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) w3[q] = tw[q * 16 + u];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {      // stage 3, butterfly 16 h + u
+        float2 v[4] = {x[h], x[h + 4], x[h + 8], x[h + 12]};
+#pragma unroll
+        for (int q = 1; q < 4; ++q) v[q] = cmulc(v[q], w3[q - 1]);
+        radix4<true>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[h + 4 * q] = v[q];
+    }
+#pragma unroll
+    for (int q3 = 0; q3 < 4; ++q3) {   // stage 4, butterfly u + 16 q3
+        float2 v[4] = {x[4 * q3], x[4 * q3 + 1], x[4 * q3 + 2], x[4 * q3 + 3]};
+#pragma unroll
+        for (int q = 1; q < 4; ++q) v[q] = cmulc(v[q], tw[(3 + 3 * q3 + q - 1) * 16 + u]);
+        radix4<true>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[4 * q3 + q] = v[q];
+    }
+    // x[4 q3 + q] = z[u + 16 q3 + 64 q]: to natural order
+    float2 y[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) y[m] = x[4 * (m & 3) + (m >> 2)];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) x[m] = y[m];
+}
+
+// Z of one transform from LDS (positions of kMirOff) into lane u's 16 points
+__device__ __forceinline__ void load_z(float2 (&x)[16], const float2 *xb, int u) {
+    const float2 *lo = xb + u, *hi = xb + (kMirOff + 16 - u);
+#pragma unroll
+    for (int m = 0; m < 8; ++m) x[m] = lo[16 * m];
+#pragma unroll
+    for (int m = 8; m < 16; ++m) x[m] = hi[16 * (15 - m)];
+}
+
+// Four transforms (lane row f's at xb, kFftLd float2 that are free to overwrite)
+__device__ __forceinline__ void ifft256_rows4(float2 (&x)[16], float gs, float2 *xb, const float2 *tw, int u) {
+    load_z(x, xb, u);
+    ifft256_head(x, gs);
+    wave_lds_sync();
+    ifft256_put(x, xb, u);
+    wave_lds_sync();
+    ifft256_get(x, xb, u);
+    ifft256_tail(x, tw, u);
+}
+
+// max over the 16 lanes of each lane row, then the wavefront's (uniform)
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true)));
+    const float a = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+    const float b = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+    const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+    const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
+    return fmaxf(fmaxf(a, b), fmaxf(c, d));
+}
+
+// Running first maximum of one (particle, reference) over (mirror, shift, psi): value,
+// flat index shift * 256 + psi sample, and (LDS) the seven samples around it.
+struct PeakState {
+    float bv[2];
+    int bf[2];
+    __device__ __forceinline__ void reset(float v, int f) {
+        bv[0] = bv[1] = v;
+        bf[0] = bf[1] = f;
+    }
+};
+
+// Takes lane rows [f0, f0 + cnt) of a batch (lane row f holds the transform of shift
+// s + f - f0) into the running maximum.  Rows arrive in increasing shift order, so a
+// later equal value never displaces an earlier one, and the search for the position
+// runs only when some lane beats the running maximum.  xb: the lane's transform
+// buffer, free to overwrite.  SINGLE: the search starts from value 0 at index 0 like
+// the reference's row argmax (cuda/gpu_aln_noref.cu:1638-1664), so when no value of
+// the first shift is positive the record is that shift's sample 0.  MASKED: only the
+// samples u + 16 m whose bit m (mirror 0) / 16 + m (mirror 1) of `allow` is set
+// compete; the seven neighbours stay the unmasked values.
+template <bool SINGLE, bool MASKED>
+__device__ __forceinline__ void peak_update(PeakState &st, const float2 (&x)[16], int f0, int cnt, int s,
+                                            int lane, float2 *xb, float (*nb)[8], unsigned allow) {
+    const int f = lane >> 4, u = lane & 15;
+    const bool in = f >= f0 && f < f0 + cnt;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        auto val = [&](int i) {
+            const float v = m ? x[i].y : x[i].x;
+            return (MASKED && !((allow >> (16 * m + i)) & 1u)) ? -INFINITY : v;
+        };
+        float lm = val(0);
+#pragma unroll
+        for (int i = 1; i < 16; ++i) lm = fmaxf(lm, val(i));
+        lm = in ? lm : -INFINITY;
+        const bool beats = __any(lm > st.bv[m]);
+        const bool sentinel = SINGLE && m == 0 && s == 0 && !beats;
+        if (!beats && !sentinel) continue;
+        int fw = f0, t = 0;
+        if (beats) {
+            const float top = wave_max(lm);
+            int tl = INT_MAX;
+#pragma unroll
+            for (int i = 15; i >= 0; --i)
+                if (val(i) == top) tl = u + 16 * i;
+            const unsigned long long hit = __ballot(in && lm == top);
+            fw = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)hit) - 1) >> 4;   // smallest shift
+            int tm = (f == fw && lm == top) ? tl : INT_MAX;
+            tm = min(tm, __builtin_amdgcn_update_dpp(0, tm, 0x128, 0xf, 0xf, true));
+            tm = min(tm, __builtin_amdgcn_update_dpp(0, tm, 0x124, 0xf, 0xf, true));
+            tm = min(tm, __builtin_amdgcn_update_dpp(0, tm, 0x122, 0xf, 0xf, true));
+            tm = min(tm, __builtin_amdgcn_update_dpp(0, tm, 0x121, 0xf, 0xf, true));
+            t = __builtin_amdgcn_readlane(tm, fw * 16);
+            st.bv[m] = top;
+            st.bf[m] = (s + fw - f0) * kRingLen + t;
+        }
+        wave_lds_sync();
+        float *zb = reinterpret_cast<float *>(xb);
+        if (f == fw) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) zb[u + 16 * i] = m ? x[i].y : x[i].x;
+        }
+        wave_lds_sync();
+        if (f == fw && u < 7) nb[m][u] = zb[(t + u - 3) & 255];
+        wave_lds_sync();
+    }
+}
+
+__device__ __forceinline__ void write_rec(PeakRec *o, const PeakState &st, const float (*nb)[8], int lane) {
+    const int m = (st.bv[1] > st.bv[0]) ? 1 : 0;
+    const bool none = st.bf[m] == INT_MAX;   // never updated: empty, or all values NaN
+    const int f = none ? 0 : st.bf[m];
     if (lane == 0) {
-        o->val = bv[m];
+        o->val = st.bv[m];
         o->m = m;
         o->s = f / kRingLen;
         o->t = f % kRingLen;
         o->pad = 0;
     }
-    if (lane < 7) o->x[lane] = nb[m][lane];
+    if (lane < 7) o->x[lane] = none ? 0.0f : nb[m][lane];
 }
 
-// Items (particle, reference): one wavefront per item walks the shifts four at a
-// time (4 rows x 1 reference).  Item i uses particle i / K and reference
-// ref_of[i * ref_stride].  ZERO_INIT: the search starts from value 0 at flat index
-// 0 like the reference's row argmax for pre-alignment / reference-free
-// (cuda/gpu_aln_noref.cu:1638-1664); otherwise from -FLT_MAX like the
-// multi-reference wizard, giving exactly the FP32 multi-reference kernel's
-// arithmetic for that pair (used to re-score candidates).
-template <bool ZERO_INIT>
-__global__ __launch_bounds__(256) void k_ccf_items(
+constexpr float kNoPeak = -3.40282e+38f;
+
+// A lane's two slots of a ring row: k = u + 16 (4 mh + 2 jp) and k + 16, with
+// (mh, jp) = lane row; two 8-byte loads per row.
+__device__ __forceinline__ int lane_slot(int lane) { return (lane & 15) + 64 * (lane >> 5) + 32 * ((lane >> 4) & 1); }
+__device__ __forceinline__ void load_pair(const float2 *row, int lane, float2 &re, float2 &im) {
+    const float2 *q = row + (lane >> 5) * 64 + (lane & 15) * 4 + ((lane >> 4) & 1);
+    re = q[0];
+    im = q[kPartOff / 2];
+}
+
+// Products of one reference's lane slots (br, bi) with a row's: P1..P4 = rr sr, ri si,
+// rr si, ri sr of both slots, summed over rings
+__device__ __forceinline__ void pair_fma(float (&acc)[2][4], float2 br, float2 bi, float2 ar, float2 ai) {
+    acc[0][0] += br.x * ar.x;
+    acc[0][1] += bi.x * ai.x;
+    acc[0][2] += br.x * ai.x;
+    acc[0][3] += bi.x * ar.x;
+    acc[1][0] += br.y * ar.y;
+    acc[1][1] += bi.y * ai.y;
+    acc[1][2] += br.y * ai.y;
+    acc[1][3] += bi.y * ar.y;
+}
+
+// Z of one (shift row, reference) from the ring products, into LDS at the transform's
+// positions: C0 = R conj S = (P1 + P2, P4 - P3), C1 = conj(R S) = (P1 - P2, -(P3 + P4));
+// Z[k] = C0 + i C1, Z[256 - k] its Hermitian partner; slot 0 packs the real bins 0
+// (with the mean correction) and 128.  nm = (mu L, 1 / sd) scales the row, but for
+// Z[64..127], which ifft256_lane16 scales.
+__device__ __forceinline__ void store_pair_z(float2 *xb, const float (&acc)[2][4], float2 nm, float rs0, int lane) {
+    const int k0 = lane_slot(lane);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = k0 + 16 * h;
+        const float a = acc[h][0] + acc[h][1], e = acc[h][2] + acc[h][3];
+        const float c = acc[h][0] - acc[h][1], b = acc[h][3] - acc[h][2];
+        const float gz = lane < 32 ? nm.y : 1.0f;   // lane rows 2, 3: slots 64..127
+        float2 z = f2(gz * (a + e), gz * (b + c)), y = f2(nm.y * (a - e), nm.y * (c - b));
+        int ky = kMirOff + k;
+        if (h == 0 && lane == 0) {
+            const float c0 = nm.y * fmaf(-nm.x, rs0, acc[0][0]);
+            const float cn = nm.y * acc[0][1];
+            z = f2(c0, c0);
+            y = f2(cn, cn);
+            ky = kMirOff + 128;
+        }
+        xb[k] = z;
+        xb[ky] = y;
+    }
+}
+
+// The value of the lane's row of 16 lanes.
+__device__ __forceinline__ float lane_row_of(float r0, float r1, float r2, float r3, int lane) {
+    const float lo = (lane & 16) ? r1 : r0, hi = (lane & 16) ? r3 : r2;
+    return (lane & 32) ? hi : lo;
+}
+
+// One wavefront per particle, against its own reference ref_of[i * ref_stride]: four
+// shift rows at a time (4 rows x 1 reference, two slots per lane), psi transforms of
+// the four rows side by side.  The search starts from value 0 at index 0.
+__global__ __launch_bounds__(256) void k_ccf_single(
     const float2 *__restrict__ spec, const float2 *__restrict__ norm,
     const float2 *__restrict__ rspec, const float *__restrict__ rsum0,
-    const int *__restrict__ ref_of, int ref_stride, int K, int n_items, int S, int R, int N,
-    const float2 *__restrict__ twg, PeakRec *__restrict__ rec, const int *__restrict__ pidx) {
-    __shared__ float2 tw[256];
-    __shared__ float2 fbuf[4][512];
-    __shared__ float zbuf[4][256];
+    const int *__restrict__ ref_of, int ref_stride, int n_items, int S, int R, int N,
+    const float2 *__restrict__ twg, PeakRec *__restrict__ rec) {
+    __shared__ float2 tw[kIfftTw];
+    __shared__ float2 fbuf[4][4 * kFftLd];
     __shared__ float nbuf[4][2][8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    fill_fft_twiddles(tw, twg, tid, 256);
+    fill_ifft_twiddles(tw, twg, tid, 256);
     __syncthreads();
-    const int item = blockIdx.x * 4 + wave;
-    if (item >= n_items) return;
-    const int p = pidx ? pidx[item / K] : item / K;   // spectra row of the item's particle
-    float bv[2];
-    int bf[2];
-    bv[0] = bv[1] = ZERO_INIT ? 0.0f : -3.40282e+38f;
-    bf[0] = bf[1] = ZERO_INIT ? 0 : INT_MAX;
-    const int n_raw = ref_of[(size_t)item * ref_stride];
-    if (!ZERO_INIT && n_raw < 0) {   // no reference for this item: an empty record
-        if (lane < 8) nbuf[wave][0][lane] = 0.0f;
-        write_rec(rec + item, bv, bf, nbuf[wave], lane);
-        return;
-    }
+    const int p = blockIdx.x * 4 + wave;
+    if (p >= n_items) return;
+    PeakState st;
+    st.reset(0.0f, 0);
     // the host validates ref ids; the clamp keeps every read in bounds
-    const int n = min(max(n_raw, 0), N - 1);
+    const int n = min(max(ref_of[(size_t)p * ref_stride], 0), N - 1);
     const float rs0 = rsum0[n];
     const float2 *rb0 = rspec + (size_t)n * R * kSlots;
     const size_t img_stride = (size_t)S * R * kSlots;
+    float2 *xb = fbuf[wave] + (lane >> 4) * kFftLd;
     for (int s0 = 0; s0 < S; s0 += 4) {
         float acc[4][2][4];
 #pragma unroll
@@ -745,34 +928,27 @@ __global__ __launch_bounds__(256) void k_ccf_items(
         for (int r = 0; r < 4; ++r)
             arow[r] = spec + (size_t)p * img_stride + (size_t)min(s0 + r, S - 1) * R * kSlots;
         for (int i = 0; i < R; ++i) {
-            float2 b0v, b1v;
-            load_slots(rb0 + i * kSlots, lane, b0v, b1v);
-            float2 a0s[4], a1s[4];
+            float2 br, bi, ar[4], ai[4];
+            load_pair(rb0 + i * kSlots, lane, br, bi);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) load_slots(arow[r] + i * kSlots, lane, a0s[r], a1s[r]);
+            for (int r = 0; r < 4; ++r) load_pair(arow[r] + i * kSlots, lane, ar[r], ai[r]);
             __builtin_amdgcn_sched_barrier(0);   // all of the ring's loads in flight before the FMAs
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float2 a0 = a0s[r], a1 = a1s[r];
-                acc[r][0][0] += b0v.x * a0.x;
-                acc[r][0][1] += b0v.y * a0.y;
-                acc[r][0][2] += b0v.x * a0.y;
-                acc[r][0][3] += b0v.y * a0.x;
-                acc[r][1][0] += b1v.x * a1.x;
-                acc[r][1][1] += b1v.y * a1.y;
-                acc[r][1][2] += b1v.x * a1.y;
-                acc[r][1][3] += b1v.y * a1.x;
-            }
+            for (int r = 0; r < 4; ++r) pair_fma(acc[r], br, bi, ar[r], ai[r]);
         }
+        wave_lds_sync();
+        float2 nm[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int s = s0 + r;
-            if (s >= S) break;
-            psi_update<ZERO_INIT>(acc[r][0], acc[r][1], norm[(size_t)p * S + s], rs0, s, lane,
-                                  fbuf[wave], fbuf[wave] + 256, tw, zbuf[wave], nbuf[wave], bv, bf);
+            nm[r] = norm[(size_t)p * S + min(s0 + r, S - 1)];
+            store_pair_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
         }
+        wave_lds_sync();
+        float2 x[16];
+        ifft256_rows4(x, lane_row_of(nm[0].y, nm[1].y, nm[2].y, nm[3].y, lane), xb, tw, lane & 15);
+        peak_update<true, false>(st, x, 0, min(4, S - s0), s0, lane, xb, nbuf[wave], 0u);
     }
-    write_rec(rec + item, bv, bf, nbuf[wave], lane);
+    write_rec(rec + p, st, nbuf[wave], lane);
 }
 
 // Top-K references of every particle by approximate peak value (descending; ties
@@ -880,7 +1056,7 @@ __global__ __launch_bounds__(256) void k_rescore_f64(
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = lane + 64 * h;
-            const float2 av = a[i * kSlots + slot_pos(k)], bv = b[i * kSlots + slot_pos(k)];
+            const float2 av = load_slot(a + i * kSlots, k), bv = load_slot(b + i * kSlots, k);
             const double x = ((k == 0) ? ((double)av.x - muL) : (double)av.x) * g;
             const double y = (double)av.y * g;
             P[h][0] += (double)bv.x * x;
@@ -930,250 +1106,274 @@ __global__ void k_resolve_ties(const int *__restrict__ cand, const double *__res
     }
 }
 
-// Multi-reference: one workgroup = one particle x NW groups of 4 references (one
-// group per wavefront).  The workgroup walks the shifts four at a time; the four
-// shift rows' ring spectra are staged cooperatively in LDS in double-buffered
-// chunks of kRingChunk rings, so only the references' spectra come through the
-// vector L1.  Lane l accumulates, over rings, P1..P4 of slots l and l+64 for
-// 4 rows x 4 references (128 accumulators), then each (row, reference) pair goes
-// through psi_update.
-constexpr int kRingChunk = 4;
+// Multi-reference search, FP32.  Workgroup = 8 references (a tile) x a run of consecutive
+// (particle, shift) rows, sixteen wavefronts, one workgroup per CU.  Per block of 8 rows:
+//  * ring contraction (wavefronts 0..7) on v_mfma_f32_16x16x1_f32 (four 16 x 16 blocks,
+//    K = 1 ring): the four blocks are four spectrum slots, rows = 8 particle rows x (re,
+//    im), columns = 8 references x (re, im), so one instruction adds P1..P4 of 64 pairs
+//    in four slots.  Each step is one fused multiply-add, rings in order: the bits of an
+//    fmaf chain.  A wavefront owns 16 slots (4 instructions a ring, 64 accumulators);
+//    the operands of one ring are one 16-byte load per lane and side;
+//  * the cross-spectra of the 64 pairs (128 KB) go through LDS to the psi transforms;
+//  * psi transforms and search (wavefronts 8..15): one reference each, four rows side by
+//    side, while the others contract the next block.
+// The tiles of a run are neighbouring workgroups on one XCD and read its rows through
+// one L2.
+//
+// Why this form: with both stages on the vector unit (an earlier kernel, 4 rows x 16
+// references per workgroup at two wavefronts per SIMD) instruction issue bound the
+// search, 115 ms for 20 000 x 100 at 76 px, 35 rings, 49 shifts; this one takes 65 ms.
+// On this chip a SIMD's matrix and vector instructions do not overlap (4 matrix
+// instructions of 32 cycles and 64 adds take the sum of their times, at 1, 2 and 4
+// wavefronts), so the floor of a block is the sum: 8 960 matrix cycles at 35 rings and
+// about 5 600 vector cycles, 36 ms in all.  What is left above it: 528 KB of operand
+// loads a block (without them 53 ms; 8 KB a ring at 25-32 bytes per cycle and CU), the
+// psi wavefronts' LDS round trips, and the two barriers.  Splitting the wavefronts by
+// stage beat every form in which each does both (spills at 128 registers, or phases
+// that leave the load path idle): 75 ms with two workgroups of 8 wavefronts per CU, 82 ms
+// with one whose wavefronts keep 28 rings of the rows.
+constexpr int kMrefPre = 4;       // rings of the rows in flight
+constexpr int kRefPre = 2;        // and of the references' rings past the resident ones
+// rings of the references kept in registers over a run: 4 096 x 100 at 76 px takes 14.9 ms
+// with none, 13.5 with 4, 14.3 with 6, 15.0 with 8 (a wavefront has 128 registers)
+constexpr int kMrefKeep = 4;
 
-// RW shift rows per group x RB references per wavefront (RW RB = 16: 128 accumulators),
-// rows staged CH rings at a time.
-template <int NW, int RW = 4, int RB = 4, int CH = kRingChunk>
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
 struct MrefLds {
-    float2 tw[256];
-    float4 abuf4[2][RW * CH * kSlots / 2];   // [buf][ring][row][slot pairs]
-    float2 fbuf[NW][512];
-    float zbuf[NW][256];
-    float nbuf[NW][RB][2][8];
+    float2 z[64 * kFftLd];            // transform (reference n, row r) at n + 8 r
+    float2 tw[kIfftTw];
+    float nb[kMrefRefs][2][8];        // seven samples around the running maxima
 };
 
-// Work of one workgroup: particle p of job j, reference groups gb*NW .. gb*NW+NW-1
-// (the twiddles must already be in sh.tw), rows staged CH rings at a time.  CAND:
-// the candidate form of MrefJob, p is the list index; every slot of an active
-// group gets a record (an empty one for a negative id), and each listed
-// reference's record is the one the exhaustive form computes for it.
-template <int NW, int RW = 4, int RB = 4, int CH = kRingChunk, bool CAND = false>
-__device__ __forceinline__ void mref_block(const MrefJob &j, int p, int gb,
-                                           MrefLds<NW, RW, RB, CH> &sh) {
-    static_assert(RW * RB == 16, "128 accumulators per lane");
-    static_assert(CH % 2 == 0, "rings are taken in pairs within a chunk");
-    constexpr int CH4 = RW * CH * kSlots / 2;   // float4 per staged chunk
-    const int S = j.S, R = j.R, N = j.N;
-    const int tid = threadIdx.x, lane = tid & 63;
-    // uniform over the wavefront: the reference indices and spectrum addresses
-    // built from it live in scalar registers
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = gb * NW + wave;
-    const bool active = g < j.G;
-    const int ps = (CAND && j.pidx) ? j.pidx[p] : p;   // spectra row
-    int nref[RB];
-    bool nval[RB];
-#pragma unroll
-    for (int c = 0; c < RB; ++c) {
-        if (CAND) {
-            // the host validates candidate ids; the clamp keeps every read in bounds
-            const int raw = active ? j.cand[(size_t)p * j.K + g * RB + c] : -1;
-            nval[c] = raw >= 0;
-            nref[c] = min(max(raw, 0), N - 1);
-            if (active && !nval[c] && lane < 8) sh.nbuf[wave][c][0][lane] = 0.0f;
-        } else {
-            const int n = g * RB + c;
-            nval[c] = active && n < N;
-            nref[c] = min(n, N - 1);
-        }
-    }
-    // candidate form: a wavefront whose four slots are all empty only helps stage
-    // the rows, and a workgroup whose slots are all empty skips the rows
-    bool wlive = true, wg_live = true;
-    if (CAND) {
-        wlive = false;
-#pragma unroll
-        for (int c = 0; c < RB; ++c) wlive = wlive || nval[c];
-        wg_live = false;
-        for (int w = 0; w < NW; ++w) {
-            const int gw = gb * NW + w;
-            if (gw >= j.G) break;
-            for (int c = 0; c < RB; ++c) wg_live = wg_live || j.cand[(size_t)p * j.K + gw * RB + c] >= 0;
-        }
-    }
-    float bv[RB][2];
-    int bf[RB][2];
-    float rs0[RB];
-#pragma unroll
-    for (int c = 0; c < RB; ++c) {
-        rs0[c] = j.rsum0[nref[c]];
-        bv[c][0] = bv[c][1] = -3.40282e+38f;
-        bf[c][0] = bf[c][1] = INT_MAX;
-    }
-    const size_t img_stride = (size_t)S * R * kSlots;
-    const int nchunk = (R + CH - 1) / CH;
-    const float2 *abuf = reinterpret_cast<const float2 *>(&sh.abuf4[0][0]);
+// value of the neighbouring lane (lane ^ 1)
+__device__ __forceinline__ float dpp_xor1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+}
 
-    for (int s0 = 0; wg_live && s0 < S; s0 += RW) {
-        const float4 *rows4[RW];
+// f(0), f(1), .., f(N - 1) with compile-time arguments
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
+}
+
+// Reference of column c of tile g (negative: none).  LIST: the candidate form of MrefJob,
+// list p0's K references.
+template <bool LIST>
+__device__ __forceinline__ int mref_ref_at(const MrefJob &j, int p0, int g, int c) {
+    if (LIST) return c < j.K ? j.cand[(size_t)p0 * j.K + c] : -1;
+    return kMrefRefs * g + c < j.N ? kMrefRefs * g + c : -1;
+}
+
+// Contraction wavefront w of a run.  KR: rings of the references kept in registers (at
+// most R).
+template <bool LIST, int KR>
+__device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, int np, int g, MrefLds &sh) {
+    const int S = j.S, R = j.R, N = j.N;
+    const int lane = threadIdx.x & 63;
+    const int f = lane >> 4, u = lane & 15;
+    const int ps = (LIST && j.pidx) ? j.pidx[p0] : p0;   // spectra row of the first particle
+    const int n_rows = np * S;
+    const int n_blk = (n_rows + 7) / 8;
+
+    // operand addresses.  Lane 16 b + i of an instruction: block b (slot), i = 2 t + part;
+    // matrix row pair t holds shift row (t >> 1) + 4 (t & 1), so accumulators 0, 1 of a
+    // block belong to row f and 2, 3 to row 4 + f (f = lane row); columns 2 t + part.
+    const int part = u & 1, t = u >> 1, ar = (t >> 1) + 4 * (t & 1);
+    const unsigned row_bytes = (unsigned)R * (kSlots * 8);
+    const unsigned ring_off = (unsigned)(w * 8 + f * 2 + part) * 16u;   // in a ring row
+    const char *ab = reinterpret_cast<const char *>(j.spec) + (size_t)ps * S * row_bytes;
+    const float sgn = part ? -1.0f : 1.0f;
+    // the host validates candidate ids; the clamp keeps every read in bounds
+    const int ref = min(max(mref_ref_at<LIST>(j, p0, g, t), 0), N - 1);
+    const char *bp = reinterpret_cast<const char *>(j.rspec) + (size_t)ref * row_bytes + ring_off;
+    const float rs0 = j.rsum0[ref];
+
+    // LDS positions: this lane's Z values (reference t, row f or 4 + f; even lanes Z[k],
+    // odd lanes Z[256 - k]) of its wavefront's slots 16 (4 mh + jj) + 4 uq + b, w = 4 mh + uq
+    float2 *zw = sh.z + (t + 8 * f) * kFftLd + part * kMirOff + 64 * (w >> 2) + 4 * (w & 3);
+
+    const char *ablk = ab;   // the block's rows, and this lane's row among them
+    unsigned aoff = (unsigned)min(ar, n_rows - 1) * row_bytes + ring_off;
+    f32x4_t keep[KR > 0 ? KR : 1], rb[kRefPre], ra[kMrefPre];
+    auto load_b = [&](int i) {
+        return *reinterpret_cast<const f32x4_t *>(bp + (size_t)(unsigned)min(i, R - 1) * (kSlots * 8));
+    };
+    auto load_a = [&](int i) {
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(ablk), (short)0, -1, 0x00020000);
+        return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                               rs, aoff, (unsigned)min(i, R - 1) * (kSlots * 8), 0));
+    };
+    static_for<KR>([&](auto ic) { keep[decltype(ic)::value] = load_b(decltype(ic)::value); });
+    static_for<kMrefPre>([&](auto dc) { ra[decltype(dc)::value] = load_a(decltype(dc)::value); });
+    for (int blk = 0; blk < n_blk; ++blk) {
+        float2 nm[2];
 #pragma unroll
-        for (int r = 0; r < RW; ++r)
-            rows4[r] = reinterpret_cast<const float4 *>(j.spec + (size_t)ps * img_stride +
-                                                        (size_t)min(s0 + r, S - 1) * R * kSlots);
-        // Stage one chunk (4 rows x CH rings, 1 KB per row-ring) with direct
-        // global->LDS loads: one wavefront instruction moves one row-ring, each lane
-        // 16 bytes to LDS base + 16*lane.
-        auto load_chunk = [&](int ch, int buf) {
-            for (int rr = wave; rr < RW * CH; rr += NW) {
-                const int ii = rr / RW, r = rr % RW;
-                const int ring = ch * CH + ii;
-                if (ring >= R) continue;
-                __builtin_amdgcn_global_load_lds(
-                    (const void *)(rows4[r] + ring * (kSlots / 2) + lane),
-                    (__attribute__((address_space(3))) void *)(&sh.abuf4[buf][(ii * RW + r) * (kSlots / 2)]),
-                    16, 0, 0);
-            }
+        for (int hh = 0; hh < 2; ++hh)
+            nm[hh] = j.norm[(size_t)ps * S + 8 * (size_t)blk + min(4 * hh + f, n_rows - 1 - 8 * blk)];
+        static_for<kRefPre>([&](auto dc) { rb[decltype(dc)::value] = load_b(KR + decltype(dc)::value); });
+
+        f32x16_t acc[4] = {};
+        auto step = [&](const f32x4_t &a, const f32x4_t &b) {
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+                acc[jj] = __builtin_amdgcn_mfma_f32_16x16x1f32(a[jj], b[jj], acc[jj], 0, 0, 0);
         };
-        float acc[RW][RB][2][4];
-#pragma unroll
-        for (int r = 0; r < RW; ++r)
-#pragma unroll
-            for (int c = 0; c < RB; ++c)
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[r][c][h][e] = 0.0f;
-        // Reference spectra of ring i + 1 load while ring i's FMAs run (ping-pong
-        // registers bA / bB, rings taken in pairs), and the next chunk's rows are
-        // staged from the chunk's last ring on: every load is issued after the
-        // LDS reads of the ring in flight, so the waits the compiler places
-        // before the next LDS reads find them a ring of FMAs old.
-        auto load_refs = [&](int i, float2 (&b)[RB][2]) {
-            if (CAND && !wlive) return;
-#pragma unroll
-            for (int c = 0; c < RB; ++c)
-                load_slots(j.rspec + ((size_t)nref[c] * R + i) * kSlots, lane, b[c][0], b[c][1]);
-        };
-        auto ring = [&](int ii, int buf, const float2 (&b)[RB][2], auto &&issue) {
-            if (CAND && !wlive) {   // uniform over the wavefront: its share of the staging only
-                issue();
-                return;
+        static_for<KR>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            step(ra[i % kMrefPre], keep[i]);
+            ra[i % kMrefPre] = load_a(i + kMrefPre);
+            __builtin_amdgcn_sched_barrier(0);   // keeps the loads ahead of their use
+        });
+        int i0 = KR;
+        for (; i0 + kMrefPre <= R; i0 += kMrefPre)
+            static_for<kMrefPre>([&](auto dc) {
+                constexpr int d = decltype(dc)::value;
+                step(ra[(KR + d) % kMrefPre], rb[d % kRefPre]);
+                rb[d % kRefPre] = load_b(i0 + d + kRefPre);
+                ra[(KR + d) % kMrefPre] = load_a(i0 + d + kMrefPre);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        static_for<kMrefPre - 1>([&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            if (i0 + d < R) {   // uniform
+                if constexpr (d < kRefPre) step(ra[(KR + d) % kMrefPre], rb[d]);
+                else step(ra[(KR + d) % kMrefPre], load_b(i0 + d));
             }
-            float2 a[RW][2];
+        });
+        // the next block's first rings load while this one's cross-spectra go to LDS
+        if (blk + 1 < n_blk) {
+            ablk += 8 * (size_t)row_bytes;
+            aoff = (unsigned)min(ar, n_rows - 9 - 8 * blk) * row_bytes + ring_off;
+        }
+        static_for<kMrefPre>([&](auto dc) { ra[decltype(dc)::value] = load_a(decltype(dc)::value); });
+
+        __syncthreads();   // the transforms of the previous block are done
 #pragma unroll
-            for (int r = 0; r < RW; ++r) {
-                const float2 *ar = abuf + (size_t)buf * (2 * CH4) + (ii * RW + r) * kSlots;
-                load_slots(ar, lane, a[r][0], a[r][1]);
+        for (int hh = 0; hh < 2; ++hh) {
+            const float gs = nm[hh].y;
+            const float gw = (w >= 4 && !part) ? 1.0f : gs;   // Z[64..127] is scaled by the transform
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    // even lanes hold (sr, si) rr = P1, P3 and odd lanes (sr, si) ri = P4, P2 of
+                    // a slot; with the neighbour's values both form C0 and C1:
+                    // Z[k] = (s + t', d + e) in even lanes, Z[256 - k] = (t' - s, e - d) in odd
+                    const float x0 = acc[jj][4 * b + 2 * hh], x1 = acc[jj][4 * b + 2 * hh + 1];
+                    const float y0 = dpp_xor1(x0), y1 = dpp_xor1(x1);
+                    const float ss = x0 + y1, tt = x1 + y0, dd = x0 - y1, ee = y0 - x1;
+                    zw[32 * hh * kFftLd + 16 * jj + b] = f2(gw * fmaf(sgn, ss, tt), gw * fmaf(sgn, dd, ee));
+                }
+            if (w == 0) {   // slot 0 packs the real bins 0 (mean-corrected) and 128
+                const float x0 = acc[0][2 * hh], x1 = acc[0][2 * hh + 1];
+                const float c = gs * (part ? x1 : fmaf(-nm[hh].x, rs0, x0));
+                wave_lds_sync();
+                sh.z[(t + 8 * (4 * hh + f)) * kFftLd + part * (kMirOff + 128)] = f2(c, c);
             }
-            issue();
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < RW; ++r)
-#pragma unroll
-                for (int c = 0; c < RB; ++c)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        acc[r][c][h][0] += b[c][h].x * a[r][h].x;
-                        acc[r][c][h][1] += b[c][h].y * a[r][h].y;
-                        acc[r][c][h][2] += b[c][h].x * a[r][h].y;
-                        acc[r][c][h][3] += b[c][h].y * a[r][h].x;
-                    }
-        };
-        float2 bA[RB][2], bB[RB][2];
-        load_chunk(0, 0);
-        load_refs(0, bA);
-        __builtin_amdgcn_s_waitcnt(0);
+        }
         __syncthreads();
-        for (int ch = 0; ch < nchunk; ++ch) {
-            const int buf = ch & 1;
-            const int i0 = ch * CH, i1 = min(R, i0 + CH);
-            // CH is even, so only the last chunk can end on an unpaired ring
-            for (int i = i0; i < i1; i += 2) {
-                const bool last_pair = i + 2 >= i1;
-                ring(i - i0, buf, bA, [&] {
-                    if (i + 1 < R) load_refs(i + 1, bB);
-                    if (last_pair && i + 1 >= i1 && ch + 1 < nchunk) load_chunk(ch + 1, buf ^ 1);
-                });
-                if (i + 1 < i1)
-                    ring(i + 1 - i0, buf, bB, [&] {
-                        if (i + 2 < R) load_refs(i + 2, bA);
-                        if (last_pair && ch + 1 < nchunk) load_chunk(ch + 1, buf ^ 1);
-                    });
-            }
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-        }
-        if (!active) continue;
-#pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            const int s = s0 + r;
-            if (s >= S) break;
-            const float2 nm = j.norm[(size_t)ps * S + s];
-#pragma unroll
-            for (int c = 0; c < RB; ++c) {
-                if (!nval[c]) continue;
-                psi_update<false>(acc[r][c][0], acc[r][c][1], nm, rs0[c], s, lane, sh.fbuf[wave],
-                                  sh.fbuf[wave] + 256, sh.tw, sh.zbuf[wave], sh.nbuf[wave][c],
-                                  bv[c], bf[c]);
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < RB; ++c) {
-        if (CAND) {
-            if (active)
-                write_rec(j.rec + (size_t)p * j.K + g * RB + c, bv[c], bf[c], sh.nbuf[wave][c], lane);
-        } else if (nval[c]) {
-            write_rec(j.rec + (size_t)p * N + nref[c], bv[c], bf[c], sh.nbuf[wave][c], lane);
-        }
     }
 }
 
-// Multi-reference: one workgroup = one particle x NW groups of 4 references (one
-// group per wavefront).  The workgroup walks the shifts four at a time; the four
-// shift rows' ring spectra are staged cooperatively in LDS in double-buffered
-// chunks of kRingChunk rings, so only the references' spectra come through the
-// vector L1.  Lane l accumulates, over rings, P1..P4 of slots l and l+64 for
-// 4 rows x 4 references (128 accumulators), then each (row, reference) pair goes
-// through psi_update.
-template <int NW, int RW = 4, int RB = 4>
-__global__ __launch_bounds__(NW * 64, 2) void k_ccf_mref(MrefJob j, const float2 *__restrict__ twg) {
-    __shared__ MrefLds<NW, RW, RB> sh;
-    fill_fft_twiddles(sh.tw, twg, threadIdx.x, NW * 64);
-    __syncthreads();
+// Psi wavefront c of a run: column c of the tile.
+template <bool LIST>
+__device__ __forceinline__ void mref_psi(const MrefJob &j, int c, int p0, int np, int g, MrefLds &sh) {
+    const int S = j.S;
+    const int lane = threadIdx.x & 63;
+    const int f = lane >> 4, u = lane & 15;
+    const int ps = (LIST && j.pidx) ? j.pidx[p0] : p0;
+    const int n_rows = np * S;
+    const int n_blk = (n_rows + 7) / 8;
+    const int ref = mref_ref_at<LIST>(j, p0, g, c);
+    PeakState st;
+    st.reset(kNoPeak, INT_MAX);
+    int p = 0, s = 0;   // particle and shift of the next row
+    for (int blk = 0; blk < n_blk; ++blk) {
+        const int rows = min(8, n_rows - 8 * blk);
+        const size_t row0 = (size_t)ps * S + 8 * (size_t)blk;
+        const float gs0 = j.norm[row0 + min(f, rows - 1)].y, gs1 = j.norm[row0 + min(4 + f, rows - 1)].y;
+        __syncthreads();   // the contraction of this block is done
+        __syncthreads();   // and its cross-spectra are in LDS
+        if (ref < 0) continue;   // uniform over the wavefront
+        float2 *xb = sh.z + (c + 8 * f) * kFftLd;
+        for (int hh = 0; 4 * hh < rows; ++hh, xb += 32 * kFftLd) {
+            float2 x[16];
+            ifft256_rows4(x, hh ? gs1 : gs0, xb, sh.tw, u);
+            // the rows may end a particle and begin the next
+            for (int f0 = 0; f0 < min(4, rows - 4 * hh);) {
+                const int cnt = min(min(4, rows - 4 * hh) - f0, S - s);
+                peak_update<false, false>(st, x, f0, cnt, s, lane, xb, sh.nb[c], 0u);
+                f0 += cnt;
+                s += cnt;
+                if (s == S) {
+                    wave_lds_sync();
+                    write_rec(LIST ? j.rec + (size_t)p0 * j.K + c : j.rec + (size_t)(p0 + p) * j.N + ref, st, sh.nb[c],
+                              lane);
+                    wave_lds_sync();
+                    st.reset(kNoPeak, INT_MAX);
+                    s = 0;
+                    ++p;
+                }
+            }
+        }
+    }
+    // an empty slot of a list: an empty record
+    if (LIST && ref < 0 && c < j.K) write_rec(j.rec + (size_t)p0 * j.K + c, st, sh.nb[c], lane);
+}
+
+// Work of one workgroup: reference tile g against particles p0 .. p0 + np - 1 of job j (the
+// twiddles must be in sh.tw by the first barrier).  LIST: list p0 (np = 1), its K
+// references against its particle; every slot of the list gets a record, and each listed
+// reference's record is the one the exhaustive form computes for it.
+template <bool LIST, int KR>
+__device__ __forceinline__ void mref_run(const MrefJob &j, int p0, int np, int g, MrefLds &sh) {
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (w < 8) mref_contract<LIST, KR>(j, w, p0, np, g, sh);
+    else mref_psi<LIST>(j, w - 8, p0, np, g, sh);
+}
+
+// Logical block = run of cp particles x reference tile (fastest).
+template <int KR>
+__global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_mref(MrefJob j, int cp,
+                                                                 const float2 *__restrict__ twg) {
+    __shared__ MrefLds sh;
+    fill_ifft_twiddles(sh.tw, twg, threadIdx.x, kMrefWaves * 64);
     const int lb = xcd_remap(blockIdx.x, gridDim.x);
-    const int p = lb / j.GB;
-    if (p >= j.n_img) return;  // uniform over the workgroup
-    mref_block<NW, RW, RB>(j, p, lb % j.GB, sh);
+    const int ng = (j.N + kMrefRefs - 1) / kMrefRefs;
+    const int p0 = lb / ng * cp;
+    if (p0 >= j.n_img) return;  // uniform over the workgroup
+    mref_run<false, KR>(j, p0, min(cp, j.n_img - p0), lb % ng, sh);
 }
 
 // Candidate re-scoring (the candidate form of MrefJob) by the exhaustive kernel's
-// workgroup code, so every record equals k_ccf_mref's for that (particle,
-// reference): G = K / 4 groups of four listed references, NW per workgroup, GB
-// workgroups per list.  Rows are staged two rings at a time, so that as many
-// workgroups fit the LDS as the registers allow (two wavefronts per SIMD).
-template <int NW>
-__global__ __launch_bounds__(NW * 64, 2) void k_ccf_cand_mref(MrefJob j, const float2 *__restrict__ twg) {
-    __shared__ MrefLds<NW, 4, 4, 2> sh;
-    fill_fft_twiddles(sh.tw, twg, threadIdx.x, NW * 64);
-    __syncthreads();
-    const int p = blockIdx.x / j.GB;
-    if (p >= j.n_img) return;  // uniform over the workgroup
-    mref_block<NW, 4, 4, 2, true>(j, p, blockIdx.x - p * j.GB, sh);
+// workgroup code, so every record equals k_ccf_mref's for that (particle, reference).
+template <int KR>
+__global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_cand(MrefJob j, const float2 *__restrict__ twg) {
+    __shared__ MrefLds sh;
+    fill_ifft_twiddles(sh.tw, twg, threadIdx.x, kMrefWaves * 64);
+    mref_run<true, KR>(j, blockIdx.x, 1, 0, sh);
 }
 
-// Persistent form over many jobs (batched subsets): work items (job, particle,
-// reference block) sit in 8 queues, one per XCD (items of one particle share a
-// queue, so its spectra stay in one L2); each workgroup takes items from the
-// queue of the XCD it runs on (blockIdx % 8) until the queue is exhausted.  The
-// claim is a vector atomic by one lane, broadcast through LDS.  Every workgroup
-// leaves the loop once its queue is empty.  (The one-wavefront tile asks for no
-// occupancy target: its registers leave one wavefront per SIMD either way.)
-template <int NW>
-__global__ __launch_bounds__(NW * 64, NW == 1 ? 1 : 2) void k_ccf_mref_queue(
+// Persistent form over many jobs (batched subsets): work items (job, first particle,
+// reference tile, particles) sit in 8 queues, one per XCD (the tiles of a run share a
+// queue, so its spectra stay in one L2); each workgroup takes items from the queue of
+// the XCD it runs on (blockIdx % 8) until the queue is exhausted.  The claim is a vector
+// atomic by one lane, broadcast through LDS.  Every workgroup leaves the loop once its
+// queue is empty.
+template <int KR>
+__global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_mref_queue(
     const MrefJob *__restrict__ jobs, const int4 *__restrict__ items, const int *__restrict__ qbeg,
     int *__restrict__ counters, const float2 *__restrict__ twg) {
-    __shared__ MrefLds<NW> sh;
+    __shared__ MrefLds sh;
     __shared__ int claim;
-    fill_fft_twiddles(sh.tw, twg, threadIdx.x, NW * 64);
+    fill_ifft_twiddles(sh.tw, twg, threadIdx.x, kMrefWaves * 64);
     const int q = blockIdx.x & 7;
     const int q0 = qbeg[q], q1 = qbeg[q + 1];
     for (;;) {
@@ -1182,8 +1382,8 @@ __global__ __launch_bounds__(NW * 64, NW == 1 ? 1 : 2) void k_ccf_mref_queue(
         __syncthreads();
         const int idx = q0 + claim;
         if (idx >= q1) break;
-        const int4 w = items[idx];
-        mref_block<NW>(jobs[w.x], w.y, w.z, sh);
+        const int4 it = items[idx];
+        mref_run<false, KR>(jobs[it.x], it.y, it.w, it.z, sh);
     }
 }
 
@@ -1277,31 +1477,27 @@ __global__ __launch_bounds__(512) void k_ccf_prop(
     const float2 *__restrict__ rspec, const float *__restrict__ rsum0,
     const PropItem *__restrict__ items, int K, int n_items, int S, int R, int N, int nx, int ny,
     int hw, const float2 *__restrict__ twg, PeakRec *__restrict__ rec) {
-    __shared__ float2 tw[256];
-    __shared__ float2 fbuf[kMaxProposals][512];
-    __shared__ float zbuf[kMaxProposals][256];
+    __shared__ float2 tw[kIfftTw];
+    __shared__ float2 fbuf[kMaxProposals][4 * kFftLd];
     __shared__ float nbuf[kMaxProposals][2][8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    fill_fft_twiddles(tw, twg, tid, blockDim.x);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    fill_ifft_twiddles(tw, twg, tid, blockDim.x);
     __syncthreads();
     const int item = blockIdx.x * K + wave;
     if (item >= n_items) return;
     const int p = item / K;
     const PropItem &it = items[item];
-    float bv[2];
-    int bf[2];
-    bv[0] = bv[1] = -3.40282e+38f;
-    bf[0] = bf[1] = INT_MAX;
+    PeakState st;
+    st.reset(kNoPeak, INT_MAX);
     const int n = it.ref;
     if (n >= 0 && n < N) {
-        unsigned allow = 0u;
+        const int u = lane & 15;
+        unsigned allow = 0u;   // bit 16 m + i: sample u + 16 i of mirror m
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const unsigned wd = it.mask[m * 8 + 2 * q + (lane >> 5)];
-                allow |= ((wd >> (lane & 31)) & 1u) << (m * 4 + q);
-            }
+            for (int i = 0; i < 16; ++i)
+                allow |= ((it.mask[m * 8 + (i >> 1)] >> (u + 16 * (i & 1))) & 1u) << (16 * m + i);
         // window rows j = 0..nr-1 in increasing grid order
         const int ix0 = it.s / ny, iy0 = it.s % ny;
         const int ixa = max(0, ix0 - hw), ixb = min(nx - 1, ix0 + hw);
@@ -1311,6 +1507,7 @@ __global__ __launch_bounds__(512) void k_ccf_prop(
         const float rs0 = rsum0[n];
         const float2 *rb0 = rspec + (size_t)n * R * kSlots;
         const size_t img_stride = (size_t)S * R * kSlots;
+        float2 *xb = fbuf[wave] + (lane >> 4) * kFftLd;
         for (int r0 = 0; r0 < nr; r0 += 3) {
             float acc[3][2][4];
 #pragma unroll
@@ -1324,36 +1521,30 @@ __global__ __launch_bounds__(512) void k_ccf_prop(
             for (int r = 0; r < 3; ++r)
                 arow[r] = spec + (size_t)p * img_stride + (size_t)row(min(r0 + r, nr - 1)) * R * kSlots;
             for (int i = 0; i < R; ++i) {
-                float2 b0v, b1v;
-                load_slots(rb0 + i * kSlots, lane, b0v, b1v);
-                float2 a0s[3], a1s[3];
+                float2 br, bi, ar[3], ai[3];
+                load_pair(rb0 + i * kSlots, lane, br, bi);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) load_slots(arow[r] + i * kSlots, lane, a0s[r], a1s[r]);
+                for (int r = 0; r < 3; ++r) load_pair(arow[r] + i * kSlots, lane, ar[r], ai[r]);
                 __builtin_amdgcn_sched_barrier(0);   // all of the ring's loads in flight before the FMAs
 #pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const float2 a0 = a0s[r], a1 = a1s[r];
-                    acc[r][0][0] += b0v.x * a0.x;
-                    acc[r][0][1] += b0v.y * a0.y;
-                    acc[r][0][2] += b0v.x * a0.y;
-                    acc[r][0][3] += b0v.y * a0.x;
-                    acc[r][1][0] += b1v.x * a1.x;
-                    acc[r][1][1] += b1v.y * a1.y;
-                    acc[r][1][2] += b1v.x * a1.y;
-                    acc[r][1][3] += b1v.y * a1.x;
-                }
+                for (int r = 0; r < 3; ++r) pair_fma(acc[r], br, bi, ar[r], ai[r]);
             }
+            wave_lds_sync();
+            float2 nm[3];
 #pragma unroll
             for (int r = 0; r < 3; ++r) {
-                if (r0 + r >= nr) break;
-                const int s = row(r0 + r);
-                psi_update<false, true>(acc[r][0], acc[r][1], norm[(size_t)p * S + s], rs0, s, lane,
-                                        fbuf[wave], fbuf[wave] + 256, tw, zbuf[wave], nbuf[wave], bv,
-                                        bf, allow);
+                nm[r] = norm[(size_t)p * S + row(min(r0 + r, nr - 1))];
+                store_pair_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
             }
+            wave_lds_sync();
+            float2 x[16];
+            ifft256_rows4(x, lane_row_of(nm[0].y, nm[1].y, nm[2].y, 0.0f, lane), xb, tw, u);
+            // window rows are not consecutive shifts: one at a time
+            for (int r = 0; r < min(3, nr - r0); ++r)
+                peak_update<false, true>(st, x, r, 1, row(r0 + r), lane, xb, nbuf[wave], allow);
         }
     }
-    write_rec(rec + item, bv, bf, nbuf[wave], lane);
+    write_rec(rec + item, st, nbuf[wave], lane);
 }
 
 // Is (m, s, t) of reference `ref` admitted by one of the particle's items?
@@ -2123,30 +2314,42 @@ hipError_t launch_ref_finalize(float2 *rspec, const float2 *rnorm, int n_ref, in
     return hipGetLastError();
 }
 
-// Tile of the single-job search: kMrefNW wavefronts per workgroup, each with
-// kMrefRW shift rows x kMrefRB references.
-constexpr int kMrefNW = 4, kMrefRW = 4, kMrefRB = 4;
-
-template <int NW>
-static hipError_t launch_mref_nw(const MrefJob &j, const float2 *tw, hipStream_t st) {
-    const long long blocks = (long long)j.n_img * j.GB;
-    hipLaunchKernelGGL((k_ccf_mref<NW, kMrefRW, kMrefRB>), dim3((unsigned)blocks), dim3(NW * 64), 0,
-                       st, j, tw);
-    return hipGetLastError();
+// Particles per workgroup of the search, 1, 2, 4 or 8: a run of cp particles fills
+// ceil(cp S / 8) row blocks (8 particles fill S without a partial block), and the
+// device holds one workgroup per CU at a time.  The count with the fewest block steps
+// (rounds of workgroups x blocks of each) wins, at equal cost the larger run.  4 096 x
+// 100 at 76 px, 49 shifts: 13.5 ms with 8, 14.3 with 4, 15.5 with 1 (7 blocks for 6.1);
+// small searches take 1, so that every CU has work.
+static int particles_per_workgroup(int n_img, int S, int N) {
+    const long long ng = (N + kMrefRefs - 1) / kMrefRefs, cus = 256;
+    int best = 1;
+    long long best_cost = LLONG_MAX;
+    for (int cp = 1; cp <= 8; cp *= 2) {
+        const long long wgs = ((long long)n_img + cp - 1) / cp * ng;
+        const long long cost = (wgs + cus - 1) / cus * (((long long)cp * S + 7) / 8);
+        if (cost <= best_cost) {
+            best_cost = cost;
+            best = cp;
+        }
+    }
+    return best;
 }
 
 hipError_t launch_ccf_mref(const float2 *spec, const float2 *norm, const float2 *rspec,
                            const float *rsum0, int n_img, int n_shift, int n_ring, int n_ref,
                            const float2 *twiddle, PeakRec *rec, hipStream_t st) {
     if (n_img <= 0 || n_ref <= 0) return hipSuccess;
-    MrefJob j = mref_job(spec, norm, rspec, rsum0, rec, n_img, n_shift, n_ring, n_ref, kMrefNW);
-    j.G = (n_ref + kMrefRB - 1) / kMrefRB;   // groups of kMrefRB references, one per wavefront
-    j.GB = (j.G + kMrefNW - 1) / kMrefNW;
-    return launch_mref_nw<kMrefNW>(j, twiddle, st);
+    const MrefJob j = mref_job(spec, norm, rspec, rsum0, rec, n_img, n_shift, n_ring, n_ref);
+    const int cp = particles_per_workgroup(n_img, n_shift, n_ref);
+    const long long blocks = (long long)((n_img + cp - 1) / cp) * ((n_ref + kMrefRefs - 1) / kMrefRefs);
+    const dim3 grid((unsigned)blocks), wg(kMrefWaves * 64);
+    if (n_ring >= kMrefKeep) hipLaunchKernelGGL(k_ccf_mref<kMrefKeep>, grid, wg, 0, st, j, cp, twiddle);
+    else hipLaunchKernelGGL(k_ccf_mref<0>, grid, wg, 0, st, j, cp, twiddle);
+    return hipGetLastError();
 }
 
 MrefJob mref_job(const float2 *spec, const float2 *norm, const float2 *rspec, const float *rsum0,
-                 PeakRec *rec, int n_img, int n_shift, int n_ring, int n_ref, int nw) {
+                 PeakRec *rec, int n_img, int n_shift, int n_ring, int n_ref) {
     MrefJob j;
     j.spec = spec;
     j.norm = norm;
@@ -2157,36 +2360,27 @@ MrefJob mref_job(const float2 *spec, const float2 *norm, const float2 *rspec, co
     j.S = n_shift;
     j.R = n_ring;
     j.N = n_ref;
-    j.G = (n_ref + 3) / 4;
-    j.GB = (j.G + nw - 1) / nw;
     return j;
 }
 
-int mref_queue_blocks_per_cu(int nw) {
+int mref_queue_blocks_per_cu() {
     int n = 0;
-    hipError_t e = hipErrorInvalidValue;
-    if (nw == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_ccf_mref_queue<1>, 64, 0);
-    if (nw == 2) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_ccf_mref_queue<2>, 128, 0);
-    if (nw == 4) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_ccf_mref_queue<4>, 256, 0);
+    const hipError_t e =
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_ccf_mref_queue<kMrefKeep>, kMrefWaves * 64, 0);
     return e == hipSuccess ? n : 0;
 }
 
 hipError_t launch_ccf_mref_queue(const MrefJob *jobs, const int4 *items, const int *qbeg,
-                                 int *counters, int nw, int blocks, const float2 *twiddle,
+                                 int *counters, int blocks, int min_ring, const float2 *twiddle,
                                  hipStream_t st) {
-    if (nw != 1 && nw != 2 && nw != 4) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, counters, 8);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (nw == 1)
-        hipLaunchKernelGGL((k_ccf_mref_queue<1>), dim3(blocks), dim3(64), 0, st, jobs, items, qbeg,
-                           counters, twiddle);
-    else if (nw == 2)
-        hipLaunchKernelGGL((k_ccf_mref_queue<2>), dim3(blocks), dim3(128), 0, st, jobs, items, qbeg,
-                           counters, twiddle);
+    const dim3 grid(blocks), wg(kMrefWaves * 64);
+    if (min_ring >= kMrefKeep)
+        hipLaunchKernelGGL(k_ccf_mref_queue<kMrefKeep>, grid, wg, 0, st, jobs, items, qbeg, counters, twiddle);
     else
-        hipLaunchKernelGGL((k_ccf_mref_queue<4>), dim3(blocks), dim3(256), 0, st, jobs, items, qbeg,
-                           counters, twiddle);
+        hipLaunchKernelGGL(k_ccf_mref_queue<0>, grid, wg, 0, st, jobs, items, qbeg, counters, twiddle);
     return hipGetLastError();
 }
 
@@ -2195,9 +2389,8 @@ hipError_t launch_ccf_single(const float2 *spec, const float2 *norm, const float
                              int n_shift, int n_ring, int n_ref, const float2 *twiddle,
                              PeakRec *rec, hipStream_t st) {
     if (n_img <= 0) return hipSuccess;
-    const int blocks = (n_img + 3) / 4;
-    hipLaunchKernelGGL(k_ccf_items<true>, dim3(blocks), dim3(256), 0, st, spec, norm, rspec, rsum0,
-                       ref_of, ref_stride, 1, n_img, n_shift, n_ring, n_ref, twiddle, rec, nullptr);
+    hipLaunchKernelGGL(k_ccf_single, dim3((n_img + 3) / 4), dim3(256), 0, st, spec, norm, rspec, rsum0,
+                       ref_of, ref_stride, n_img, n_shift, n_ring, n_ref, twiddle, rec);
     return hipGetLastError();
 }
 
@@ -2205,24 +2398,15 @@ hipError_t launch_ccf_candidates(const float2 *spec, const float2 *norm, const f
                                  const float *rsum0, const int *cand, int K, int n_img,
                                  int n_shift, int n_ring, int n_ref, const float2 *twiddle,
                                  PeakRec *rec, hipStream_t st, const int *pidx) {
-    const int items = n_img * K;
-    if (items <= 0) return hipSuccess;
-    if (K == 4 || K == 8) {   // one workgroup per list, one wavefront per 4 slots
-        MrefJob j = mref_job(spec, norm, rspec, rsum0, rec, n_img, n_shift, n_ring, n_ref, 1);
-        j.cand = cand;
-        j.pidx = pidx;
-        j.K = K;
-        j.G = K / 4;
-        j.GB = 1;
-        const dim3 grid((unsigned)n_img);
-        if (K == 4)
-            hipLaunchKernelGGL(k_ccf_cand_mref<1>, grid, dim3(64), 0, st, j, twiddle);
-        else
-            hipLaunchKernelGGL(k_ccf_cand_mref<2>, grid, dim3(128), 0, st, j, twiddle);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL(k_ccf_items<false>, dim3((items + 3) / 4), dim3(256), 0, st, spec, norm,
-                       rspec, rsum0, cand, 1, K, items, n_shift, n_ring, n_ref, twiddle, rec, pidx);
+    if (n_img <= 0 || K <= 0) return hipSuccess;
+    if (K > kMrefRefs) return hipErrorInvalidValue;
+    MrefJob j = mref_job(spec, norm, rspec, rsum0, rec, n_img, n_shift, n_ring, n_ref);
+    j.cand = cand;
+    j.pidx = pidx;
+    j.K = K;
+    const dim3 grid((unsigned)n_img), wg(kMrefWaves * 64);
+    if (n_ring >= kMrefKeep) hipLaunchKernelGGL(k_ccf_cand<kMrefKeep>, grid, wg, 0, st, j, twiddle);
+    else hipLaunchKernelGGL(k_ccf_cand<0>, grid, wg, 0, st, j, twiddle);
     return hipGetLastError();
 }
 

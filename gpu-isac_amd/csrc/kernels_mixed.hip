@@ -200,9 +200,10 @@ __global__ __launch_bounds__(256) void k_frag_rows(const float2 *__restrict__ sp
     const int row = p * S + s;
     const float2 nm = norm[row];
     const float gs = nm.y * cp;
-    const float2 *src = spec + (size_t)row * R * kSlots + slot_pos(k);
+    const float *src = reinterpret_cast<const float *>(spec + (size_t)row * R * kSlots) + slot_re(k);
     write_operand<BF16>(rowp, k, R, g, [&](int part, int i) {
-        const float2 x = src[(size_t)i * kSlots];
+        const float *q = src + (size_t)i * 2 * kSlots;
+        const float2 x = make_float2(q[0], q[kPartOff]);
         if (k == 0) return part ? x.y * gs : (x.x - nm.x) * gs;   // S[0] - mu L, S[128]
         return part ? (x.x - x.y) * gs : (x.x + x.y) * gs;
     });
@@ -215,8 +216,9 @@ __global__ __launch_bounds__(256) void k_ref_scale(const float2 *__restrict__ rs
     const int n = blockIdx.x;
     double ss = 0.0;
     for (int e = threadIdx.x; e < R * kSlots; e += blockDim.x) {
-        const float2 x = rspec[(size_t)n * R * kSlots + e];
-        const int k = e % kSlots;   // slot_pos(0) == 0: position 0 is slot 0
+        const int i = e / kSlots, o = e % kSlots, k = (o >> 1) + 64 * (o & 1);
+        const float *q = reinterpret_cast<const float *>(rspec + ((size_t)n * R + i) * kSlots) + slot_re(k);
+        const float2 x = make_float2(q[0], q[kPartOff]);
         if (k == 0) ss += (double)x.x * x.x + (double)x.y * x.y;
         else ss += 2.0 * ((double)x.x * x.x + (double)x.y * x.y);
     }
@@ -251,9 +253,10 @@ __global__ __launch_bounds__(256) void k_frag_refs(const float2 *__restrict__ rs
         return;
     }
     const float c = cn[n];
-    const float2 *src = rspec + (size_t)n * R * kSlots + slot_pos(k);
+    const float *src = reinterpret_cast<const float *>(rspec + (size_t)n * R * kSlots) + slot_re(k);
     write_operand<BF16>(rowp, k, R, g, [&](int part, int i) {
-        const float2 x = src[(size_t)i * kSlots];
+        const float *q = src + (size_t)i * 2 * kSlots;
+        const float2 x = make_float2(q[0], q[kPartOff]);
         if (k == 0) return part ? x.y * c : x.x * c;              // R[0], R[128]
         return part ? (x.x - x.y) * c : (x.x + x.y) * c;
     });

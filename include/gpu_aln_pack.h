@@ -267,8 +267,8 @@ typedef struct IsacMrefSubset {
 /* No counterpart in the reference.  Aligns n_subsets independent subsets of
  * uneven particle count, box size, reference count, ring count and shift range;
  * results are bit-identical to one isac_mref_align_device call per subset.  In
- * ISAC_BATCH_GRAPH mode the tile shape (waves per workgroup) of each memory
- * group is chosen by timing the candidates on a sample of the group, and the
+ * ISAC_BATCH_GRAPH mode the particles per work item (1, 2 or 4) of each memory
+ * group are chosen by timing the candidates on a sample of the group, and the
  * captured graph is kept and replayed while the descriptor array is unchanged
  * (same pointers and shapes; the data behind them may change).  Returns after
  * the work has completed. */
@@ -277,8 +277,8 @@ int isac_mref_align_batched_device(const IsacMrefSubset *subsets, unsigned int n
 
 /* No counterpart in the reference.  What the last ISAC_BATCH_GRAPH call did:
  * memory groups, graph nodes, whether the graph was replayed from the cache,
- * and for the first group the chosen waves per workgroup, the persistent grid
- * size and the timed sample (ms) for 1, 2 and 4 waves. */
+ * and for the first group the chosen candidate (nw: particles per work item, 1, 2 or
+ * 4), the persistent grid size and the timed sample (ms) of each candidate. */
 void isac_batched_report(int *n_groups, int *n_nodes, int *replayed, int *nw, int *blocks,
                          float *cand_ms3);
 
