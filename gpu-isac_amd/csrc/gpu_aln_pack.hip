@@ -97,7 +97,7 @@ struct DevBuf {
 // Batched multi-reference run: concatenated per-subset tables, the group
 // workspace, work-queue tables and the captured graph (kept for replay).
 struct BatchWs {
-    DevBuf shifts_i, shifts_f, tmpl, rspec, rnorm, rsum0;   // per-subset tables
+    DevBuf shifts_i, shifts_f, tmpl, rspec, rsum0;   // per-subset tables
     DevBuf spec, norm, rec;                                // group workspace
     DevBuf jobs, items, qbeg, counters;                    // work queues of every group
     hipGraph_t graph = nullptr;
@@ -115,7 +115,7 @@ struct BatchWs {
     }
     void release() {
         drop_graph();
-        DevBuf *all[] = {&shifts_i, &shifts_f, &tmpl, &rspec, &rnorm, &rsum0, &spec, &norm,
+        DevBuf *all[] = {&shifts_i, &shifts_f, &tmpl, &rspec, &rsum0, &spec, &norm,
                          &rec, &jobs, &items, &qbeg, &counters};
         for (DevBuf *b : all) b->release();
         tuned.clear();
@@ -128,8 +128,8 @@ struct Workspace {
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;   // host-to-device copies overlapped with the search
     int tmpl_rings = 0;
-    DevBuf tmpl, twiddle, zero_shift, shifts_i, shifts_f;
-    DevBuf spec, norm, rspec, rnorm, rsum0, rec;
+    DevBuf tmpl, twiddle, shifts_i, shifts_f;
+    DevBuf spec, norm, rspec, rsum0, rec;
     DevBuf peak, dvals, acc;
     DevBuf mix_p, mix_pn, mix_r, mix_rn;   // 16-bit MFMA operands and row norms
     DevBuf cand, rec_c, best, second, tie, val64;   // candidate re-scoring
@@ -141,8 +141,8 @@ struct Workspace {
     BatchWs batch;
     void release() {
         batch.release();
-        DevBuf *all[] = {&tmpl, &twiddle, &zero_shift, &shifts_i, &shifts_f, &spec, &norm,
-                         &rspec, &rnorm, &rsum0, &rec, &peak, &dvals, &acc,
+        DevBuf *all[] = {&tmpl, &twiddle, &shifts_i, &shifts_f, &spec, &norm,
+                         &rspec, &rsum0, &rec, &peak, &dvals, &acc,
                          &mix_p, &mix_pn, &mix_r, &mix_rn, &cand, &rec_c, &best, &second,
                          &tie, &val64, &items, &smask, &fb_idx, &fb_count, &fb_img, &fb_acc,
                          &edge, &smask2, &pre_tp, &pre_mir, &pre_part, &pre_avg, &pre_shift,
@@ -227,8 +227,6 @@ int ensure_device_ws(int dev) {
         }
         HIP_OK(ws.twiddle.reserve(256 * sizeof(float2)));
         HIP_OK(hipMemcpy(ws.twiddle.p, tw.data(), 256 * sizeof(float2), hipMemcpyHostToDevice));
-        HIP_OK(ws.zero_shift.reserve(sizeof(int2)));
-        HIP_OK(hipMemset(ws.zero_shift.p, 0, sizeof(int2)));
     }
     return 0;
 }
@@ -321,13 +319,9 @@ struct ProfScope {
 // Reference spectra (centre D//2, no shift), normalised and ring-weighted.
 int ref_spectra(const float *d_ref, int N, int D, int R, hipStream_t st) {
     HIP_OK(ws.rspec.reserve((size_t)N * R * kSlots * sizeof(float2)));
-    HIP_OK(ws.rnorm.reserve((size_t)N * sizeof(float2)));
     HIP_OK(ws.rsum0.reserve((size_t)N * sizeof(float)));
-    HIP_OK(isac::launch_polar_spectra(d_ref, N, D, ShiftView{nullptr, 0}, ws.zero_shift.as<int2>(),
-                                      1, ws.tmpl.as<float2>(), R, ws.twiddle.as<float2>(),
-                                      ws.rspec.as<float2>(), ws.rnorm.as<float2>(), st));
-    HIP_OK(isac::launch_ref_finalize(ws.rspec.as<float2>(), ws.rnorm.as<float2>(), N, R,
-                                     ws.rsum0.as<float>(), st));
+    HIP_OK(isac::launch_ref_spectra(d_ref, N, D, ws.tmpl.as<float2>(), R, ws.twiddle.as<float2>(),
+                                    ws.rspec.as<float2>(), ws.rsum0.as<float>(), st));
     return 0;
 }
 
@@ -914,7 +908,6 @@ int batch_plan(const IsacMrefSubset *d, unsigned n, std::vector<BatchSub> &subs,
     HIP_OK(b.shifts_f.reserve(shf.size() * sizeof(float2)));
     HIP_OK(b.tmpl.reserve(tm.size() * sizeof(float2)));
     HIP_OK(b.rspec.reserve(rs * sizeof(float2)));
-    HIP_OK(b.rnorm.reserve(rn * sizeof(float2)));
     HIP_OK(b.rsum0.reserve(rn * sizeof(float)));
     HIP_OK(hipMemcpy(b.shifts_i.p, shi.data(), shi.size() * sizeof(int2), hipMemcpyHostToDevice));
     HIP_OK(hipMemcpy(b.shifts_f.p, shf.data(), shf.size() * sizeof(float2), hipMemcpyHostToDevice));
@@ -971,13 +964,9 @@ int batch_record(const std::vector<BatchSub> &subs, const std::vector<BatchGroup
                  hipStream_t st) {
     BatchWs &b = ws.batch;
     for (const BatchSub &u : subs) {
-        HIP_OK(isac::launch_polar_spectra(u.u->d_ref, u.N, u.D, ShiftView{nullptr, 0},
-                                          ws.zero_shift.as<int2>(), 1, b.tmpl.as<float2>() + u.tm_off,
-                                          u.R, ws.twiddle.as<float2>(), b.rspec.as<float2>() + u.rs_off,
-                                          b.rnorm.as<float2>() + u.rn_off, st));
-        HIP_OK(isac::launch_ref_finalize(b.rspec.as<float2>() + u.rs_off,
-                                         b.rnorm.as<float2>() + u.rn_off, u.N, u.R,
-                                         b.rsum0.as<float>() + u.rn_off, st));
+        HIP_OK(isac::launch_ref_spectra(u.u->d_ref, u.N, u.D, b.tmpl.as<float2>() + u.tm_off, u.R,
+                                        ws.twiddle.as<float2>(), b.rspec.as<float2>() + u.rs_off,
+                                        b.rsum0.as<float>() + u.rn_off, st));
     }
     for (size_t gi = 0; gi < groups.size(); ++gi) {
         const BatchGroup &gr = groups[gi];
@@ -1026,13 +1015,9 @@ int run_batched_graph(const IsacMrefSubset *d, unsigned n, hipStream_t st) {
     HIP_OK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
     // reference spectra first (the tuning sample needs them)
     for (const BatchSub &u : subs) {
-        HIP_OK(isac::launch_polar_spectra(u.u->d_ref, u.N, u.D, ShiftView{nullptr, 0},
-                                          ws.zero_shift.as<int2>(), 1, b.tmpl.as<float2>() + u.tm_off,
-                                          u.R, ws.twiddle.as<float2>(), b.rspec.as<float2>() + u.rs_off,
-                                          b.rnorm.as<float2>() + u.rn_off, ws.stream));
-        HIP_OK(isac::launch_ref_finalize(b.rspec.as<float2>() + u.rs_off,
-                                         b.rnorm.as<float2>() + u.rn_off, u.N, u.R,
-                                         b.rsum0.as<float>() + u.rn_off, ws.stream));
+        HIP_OK(isac::launch_ref_spectra(u.u->d_ref, u.N, u.D, b.tmpl.as<float2>() + u.tm_off, u.R,
+                                        ws.twiddle.as<float2>(), b.rspec.as<float2>() + u.rs_off,
+                                        b.rsum0.as<float>() + u.rn_off, ws.stream));
     }
     for (size_t gi = 0; gi < groups.size(); ++gi)
         if (int e = tune_group(subs, groups[gi], n_cu, gi == 0, ws.stream)) return e;
@@ -1305,7 +1290,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Byte offsets of the regions of the scratch array for one call.
 struct NoAllocLayout {
-    size_t twiddle, tmpl, zero_shift, shifts_i, shifts_f, rspec, rnorm, rsum0;
+    size_t twiddle, tmpl, shifts_i, shifts_f, rspec, rsum0;
     size_t spec, norm, rec;   // one particle batch of pb particles
     size_t end;
     int pb;
@@ -1318,11 +1303,9 @@ NoAllocLayout noalloc_layout(int N, int R, int S, int P) {
     auto take = [&](size_t bytes) { const size_t at = o; o += align256(bytes); return at; };
     L.twiddle = take(256 * sizeof(float2));
     L.tmpl = take((size_t)R * kRingLen * sizeof(float2));
-    L.zero_shift = take(sizeof(int2));
     L.shifts_i = take((size_t)S * sizeof(int2));
     L.shifts_f = take((size_t)S * sizeof(float2));
     L.rspec = take((size_t)N * R * kSlots * sizeof(float2));
-    L.rnorm = take((size_t)N * sizeof(float2));
     L.rsum0 = take((size_t)N * sizeof(float));
     const size_t fixed = o;
     auto batch_bytes = [&](size_t pb) {
@@ -1401,12 +1384,10 @@ int run_mref_noalloc(const float *d_sbj, const float *d_ref, ShiftView acc, int 
     const std::vector<float2> tm = make_template(R);
     std::vector<int2> si(shifts.size());
     for (size_t i = 0; i < shifts.size(); ++i) si[i] = make_int2((int)shifts[i].x, (int)shifts[i].y);
-    const int2 zero{0, 0};
     auto at = [&](size_t off) { return static_cast<void *>(base + off); };
     HIP_OK(hipMemcpyAsync(at(L.twiddle), tw.data(), 256 * sizeof(float2), hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(at(L.tmpl), tm.data(), tm.size() * sizeof(float2), hipMemcpyHostToDevice,
                           st));
-    HIP_OK(hipMemcpyAsync(at(L.zero_shift), &zero, sizeof(int2), hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(at(L.shifts_i), si.data(), si.size() * sizeof(int2),
                           hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(at(L.shifts_f), shifts.data(), shifts.size() * sizeof(float2),
@@ -1414,17 +1395,13 @@ int run_mref_noalloc(const float *d_sbj, const float *d_ref, ShiftView acc, int 
     const float2 *twd = static_cast<const float2 *>(at(L.twiddle));
     const float2 *tmpl = static_cast<const float2 *>(at(L.tmpl));
     float2 *rspec = static_cast<float2 *>(at(L.rspec));
-    float2 *rnorm = static_cast<float2 *>(at(L.rnorm));
     float *rsum0 = static_cast<float *>(at(L.rsum0));
     float2 *spec = static_cast<float2 *>(at(L.spec));
     float2 *norm = static_cast<float2 *>(at(L.norm));
     PeakRec *rec = static_cast<PeakRec *>(at(L.rec));
     const int2 *shi = static_cast<const int2 *>(at(L.shifts_i));
     const float2 *shf = static_cast<const float2 *>(at(L.shifts_f));
-    HIP_OK(isac::launch_polar_spectra(d_ref, N, D, ShiftView{nullptr, 0},
-                                      static_cast<const int2 *>(at(L.zero_shift)), 1, tmpl, R, twd,
-                                      rspec, rnorm, st));
-    HIP_OK(isac::launch_ref_finalize(rspec, rnorm, N, R, rsum0, st));
+    HIP_OK(isac::launch_ref_spectra(d_ref, N, D, tmpl, R, twd, rspec, rsum0, st));
     for (int p0 = 0; p0 < P; p0 += L.pb) {
         const int n = std::min(L.pb, P - p0);
         ShiftView a = acc;

@@ -155,10 +155,10 @@ hipError_t launch_polar_spectra(const float *imgs, int n_img, int img_dim, Shift
                                 int n_ring, const float2 *twiddle, float2 *spec, float2 *norm,
                                 hipStream_t st);
 
-// Normalise and ring-weight reference spectra in place (n_shift == 1 layout);
+// Reference spectra rspec[n][ring][kSlots], normalised and ring-weighted;
 // rsum0[n] = sum_i w_i R'_i[0] (needed for the particle DC correction).
-hipError_t launch_ref_finalize(float2 *rspec, const float2 *rnorm, int n_ref, int n_ring,
-                               float *rsum0, hipStream_t st);
+hipError_t launch_ref_spectra(const float *imgs, int n_ref, int img_dim, const float2 *tmpl, int n_ring,
+                              const float2 *twiddle, float2 *rspec, float *rsum0, hipStream_t st);
 
 // Stage B, multi-reference: every particle x every reference; rec[p*n_ref + n].
 hipError_t launch_ccf_mref(const float2 *spec, const float2 *norm, const float2 *rspec,

@@ -3,10 +3,12 @@
 // Data layout in HBM:
 //   images       [n][D][D] float32, row-major (y, x)
 //   spec         [n][S][R][128] float2: raw ring spectra of every image at every
-//                grid shift, packed: slot 0 = (X[0], X[128]), slot k = X[k], k=1..127
+//                grid shift, slot 0 = (X[0], X[128]), slot k = X[k], k=1..127; the
+//                order of the slots' parts within a row is slot_re's
 //   norm         [n][S] float2 = (mu*L, 1/(sd+1e-7)) of the radius-weighted
 //                normalisation (reference cuda/gpu_aln_noref.cu:1294-1351)
-//   rspec        [N][R][128] float2: reference spectra, normalised and weighted (i+1)
+//   rspec        [N][R][128] float2: reference spectra, normalised and weighted (i+1),
+//                rows as those of spec
 //   rec          PeakRec per (particle, reference)
 // The reference's psi-CCF table (particles x refs x shifts x 2 x (L+2) floats,
 // cuda/gpu_aln_noref.cu:2343-2461) is never materialised: the contraction over
@@ -14,6 +16,7 @@
 // fused in registers / LDS of one wavefront.
 #include "isac_internal.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <cmath>
@@ -130,19 +133,6 @@ __device__ __forceinline__ float bilinear(const float *img, int D, float x, floa
     return (1.0f - fy) * ((1.0f - fx) * v00 + fx * v01) + fy * ((1.0f - fx) * v10 + fx * v11);
 }
 
-// The same sample from an LDS copy of the image with a one-pixel border that
-// repeats the edge (row / column c of the copy holds pixel clamp(c - 1)): the
-// left / upper tap is clamped to -1 .. D - 1 and both taps of a row are adjacent
-// words (one ds_read2 per row), with exactly the values and weights above.
-__device__ __forceinline__ float bilinear_bordered(const float *pimg, int D, float x, float y) {
-    const float x0 = floorf(x), y0 = floorf(y);
-    const float fx = x - x0, fy = y - y0;
-    const int cx = min(max((int)x0, -1), D - 1) + 1, cy = min(max((int)y0, -1), D - 1) + 1;
-    const float *q = pimg + cy * (D + 2) + cx;
-    const float v00 = q[0], v01 = q[1], v10 = q[D + 2], v11 = q[D + 3];
-    return (1.0f - fy) * ((1.0f - fx) * v00 + fx * v01) + fy * ((1.0f - fx) * v10 + fx * v11);
-}
-
 // Blocks are dispatched round-robin over the 8 XCDs; remap so that consecutive
 // logical blocks (which share particle spectra) run on the same XCD and L2.
 __device__ __forceinline__ int xcd_remap(int b, int nb) {
@@ -151,65 +141,273 @@ __device__ __forceinline__ int xcd_remap(int b, int nb) {
     return (xcd < r) ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
-// Stores a wavefront's slots lane (lo) and lane + 64 (hi) of one ring row in the
-// operand order of slot_re: a 4 x 4 transpose between the four 16-lane rows and the
-// four parts (2 + 2 lane-row swaps), then one 16-byte store per lane.
-__device__ __forceinline__ void swap32(float &a, float &b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]);
-    b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void swap16(float &a, float &b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]);
-    b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void store_ring(float2 *row, int lane, float2 lo, float2 hi) {
-    float r0 = lo.x, r1 = lo.y, r2 = hi.x, r3 = hi.y;
-    swap32(r0, r2);
-    swap32(r1, r3);
-    swap16(r0, r1);
-    swap16(r2, r3);
-    // lane row 0 / 1: real / imaginary parts of slots u + 16 j, 2 / 3: of slots 64 on
-    const int g = lane >> 4, u = lane & 15;
-    reinterpret_cast<float4 *>(row)[(g >> 1) * 32 + u * 2 + (g & 1)] = make_float4(r0, r1, r2, r3);
-}
-
 // One slot of a ring row.
 __device__ __forceinline__ float2 load_slot(const float2 *row, int k) {
     const float *q = reinterpret_cast<const float *>(row) + slot_re(k);
     return make_float2(q[0], q[kPartOff]);
 }
 
+// Transforms over 16 lanes, four per wavefront: the twiddles of the last two stages.
+constexpr int kIfftTw = 15 * 16;  // lane twiddles of the last two stages
+
+// entry q - 1: stage 3, e^{-2 pi i 4 q u / 256}; entry 3 + 3 q3 + q - 1: stage 4,
+// e^{-2 pi i q (u + 16 q3) / 256}
+__device__ __forceinline__ void fill_ifft_twiddles(float2 *tw, const float2 *twg, int tid, int nthreads) {
+    for (int i = tid; i < kIfftTw; i += nthreads) {
+        const int e = i >> 4, u = i & 15;
+        tw[i] = e < 3 ? twg[4 * (e + 1) * u] : twg[((e - 3) % 3 + 1) * (u + 16 * ((e - 3) / 3))];
+    }
+}
+
+// v conj(w), with the operation order of cmul under INV
+__device__ __forceinline__ float2 cmulc(float2 v, float2 w) {
+    return f2(fmaf(v.x, w.x, v.y * w.y), fmaf(v.y, w.x, -(v.x * w.y)));
+}
+
+// cos, sin of -2 pi m / 256 for the m = 16 q k of the second stage (the table's values)
+__device__ __forceinline__ constexpr float2 stage2_tw(int m) {
+    return m == 16    ? float2{0.92387953251128674f, -0.38268343236508977f}
+           : m == 32  ? float2{0.70710678118654757f, -0.70710678118654757f}
+           : m == 48  ? float2{0.38268343236508984f, -0.92387953251128674f}
+           : m == 64  ? float2{6.123233995736766e-17f, -1.0f}
+           : m == 96  ? float2{-0.70710678118654746f, -0.70710678118654757f}
+                      : float2{-0.92387953251128685f, 0.38268343236508967f};   // m == 144
+}
+
+// v w, the rounding of cmul
+__device__ __forceinline__ float2 cmulf(float2 v, float2 w) {
+    return f2(fmaf(v.x, w.x, -(v.y * w.y)), fmaf(v.y, w.x, v.x * w.y));
+}
+
+// Last two radix-4 stages of a 256-point transform over 16 lanes, x[a] = point u + 16 a
+// after the second stage in, natural order u + 16 m out.
+template <bool INV>
+__device__ __forceinline__ void fft256_tail(float2 (&x)[16], const float2 *tw, int u) {
+    float2 w3[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) w3[q] = tw[q * 16 + u];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {      // stage 3, butterfly 16 h + u
+        float2 v[4] = {x[h], x[h + 4], x[h + 8], x[h + 12]};
+#pragma unroll
+        for (int q = 1; q < 4; ++q) v[q] = INV ? cmulc(v[q], w3[q - 1]) : cmulf(v[q], w3[q - 1]);
+        radix4<INV>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[h + 4 * q] = v[q];
+    }
+#pragma unroll
+    for (int q3 = 0; q3 < 4; ++q3) {   // stage 4, butterfly u + 16 q3
+        float2 v[4] = {x[4 * q3], x[4 * q3 + 1], x[4 * q3 + 2], x[4 * q3 + 3]};
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+            const float2 w4 = tw[(3 + 3 * q3 + q - 1) * 16 + u];
+            v[q] = INV ? cmulc(v[q], w4) : cmulf(v[q], w4);
+        }
+        radix4<INV>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[4 * q3 + q] = v[q];
+    }
+    // x[4 q3 + q] = z[u + 16 q3 + 64 q]: to natural order
+    float2 y[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) y[m] = x[4 * (m & 3) + (m >> 2)];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) x[m] = y[m];
+}
+
 // ------------------------------------------------------------------ stage A
-// Block = 4 wavefronts on one image (staged once in LDS); wavefront w handles
-// grid shifts w, w+4, w+8, ...
-// A wavefront samples two rings at a time (ring a real part, ring b imaginary
-// part), runs one 256-point FFT and unpacks both real spectra.  The normalisation
-// sums (radius-weighted sum and sum of squares) accumulate in double.
-// MASKED: only the shifts whose bit is set in smask[p] (S <= 64) are computed;
-// the other rows of spec / norm are left as they were.
-template <bool MASKED, int G = 4>
-__global__ __launch_bounds__(256) void k_polar_spectra(
+// Ring FFTs, four per wavefront: 16 lanes each, lane u holds points u + 16 m.  The
+// radix-4 stages run in pairs inside a lane with one LDS exchange between (real, then
+// imaginary parts, kXchLd floats per transform), in the arithmetic of the Stockham
+// stages (inputs, twiddles, operation order).
+constexpr int kXchLd = 276;       // floats per transform (two lane rows hit 32 distinct banks)
+
+// 16 x 16 transpose within each lane row: in x[4 k + q] = point 16 u + k + 4 q, out
+// x[a] = point u + 16 a.  xb: the lane row's kXchLd floats, free to overwrite.
+__device__ __forceinline__ void row_exchange(float2 (&x)[16], float *xb, int u) {
+    float *xw = xb + 17 * u;
+    const float *xr = xb + u;
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xw[k + 4 * q] = x[4 * k + q].x;
+    wave_lds_sync();
+    float re[16];
+#pragma unroll
+    for (int a = 0; a < 16; ++a) re[a] = xr[17 * a];
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xw[k + 4 * q] = x[4 * k + q].y;
+    wave_lds_sync();
+#pragma unroll
+    for (int a = 0; a < 16; ++a) x[a] = f2(re[a], xr[17 * a]);
+}
+
+// Forward transform, x[m] = point u + 16 m in and out.
+__device__ __forceinline__ void fft256_rows4(float2 (&x)[16], float *xb, const float2 *tw, int u) {
+#pragma unroll
+    for (int q2 = 0; q2 < 4; ++q2) {   // stage 1, butterfly u + 16 q2
+        float2 v[4] = {x[q2], x[q2 + 4], x[q2 + 8], x[q2 + 12]};
+        radix4<false>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q2 + 4 * q] = v[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {      // stage 2, butterfly 4 u + k
+        float2 v[4] = {x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]};
+        if (k > 0) {
+#pragma unroll
+            for (int q = 1; q < 4; ++q) v[q] = cmulf(v[q], stage2_tw(16 * q * k));
+        }
+        radix4<false>(v);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[4 * k + q] = v[q];
+    }
+    row_exchange(x, xb, u);
+    fft256_tail<false>(x, tw, u);
+}
+
+// Spectra of the two real rings of a transform Z = FFT(ring a + i ring b): lane u's slots
+// k = u + 16 m, m < 8, from Z[k] and Z[256 - k] (in lane (16 - u) & 15, through LDS).
+// Slot 0 packs the real bins 0 and 128.
+__device__ __forceinline__ void unpack_rings(const float2 (&z)[16], float2 (&a)[8], float2 (&b)[8], float *xb,
+                                             int u) {
+    // Z[128 + i] at 2 i; Z[256 - k] = entry 128 - k = (16 - u) + 16 (7 - m)
+    float2 *hw = reinterpret_cast<float2 *>(xb) + u;
+    const float2 *hr = reinterpret_cast<const float2 *>(xb) + (16 - u);
+    wave_lds_sync();
+#pragma unroll
+    for (int m = 0; m < 8; ++m) hw[16 * m] = z[8 + m];
+    wave_lds_sync();
+    float2 p[8];
+#pragma unroll
+    for (int m = 0; m < 8; ++m) p[m] = hr[16 * (7 - m)];   // entry 128 (u = 0, m = 0) is not used
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+        a[m] = f2(0.5f * (z[m].x + p[m].x), 0.5f * (z[m].y - p[m].y));
+        b[m] = f2(0.5f * (z[m].y + p[m].y), 0.5f * (p[m].x - z[m].x));
+    }
+    if (u == 0) {
+        a[0] = f2(z[0].x, z[8].x);
+        b[0] = f2(z[0].y, z[8].y);
+    }
+}
+
+// Bilinear sample at (x, y) of an LDS copy of the image with a one-pixel border that
+// repeats the edge (pitch W = D + 2): the cell is clamped to -1 .. D - 1, where both taps
+// of a row read the same edge values as clamping each tap.  img1 points at pixel (0, 0).
+__device__ __forceinline__ float tap(const float *img1, float Wf, float lim, int W, float x, float y) {
+    const float x0 = floorf(x), y0 = floorf(y);
+    const float fx = x - x0, fy = y - y0;
+    const float cx = __builtin_amdgcn_fmed3f(x0, -1.0f, lim), cy = __builtin_amdgcn_fmed3f(y0, -1.0f, lim);
+    const float *q = img1 + (int)fmaf(cy, Wf, cx);   // exact: below 2^24
+    const float v00 = q[0], v01 = q[1], v10 = q[W], v11 = q[W + 1];
+    const float gx = 1.0f - fx, gy = 1.0f - fy;
+    const float top = fmaf(fx, v01, v00 * gx), bot = fmaf(gx, v10, fx * v11);
+    return fmaf(gy, top, fy * bot);
+}
+
+__device__ __forceinline__ double row_sum(double v) {   // over each row of 16 lanes
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
+    return v;
+}
+
+// (mu L, 1 / (sd + 1e-7)) from the radius-weighted sum and sum of squares
+__device__ __forceinline__ float2 ring_norm(double a, double q, int R) {
+    const double nn = (double)kRingLen * 0.5 * (double)R * (double)(R + 1);
+    const double mu = a / nn;
+    const double sd = sqrt(fabs(q / nn - mu * mu));
+    return f2((float)(mu * kRingLen), (float)(1.0 / (sd + 1e-7)));
+}
+
+// LDS floats of a polar kernel with nw wavefronts: lane twiddles, exchange buffers, image.
+__host__ __device__ constexpr int polar_lds_floats(int D, int nw) {
+    return 2 * kIfftTw + nw * 4 * kXchLd + (D + 2) * (D + 2);
+}
+
+// Bordered copy of an image (see tap), all threads; the caller synchronises.
+__device__ __forceinline__ void load_bordered(float *img, const float *src, int D) {
+    const int W = D + 2;
+    for (int r = threadIdx.x >> 6; r < W; r += blockDim.x >> 6) {
+        const float *s = src + min(max(r - 1, 0), D - 1) * D;
+        for (int c = threadIdx.x & 63; c < W; c += 64) img[r * W + c] = s[min(max(c - 1, 0), D - 1)];
+    }
+}
+
+// Samples and transform of ring pair (i, i + 1) of one row about (cx, cy): lane u takes
+// angles u + 16 m; sums (FP64) into sA, sQ; spectra of both rings out (b = 0 past R).
+__device__ __forceinline__ void ring_pair(const float *img1, float Wf, float lim, int W, const float2 *tmpl, int i,
+                                          int R, float cx, float cy, int u, float *xb, const float2 *tw, double &sA,
+                                          double &sQ, float2 (&a)[8], float2 (&b)[8]) {
+    float2 x[16];
+    const float2 *ta = tmpl + (size_t)i * kRingLen + u;
+    double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
+    const bool hb = i + 1 < R;   // uniform over the lane row
+    const float2 *tb = hb ? ta + kRingLen : ta;
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+        const float2 pa = ta[16 * m], pb = tb[16 * m];
+        const float va = tap(img1, Wf, lim, W, cx + pa.x, cy + pa.y);
+        const float t = tap(img1, Wf, lim, W, cx + pb.x, cy + pb.y);
+        const float vb = hb ? t : 0.0f;
+        x[m] = f2(va, vb);
+        const double da = va, db = vb;
+        a1 += da;
+        a2 = fma(da, da, a2);
+        b1 += db;
+        b2 = fma(db, db, b2);
+    }
+    const double wa = (double)(i + 1), wb = (double)(i + 2);
+    sA += wa * a1 + wb * b1;
+    sQ += wa * a2 + wb * b2;
+    fft256_rows4(x, xb, tw, u);
+    unpack_rings(x, a, b, xb, u);
+}
+
+// A lane's slots u + 16 m of one ring row: four 16-byte accesses (slot_re).
+__device__ __forceinline__ void store_slots(float2 *row, const float2 (&a)[8], int u) {
+    float4 *o = reinterpret_cast<float4 *>(row) + 2 * u;
+#pragma unroll
+    for (int mh = 0; mh < 2; ++mh) {
+        o[32 * mh] = make_float4(a[4 * mh].x, a[4 * mh + 1].x, a[4 * mh + 2].x, a[4 * mh + 3].x);
+        o[32 * mh + 1] = make_float4(a[4 * mh].y, a[4 * mh + 1].y, a[4 * mh + 2].y, a[4 * mh + 3].y);
+    }
+}
+
+// Raw ring spectra of an image at every grid shift.  Workgroup = one image (staged once
+// in LDS); a wavefront takes four rows (shifts) at a time, one per 16 lanes, and their
+// rings in pairs.  split > 1: the ring pairs of a group of rows go round over `split`
+// wavefronts, and blockIdx.y names the group.  MASKED: only the shifts whose bit is set
+// in smask[p] (S <= 64) are computed; the other rows of spec / norm are left as they were.
+// What bounds it: vector instructions (about 25 a sample with its FP64 sums, 20 a point
+// of the transform) and the writes; 6000 images of 76 x 76, 49 shifts, 34 rings, 10.2 GB:
+// 3.5 ms, 2.7 without the stores, 2.7 with stores but no transforms.  A transform over 64
+// lanes with an exchange at each stage made it 3.9.  Four wavefronts per SIMD (128
+// registers) are needed to hide the taps.
+template <bool MASKED>
+__global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     const float *__restrict__ imgs, int D, ShiftView acc, const int2 *__restrict__ shift_i,
     int S, const float2 *__restrict__ tmpl, int R, const float2 *__restrict__ twg,
     float2 *__restrict__ spec, float2 *__restrict__ norm,
-    const unsigned long long *__restrict__ smask) {
+    const unsigned long long *__restrict__ smask, int split) {
     extern __shared__ float4 smem4[];
+    __shared__ double red[2][4 * 16];
     __shared__ int slist[64];
     __shared__ int scnt;
-    float2 *tw = reinterpret_cast<float2 *>(smem4);
-    float2 *fb = tw + 256;
-    float *img = reinterpret_cast<float *>(fb + 4 * 512);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = blockDim.x >> 6, f = lane >> 4, u = lane & 15;
     const int p = blockIdx.x;
     if (MASKED && smask[p] == 0ull) return;   // uniform over the workgroup
-    const float *src = imgs + (size_t)p * D * D;
-    for (int i = tid; i < (D + 2) * (D + 2); i += 256) {   // bordered copy (bilinear_bordered)
-        const int r = i / (D + 2), c = i - r * (D + 2);
-        img[i] = src[min(max(r - 1, 0), D - 1) * D + min(max(c - 1, 0), D - 1)];
-    }
-    fill_fft_twiddles(tw, twg, tid, 256);
+    float2 *tw = reinterpret_cast<float2 *>(smem4);
+    float *xb = reinterpret_cast<float *>(tw + kIfftTw) + (wave * 4 + f) * kXchLd;
+    float *img = reinterpret_cast<float *>(tw + kIfftTw) + nw * 4 * kXchLd;
+    const int W = D + 2;
+    load_bordered(img, imgs + (size_t)p * D * D, D);
+    fill_ifft_twiddles(tw, twg, tid, blockDim.x);
     if (MASKED && tid == 0) {
         const unsigned long long mk = smask[p];
         int c = 0;
@@ -224,82 +422,104 @@ __global__ __launch_bounds__(256) void k_polar_spectra(
         ax = acc.base[(size_t)p * acc.stride];
         ay = acc.base[(size_t)p * acc.stride + 1];
     }
-    float2 *b0 = fb + wave * 512;
-    float2 *b1 = b0 + 256;
-    const int pl = (64 - lane) & 63;
-    // rows j0, j0 + 4, ..., j0 + 4 (G - 1) of this wavefront share each ring
-    // pair's template samples (loaded once per group instead of once per row)
-    for (int j0 = wave; j0 < n_rows; j0 += 4 * G) {
-        int sg[G];
-        float cxg[G], cyg[G];
-        double sA[G], sQ[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int j = min(j0 + 4 * g, n_rows - 1);
-            sg[g] = MASKED ? slist[j] : j;
-            const int2 si = shift_i[sg[g]];
-            cxg[g] = (float)(D / 2 + si.x) + ax;
-            cyg[g] = (float)(D / 2 + si.y) + ay;
-            sA[g] = 0.0;
-            sQ[g] = 0.0;
-        }
-        for (int i = 0; i < R; i += 2) {
-            const bool hb = (i + 1) < R;
-            const double wa = (double)(i + 1), wb = (double)(i + 2);
-            float2 ta[4], tb[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                ta[q] = tmpl[i * kRingLen + lane + 64 * q];
-                tb[q] = hb ? tmpl[(i + 1) * kRingLen + lane + 64 * q] : f2(0.0f, 0.0f);
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                if (j0 + 4 * g >= n_rows) break;   // uniform over the wavefront
-                float2 v[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float va = bilinear_bordered(img, D, cxg[g] + ta[q].x, cyg[g] + ta[q].y);
-                    const float vb = hb ? bilinear_bordered(img, D, cxg[g] + tb[q].x, cyg[g] + tb[q].y) : 0.0f;
-                    v[q] = f2(va, vb);
-                    sA[g] += wa * (double)va + wb * (double)vb;
-                    sQ[g] += wa * (double)va * (double)va + wb * (double)vb * (double)vb;
-                }
-                fft256_wave<false>(v, b0, b1, tw, lane);
-                // v[q] = Z[lane + 64 q].  Partners Z[256-k]: k=lane -> lane pl, q=3;
-                // k=lane+64 -> lane pl, q=2 (lane 0: Z[0] itself and Z[192] = own q=3).
-                const float2 u2 = shfl2(v[2], pl), u3 = shfl2(v[3], pl);
-                const float2 zl = v[0], zlp = lane ? u3 : v[0];
-                const float2 zh = v[1], zhp = lane ? u2 : v[3];
-                float2 al = f2(0.5f * (zl.x + zlp.x), 0.5f * (zl.y - zlp.y));
-                float2 bl = f2(0.5f * (zl.y + zlp.y), 0.5f * (zlp.x - zl.x));
-                const float2 ah = f2(0.5f * (zh.x + zhp.x), 0.5f * (zh.y - zhp.y));
-                const float2 bh = f2(0.5f * (zh.y + zhp.y), 0.5f * (zhp.x - zh.x));
-                if (lane == 0) {  // pack Nyquist: A[128] = Re Z[128], B[128] = Im Z[128]
-                    al = f2(zl.x, v[2].x);
-                    bl = f2(zl.y, v[2].y);
-                }
-                float2 *oa = spec + (((size_t)p * S + sg[g]) * (size_t)R + i) * kSlots;
-                store_ring(oa, lane, al, ah);
-                if (hb) store_ring(oa + kSlots, lane, bl, bh);
+    const float *img1 = img + W + 1;
+    const float Wf = (float)W, lim = (float)(D - 1);
+    const int q0 = split > 1 ? wave : 0;          // first ring pair of this wavefront
+    const int jw = split > 1 ? blockIdx.y : wave, jn = split > 1 ? gridDim.y : nw;
+    for (int j0 = 4 * jw; j0 < n_rows; j0 += 4 * jn) {
+        const bool live = j0 + f < n_rows;   // lanes past the last row repeat it, without its stores
+        const int j = min(j0 + f, n_rows - 1);
+        const int s = MASKED ? slist[j] : j;
+        const int2 si = shift_i[s];
+        const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
+        double sA = 0.0, sQ = 0.0;
+        float2 *row = spec + ((size_t)p * S + s) * (size_t)R * kSlots;
+        for (int i = 2 * q0; i < R; i += 2 * split) {
+            float2 a[8], b[8];
+            ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, sA, sQ, a, b);
+            if (live) {
+                store_slots(row + (size_t)i * kSlots, a, u);
+                if (i + 1 < R) store_slots(row + (size_t)(i + 1) * kSlots, b, u);
             }
         }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            if (j0 + 4 * g >= n_rows) break;
-            double a2 = sA[g], q2 = sQ[g];
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) {
-                a2 += __shfl_xor(a2, off, kWave);
-                q2 += __shfl_xor(q2, off, kWave);
+        sA = row_sum(sA);
+        sQ = row_sum(sQ);
+        if (split > 1) {   // one group per workgroup: all wavefronts arrive here once
+            if (u == 0) {
+                red[0][4 * wave + f] = sA;
+                red[1][4 * wave + f] = sQ;
             }
-            if (lane == 0) {
-                const double nn = (double)kRingLen * 0.5 * (double)R * (double)(R + 1);
-                const double mu = a2 / nn;
-                const double sd = sqrt(fabs(q2 / nn - mu * mu));
-                norm[(size_t)p * S + sg[g]] = f2((float)(mu * kRingLen), (float)(1.0 / (sd + 1e-7)));
+            __syncthreads();
+            if (wave > 0) break;
+            for (int w = 1; w < split; ++w) {
+                sA += red[0][4 * w + f];
+                sQ += red[1][4 * w + f];
             }
         }
-    }  // row groups
+        if (live && u == 0) norm[(size_t)p * S + s] = ring_norm(sA, sQ, R);
+    }
+}
+
+// Reference spectra (centre D / 2, no shift), normalised and multiplied by the ring
+// weight i + 1; rsum0[n] = sum of slot 0's real parts (the particle DC correction).
+// Workgroup = one reference, one ring pair per 16 lanes (up to 64 pairs), so the
+// transforms of all its rings run at once and stay in registers until the sums are
+// complete: a search of few references waits for one such pass.  5 references of
+// 64 x 64, 29 rings: 12 us, 100 of 76 x 76, 34 rings: 21 us; with four wavefronts for all
+// rings and a normalising pass the 5 took 25 + 6.
+__global__ __launch_bounds__(1024) void k_ref_spectra(const float *__restrict__ imgs, int D,
+                                                      const float2 *__restrict__ tmpl, int R,
+                                                      const float2 *__restrict__ twg, float2 *__restrict__ rspec,
+                                                      float *__restrict__ rsum0) {
+    extern __shared__ float4 smem4[];
+    __shared__ double red[2][64];
+    __shared__ float dc[2 * 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = blockDim.x >> 6, f = lane >> 4, u = lane & 15;
+    const int n = blockIdx.x, W = D + 2;
+    float2 *tw = reinterpret_cast<float2 *>(smem4);
+    float *xb = reinterpret_cast<float *>(tw + kIfftTw) + (wave * 4 + f) * kXchLd;
+    float *img = reinterpret_cast<float *>(tw + kIfftTw) + nw * 4 * kXchLd;
+    load_bordered(img, imgs + (size_t)n * D * D, D);
+    fill_ifft_twiddles(tw, twg, tid, blockDim.x);
+    __syncthreads();
+    const int i = 2 * (4 * wave + f);
+    const bool live = i < R;
+    double sA = 0.0, sQ = 0.0;
+    float2 a[8], b[8];
+    const float c = (float)(D / 2);
+    ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, live ? i : 0, R, c, c, u, xb, tw, sA, sQ, a, b);
+    sA = row_sum(sA);
+    sQ = row_sum(sQ);
+    if (u == 0) {
+        red[0][4 * wave + f] = live ? sA : 0.0;
+        red[1][4 * wave + f] = live ? sQ : 0.0;
+    }
+    __syncthreads();
+    double tA = 0.0, tQ = 0.0;
+    for (int k = 0; k < 4 * nw; ++k) {
+        tA += red[0][k];
+        tQ += red[1][k];
+    }
+    const float2 nm = ring_norm(tA, tQ, R);
+    auto finish = [&](float2 (&v)[8], int ring) {
+        const float gw = nm.y * (float)(ring + 1);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const float re = (m == 0 && u == 0) ? v[m].x - nm.x : v[m].x;
+            v[m] = f2(re * gw, v[m].y * gw);
+        }
+        store_slots(rspec + ((size_t)n * R + ring) * kSlots, v, u);
+        if (u == 0) dc[ring] = v[0].x;
+    };
+    if (live) finish(a, i);
+    if (live && i + 1 < R) finish(b, i + 1);
+    __syncthreads();
+    if (tid == 0) {
+        double s = 0.0;
+        for (int k = 0; k < R; ++k) s += (double)dc[k];
+        rsum0[n] = (float)s;
+    }
 }
 
 // Stage A of the mixed-precision search: the normalised ring spectra of every
@@ -587,30 +807,6 @@ __global__ __launch_bounds__(256, 2) void k_polar_frag(
     }
 }
 
-__global__ __launch_bounds__(128) void k_ref_finalize(float2 *__restrict__ rspec,
-                                                      const float2 *__restrict__ rnorm, int R,
-                                                      float *__restrict__ rsum0) {
-    const int n = blockIdx.x, k = threadIdx.x;
-    const float2 nm = rnorm[n];
-    double acc0 = 0.0;
-    for (int i = 0; i < R; ++i) {
-        float *px = reinterpret_cast<float *>(rspec + ((size_t)n * R + i) * kSlots) + slot_re(k);
-        float2 x = f2(px[0], px[kPartOff]);
-        const float gw = nm.y * (float)(i + 1);
-        if (k == 0) {
-            x.x = (x.x - nm.x) * gw;
-            x.y = x.y * gw;
-            acc0 += (double)x.x;
-        } else {
-            x.x *= gw;
-            x.y *= gw;
-        }
-        px[0] = x.x;
-        px[kPartOff] = x.y;
-    }
-    if (k == 0) rsum0[n] = (float)acc0;
-}
-
 // ------------------------------------------------------------------ stage B
 // Psi transform: 256-point inverse FFTs, four per wavefront (16 lanes each, 16 points
 // per lane).  The four radix-4 stages run in pairs inside a lane, so one exchange
@@ -620,32 +816,6 @@ __global__ __launch_bounds__(128) void k_ref_finalize(float2 *__restrict__ rspec
 constexpr int kFftLd = 273;       // float2 per transform in LDS (odd mod 32: no bank conflicts
                                   // between transforms; 17 x 16 + 1 hold the padded exchange)
 constexpr int kMirOff = 136;      // Z[k], k < 128, at k; Z[256 - k] at kMirOff + k (k = 1..128)
-constexpr int kIfftTw = 15 * 16;  // lane twiddles of the last two stages
-
-// entry q - 1: stage 3, e^{-2 pi i 4 q u / 256}; entry 3 + 3 q3 + q - 1: stage 4,
-// e^{-2 pi i q (u + 16 q3) / 256}
-__device__ __forceinline__ void fill_ifft_twiddles(float2 *tw, const float2 *twg, int tid, int nthreads) {
-    for (int i = tid; i < kIfftTw; i += nthreads) {
-        const int e = i >> 4, u = i & 15;
-        tw[i] = e < 3 ? twg[4 * (e + 1) * u] : twg[((e - 3) % 3 + 1) * (u + 16 * ((e - 3) / 3))];
-    }
-}
-
-// v conj(w), with the operation order of cmul under INV
-__device__ __forceinline__ float2 cmulc(float2 v, float2 w) {
-    return f2(fmaf(v.x, w.x, v.y * w.y), fmaf(v.y, w.x, -(v.x * w.y)));
-}
-
-// cos, sin of -2 pi m / 256 for the m = 16 q k of the second stage (the table's values)
-__device__ __forceinline__ constexpr float2 stage2_tw(int m) {
-    return m == 16    ? float2{0.92387953251128674f, -0.38268343236508977f}
-           : m == 32  ? float2{0.70710678118654757f, -0.70710678118654757f}
-           : m == 48  ? float2{0.38268343236508984f, -0.92387953251128674f}
-           : m == 64  ? float2{6.123233995736766e-17f, -1.0f}
-           : m == 96  ? float2{-0.70710678118654746f, -0.70710678118654757f}
-                      : float2{-0.92387953251128685f, 0.38268343236508967f};   // m == 144
-}
-
 // First two stages.  In: x[m] = Z[u + 16 m], Z[64..127] (m = 4..7) without the row's
 // scale gs, which the first butterflies apply in one rounding.  Out: x[4 k + q] is
 // point 17 u + k + 4 q of the exchange.
@@ -688,37 +858,6 @@ __device__ __forceinline__ void ifft256_get(float2 (&x)[16], const float2 *xb, i
     for (int a = 0; a < 16; ++a) x[a] = xr[17 * a];
 }
 
-// Last two stages.  Out: x[m] = z[u + 16 m].
-__device__ __forceinline__ void ifft256_tail(float2 (&x)[16], const float2 *tw, int u) {
-    float2 w3[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) w3[q] = tw[q * 16 + u];
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {      // stage 3, butterfly 16 h + u
-        float2 v[4] = {x[h], x[h + 4], x[h + 8], x[h + 12]};
-#pragma unroll
-        for (int q = 1; q < 4; ++q) v[q] = cmulc(v[q], w3[q - 1]);
-        radix4<true>(v);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[h + 4 * q] = v[q];
-    }
-#pragma unroll
-    for (int q3 = 0; q3 < 4; ++q3) {   // stage 4, butterfly u + 16 q3
-        float2 v[4] = {x[4 * q3], x[4 * q3 + 1], x[4 * q3 + 2], x[4 * q3 + 3]};
-#pragma unroll
-        for (int q = 1; q < 4; ++q) v[q] = cmulc(v[q], tw[(3 + 3 * q3 + q - 1) * 16 + u]);
-        radix4<true>(v);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[4 * q3 + q] = v[q];
-    }
-    // x[4 q3 + q] = z[u + 16 q3 + 64 q]: to natural order
-    float2 y[16];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) y[m] = x[4 * (m & 3) + (m >> 2)];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) x[m] = y[m];
-}
-
 // Z of one transform from LDS (positions of kMirOff) into lane u's 16 points
 __device__ __forceinline__ void load_z(float2 (&x)[16], const float2 *xb, int u) {
     const float2 *lo = xb + u, *hi = xb + (kMirOff + 16 - u);
@@ -736,7 +875,7 @@ __device__ __forceinline__ void ifft256_rows4(float2 (&x)[16], float gs, float2 
     ifft256_put(x, xb, u);
     wave_lds_sync();
     ifft256_get(x, xb, u);
-    ifft256_tail(x, tw, u);
+    fft256_tail<true>(x, tw, u);
 }
 
 // max over the 16 lanes of each lane row, then the wavefront's (uniform)
@@ -2231,12 +2370,35 @@ __global__ void k_row_c2r(float *__restrict__ refs, int D, const float2 *__restr
 
 // ---------------------------------------------------------------- launchers
 
+// Launch shape of the polar pass.  A workgroup's wavefronts take the row groups (four
+// shifts each) in equal passes: 13 groups run as 2 x 7, not 8 + 5.  Up to 8 wavefronts
+// where two workgroups fit in a CU's LDS, up to 16 where only one does.  With fewer
+// groups than the chip has wavefront slots (16 per CU), the ring pairs of a group are
+// split over wavefronts, one group per workgroup: 24 images of 64 x 64, 9 shifts, 29
+// rings take 21 us instead of 77.
+struct PolarShape {
+    int waves, split, groups_y;
+};
+static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_ring) {
+    const int g = (n_shift + 3) / 4, pairs = (n_ring + 1) / 2;
+    const long long fill = 4096 / (n_img * g);
+    if (fill >= 2 && pairs >= 2) {
+        const int split = (int)std::min<long long>({fill, pairs, 16});
+        return {split, split, g};
+    }
+    const int cap = 2 * polar_lds_floats(img_dim, 8) * sizeof(float) <= 160 * 1024 - 4096 ? 8 : 16;
+    const int passes = (g + cap - 1) / cap;
+    return {(g + passes - 1) / passes, 1, 1};
+}
+
 hipError_t prepare_launches() {
     static bool lds_raised = false;
     if (!lds_raised) {
-        const int lds = (int)((256 + 4 * 512) * sizeof(float2) +
-                              (kMaxImgDim + 2) * (kMaxImgDim + 2) * sizeof(float));
-        hipError_t e = hipFuncSetAttribute((const void *)k_polar_spectra<false>,
+        const int lds = (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float));
+        hipError_t e = hipFuncSetAttribute((const void *)k_ref_spectra, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float)));
+        if (e != hipSuccess) return e;
+        e = hipFuncSetAttribute((const void *)k_polar_spectra<false>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute((const void *)k_polar_spectra<true>,
@@ -2261,11 +2423,11 @@ hipError_t launch_polar_spectra(const float *imgs, int n_img, int img_dim, Shift
                                 const float2 *twiddle, float2 *spec, float2 *norm,
                                 hipStream_t st) {
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
-    const size_t lds = (256 + 4 * 512) * sizeof(float2) + (size_t)(img_dim + 2) * (img_dim + 2) * sizeof(float);
     if (hipError_t e = prepare_launches()) return e;
-    dim3 grid(n_img);
-    hipLaunchKernelGGL(k_polar_spectra<false>, grid, dim3(256), lds, st, imgs, img_dim, acc,
-                       shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, nullptr);
+    const PolarShape ps = polar_shape(n_img, n_shift, img_dim, n_ring);
+    const size_t lds = polar_lds_floats(img_dim, ps.waves) * sizeof(float);
+    hipLaunchKernelGGL(k_polar_spectra<false>, dim3(n_img, ps.groups_y), dim3(64 * ps.waves), lds, st, imgs,
+                       img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, nullptr, ps.split);
     return hipGetLastError();
 }
 
@@ -2300,17 +2462,22 @@ hipError_t launch_polar_spectra_masked(const float *imgs, int n_img, int img_dim
                                        hipStream_t st) {
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
     if (n_shift > 64) return hipErrorInvalidValue;
-    const size_t lds = (256 + 4 * 512) * sizeof(float2) + (size_t)(img_dim + 2) * (img_dim + 2) * sizeof(float);
     if (hipError_t e = prepare_launches()) return e;
-    hipLaunchKernelGGL(k_polar_spectra<true>, dim3(n_img), dim3(256), lds, st, imgs, img_dim, acc,
-                       shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, smask);
+    // unsplit: how many of a particle's shifts are set is not known here
+    const PolarShape ps = polar_shape(4096, n_shift, img_dim, n_ring);
+    const size_t lds = polar_lds_floats(img_dim, ps.waves) * sizeof(float);
+    hipLaunchKernelGGL(k_polar_spectra<true>, dim3(n_img), dim3(64 * ps.waves), lds, st, imgs, img_dim, acc,
+                       shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, smask, 1);
     return hipGetLastError();
 }
 
-hipError_t launch_ref_finalize(float2 *rspec, const float2 *rnorm, int n_ref, int n_ring,
-                               float *rsum0, hipStream_t st) {
+hipError_t launch_ref_spectra(const float *imgs, int n_ref, int img_dim, const float2 *tmpl, int n_ring,
+                              const float2 *twiddle, float2 *rspec, float *rsum0, hipStream_t st) {
     if (n_ref <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_ref_finalize, dim3(n_ref), dim3(kSlots), 0, st, rspec, rnorm, n_ring, rsum0);
+    if (hipError_t e = prepare_launches()) return e;
+    const int nw = (n_ring + 7) / 8;   // wavefronts of four ring pairs
+    hipLaunchKernelGGL(k_ref_spectra, dim3(n_ref), dim3(64 * nw), polar_lds_floats(img_dim, nw) * sizeof(float), st,
+                       imgs, img_dim, tmpl, n_ring, twiddle, rspec, rsum0);
     return hipGetLastError();
 }
 
