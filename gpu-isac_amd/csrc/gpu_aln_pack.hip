@@ -167,7 +167,7 @@ struct Context {
     size_t n_param = 0;
     enum Mode { kNone, kMref, kPre, kRefFree } mode = kNone;
     // pre-align / reference-free device data
-    DevBuf sbj_img, ref_img, prm, tr, cid_idx, ref_of, twd, tanl_work;
+    DevBuf sbj_img, ref_img, prm, tp, mir, cid_idx, ref_of, twd, tanl_work;
     unsigned sbj_cap = 0, ref_cap = 0, sbj_count = 0, ref_count = 0;
     int twd_dim = 0;
     // multi_ref_align host staging
@@ -1471,7 +1471,7 @@ void gpu_clear(void) {
     if (g.h_stage) (void)hipHostFree(g.h_stage);
     g.h_stage = nullptr;
     g.h_stage_cap = 0;
-    DevBuf *bufs[] = {&g.sbj_img, &g.ref_img, &g.prm, &g.tr, &g.cid_idx, &g.ref_of, &g.twd, &g.tanl_work};
+    DevBuf *bufs[] = {&g.sbj_img, &g.ref_img, &g.prm, &g.tp, &g.mir, &g.cid_idx, &g.ref_of, &g.twd, &g.tanl_work};
     for (DevBuf *b : bufs) b->release();
     g.sbj_cap = g.ref_cap = g.sbj_count = g.ref_count = 0;
     g.twd_dim = 0;
@@ -1980,14 +1980,13 @@ void ref_free_alignment_2D(void) {
     if (run_single(g.sbj_img.as<float>(), prm, &prm[0].ref_id, (int)(sizeof(DevParam) / sizeof(int)),
                    P, g.ref_img.as<float>(), N, D, R, g.shifts, lim, st))
         return;
-    if (g.tr.reserve((size_t)std::max(P, 1) * D * D * sizeof(float)) != hipSuccess) {
+    if (g.tp.reserve((size_t)std::max(P, 1) * sizeof(float4)) != hipSuccess ||
+        g.mir.reserve((size_t)std::max(P, 1) * sizeof(int)) != hipSuccess) {
         set_error(kErrHip, "ref_free_alignment_2D: allocation failed");
         return;
     }
-    hipError_t e = isac::launch_transform(g.sbj_img.as<float>(), P, D, prm, g.tr.as<float>(), st);
-    if (e == hipSuccess)
-        e = isac::launch_class_average(g.tr.as<float>(), D, g.cid_idx.as<int>(), N,
-                                       g.ref_img.as<float>(), st);
+    const hipError_t e = isac::launch_class_average(g.sbj_img.as<float>(), P, D, prm, g.cid_idx.as<int>(), N,
+                                                    g.tp.as<float4>(), g.mir.as<int>(), g.ref_img.as<float>(), st);
     if (e != hipSuccess) {
         set_error(kErrHip, "ref_free_alignment_2D: kernel launch failed: %s", hipGetErrorString(e));
         return;

@@ -212,12 +212,8 @@ hipError_t launch_decode_single(const PeakRec *rec, int cnt, DevParam *prm,
                                 const float2 *shifts_f, int n_shift, float shift_limit,
                                 hipStream_t st);
 
-// Apply found parameters to images: out[i] = T_i(imgs[i]).
-hipError_t launch_transform(const float *imgs, int n, int img_dim, const DevParam *prm,
-                            float *out, hipStream_t st);
-
-// Pre-alignment loop: avg = mean over P particles of T_p(imgs[p]) (the transform of
-// launch_transform), tp / mir hold P entries, part pre_average_scratch_floats(P, D);
+// Pre-alignment loop: avg = mean over P particles of T_p(imgs[p]) (the transform by the
+// parameters found), tp / mir hold P entries, part pre_average_scratch_floats(P, D);
 // shift[0] = the centring move (-sx_sum / P, -sy_sum / P) of the driver's
 // average-shift centring.
 size_t pre_average_scratch_floats(int P, int D);
@@ -225,9 +221,10 @@ hipError_t launch_pre_average(const float *imgs, int P, int D, const DevParam *p
                               int *mir, float *part, float *avg, hipStream_t st);
 hipError_t launch_pre_center(const DevParam *prm, int P, float2 *shift, hipStream_t st);
 
-// Per-class mean of transformed images into refs.
-hipError_t launch_class_average(const float *tr, int img_dim, const int *cid_idx, int n_cls,
-                                float *refs, hipStream_t st);
+// Per-class mean of T_p(imgs[p]) into refs, class k = particles [cid_idx[k], cid_idx[k + 1]);
+// tp / mir hold P entries.
+hipError_t launch_class_average(const float *imgs, int P, int img_dim, const DevParam *prm, const int *cid_idx,
+                                int n_cls, float4 *tp, int *mir, float *refs, hipStream_t st);
 
 // Tangent low-pass filter of refs in place; work holds n*img_dim*(img_dim/2+1) float2,
 // tw_d holds img_dim twiddles e^{-2 pi i m / img_dim}.
