@@ -662,6 +662,17 @@ int run_single(const float *d_sbj, DevParam *prm, const int *ref_of, int ref_str
     if (int e = ensure_template(R)) return e;
     if (int e = ensure_shifts(shifts)) return e;
     if (int e = ref_spectra(d_ref, N, D, R, st)) return e;
+    if (isac::polar_single_fills(cnt, S)) {
+        HIP_OK(ws.rec.reserve((size_t)cnt * sizeof(PeakRec)));
+        HIP_OK(isac::launch_polar_single(d_sbj, cnt, D, {&prm[0].shift_x, (int)(sizeof(DevParam) / sizeof(float))},
+                                         ws.shifts_i.as<int2>(), S, ws.tmpl.as<float2>(), R,
+                                         ws.twiddle.as<float2>(), ws.rspec.as<float2>(), ws.rsum0.as<float>(),
+                                         ref_of, ref_stride, N, ws.rec.as<PeakRec>(), st));
+        HIP_OK(isac::launch_decode_single(ws.rec.as<PeakRec>(), cnt, prm, ws.shifts_f.as<float2>(), S, shift_limit,
+                                          st));
+        if (sync) HIP_OK(hipStreamSynchronize(st));
+        return 0;
+    }
     const size_t per = (size_t)S * R * kSlots * sizeof(float2) + (size_t)S * sizeof(float2) +
                        sizeof(PeakRec);
     const int pb = batch_for(per, 0, 0.9f, cnt);

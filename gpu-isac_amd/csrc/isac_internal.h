@@ -171,6 +171,13 @@ hipError_t launch_ccf_single(const float2 *spec, const float2 *norm, const float
                              const float *rsum0, const int *ref_of, int ref_stride, int n_img,
                              int n_shift, int n_ring, int n_ref, const float2 *twiddle,
                              PeakRec *rec, hipStream_t st);
+// The same search from the pixels, without the spectra in memory; polar_single_fills says
+// where it is the faster one.
+hipError_t launch_polar_single(const float *imgs, int n_img, int img_dim, ShiftView acc, const int2 *shift_i,
+                               int n_shift, const float2 *tmpl, int n_ring, const float2 *twiddle,
+                               const float2 *rspec, const float *rsum0, const int *ref_of, int ref_stride, int n_ref,
+                               PeakRec *rec, hipStream_t st);
+bool polar_single_fills(int n_img, int n_shift);
 
 // Exact FP32 re-scoring of K candidate references per particle (ref cand[p*K+k];
 // a negative entry gives an empty record), same arithmetic as launch_ccf_mref;

@@ -1106,6 +1106,127 @@ __global__ __launch_bounds__(256) void k_ccf_single(
     write_rec(rec + p, st, nbuf[wave], lane);
 }
 
+// a b, rounded before any sum that takes it (not fused into it)
+__device__ __forceinline__ float mul_rn(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+// Each image against its own reference ref_of[p * ref_stride], from the pixels: k_polar_spectra's
+// workgroup and wavefronts (one image, four shift rows at a time, a ring pair at a time), but
+// the spectra of a pair are contracted with the reference's at once, in the ring order and
+// operation order of k_ccf_single, and never leave the registers; then the psi transforms of
+// the four rows.  The wavefronts' first maxima are merged: larger value, then smaller shift.
+// What bounds it: vector instructions, as k_polar_spectra without its stores.  5000 images
+// of 76 x 76, 34 rings, 49 and 9 shifts in turn: 2.1 ms a search; the two passes, with 8.6 GB
+// of spectra written and read at 49 shifts, took 3.3.
+__global__ __launch_bounds__(1024, 4) void k_polar_single(
+    const float *__restrict__ imgs, int D, ShiftView acc, const int2 *__restrict__ shift_i, int S,
+    const float2 *__restrict__ tmpl, int R, const float2 *__restrict__ twg, const float2 *__restrict__ rspec,
+    const float *__restrict__ rsum0, const int *__restrict__ ref_of, int ref_stride, int N,
+    PeakRec *__restrict__ rec) {
+    extern __shared__ float4 smem4[];
+    __shared__ float nbuf[16][2][8];
+    __shared__ float pv[16][2];
+    __shared__ int pf[16][2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = blockDim.x >> 6, f = lane >> 4, u = lane & 15;
+    const int p = blockIdx.x, W = D + 2;
+    float2 *tw = reinterpret_cast<float2 *>(smem4);
+    float *xb = reinterpret_cast<float *>(tw + kIfftTw) + (wave * 4 + f) * kXchLd;
+    float *img = reinterpret_cast<float *>(tw + kIfftTw) + nw * 4 * kXchLd;
+    load_bordered(img, imgs + (size_t)p * D * D, D);
+    fill_ifft_twiddles(tw, twg, tid, blockDim.x);
+    __syncthreads();
+    const float ax = acc.base[(size_t)p * acc.stride], ay = acc.base[(size_t)p * acc.stride + 1];
+    // the host validates ref ids; the clamp keeps every read in bounds
+    const int n = min(max(ref_of[(size_t)p * ref_stride], 0), N - 1);
+    const float rs0 = rsum0[n];
+    const float4 *rb = reinterpret_cast<const float4 *>(rspec + (size_t)n * R * kSlots) + 2 * u;
+    PeakState st;
+    st.reset(0.0f, 0);
+    for (int j0 = 4 * wave; j0 < S; j0 += 4 * nw) {
+        const int2 si = shift_i[min(j0 + f, S - 1)];   // lanes past the last row repeat it
+        const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
+        double sA = 0.0, sQ = 0.0;
+        float c[8][4];
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[m][e] = 0.0f;
+        auto contract = [&](const float2 (&v)[8], int i) {
+            const float4 *r = rb + (size_t)i * (kSlots / 2);
+#pragma unroll
+            for (int mh = 0; mh < 2; ++mh) {
+                const float4 re4 = r[32 * mh], im4 = r[32 * mh + 1];
+                const float re[4] = {re4.x, re4.y, re4.z, re4.w}, im[4] = {im4.x, im4.y, im4.z, im4.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int m = 4 * mh + k;
+                    c[m][0] = fmaf(re[k], v[m].x, c[m][0]);
+                    c[m][1] = fmaf(im[k], v[m].y, c[m][1]);
+                    c[m][2] = fmaf(re[k], v[m].y, c[m][2]);
+                    c[m][3] = fmaf(im[k], v[m].x, c[m][3]);
+                }
+            }
+        };
+        for (int i = 0; i < R; i += 2) {
+            float2 a[8], b[8];
+            ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, i, R, cx, cy, u, xb, tw, sA, sQ, a, b);
+            contract(a, i);
+            if (i + 1 < R) contract(b, i + 1);
+        }
+        const float2 nm = ring_norm(row_sum(sA), row_sum(sQ), R);
+        // Z as store_pair_z makes it; Z[256 - k] goes to lane (16 - u) & 15 through LDS
+        float2 x[16];
+        float2 *zb = reinterpret_cast<float2 *>(xb);
+        wave_lds_sync();
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const float a = c[m][0] + c[m][1], e = c[m][2] + c[m][3];
+            const float g = c[m][0] - c[m][1], b = c[m][3] - c[m][2];
+            x[m] = m < 4 ? f2(mul_rn(nm.y, a + e), mul_rn(nm.y, b + g)) : f2(a + e, b + g);
+            float2 y = f2(nm.y * (a - e), nm.y * (g - b));
+            int ky = u + 16 * m;
+            if (m == 0 && u == 0) {
+                const float c0 = mul_rn(nm.y, fmaf(-nm.x, rs0, c[0][0]));
+                const float cn = nm.y * c[0][1];
+                x[0] = f2(c0, c0);
+                y = f2(cn, cn);
+                ky = 128;
+            }
+            zb[ky] = y;
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int m = 8; m < 16; ++m) x[m] = zb[128 - u - 16 * (m - 8)];
+        ifft256_head(x, nm.y);
+        row_exchange(x, xb, u);
+        fft256_tail<true>(x, tw, u);
+        peak_update<true, false>(st, x, 0, min(4, S - j0), j0, lane, zb, nbuf[wave], 0u);
+    }
+    if (lane < 2) {
+        pv[wave][lane] = lane ? st.bv[1] : st.bv[0];
+        pf[wave][lane] = lane ? st.bf[1] : st.bf[0];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        int w = 0;
+#pragma unroll 1
+        for (int k = 1; k < nw; ++k)
+            if (pv[k][m] > st.bv[m] || (pv[k][m] == st.bv[m] && pf[k][m] < st.bf[m])) {
+                st.bv[m] = pv[k][m];
+                st.bf[m] = pf[k][m];
+                w = k;
+            }
+        if (lane < 7) nbuf[0][m][lane] = nbuf[w][m][lane];   // where write_rec reads them
+    }
+    wave_lds_sync();
+    write_rec(rec + p, st, nbuf[0], lane);
+}
+
 // Top-K references of every particle by approximate peak value (descending; ties
 // to the lower reference index).  One thread per particle.
 template <int K>
@@ -2410,6 +2531,12 @@ __global__ void k_row_c2r(float *__restrict__ refs, int D, const float2 *__restr
 struct PolarShape {
     int waves, split, groups_y;
 };
+static int polar_waves(int n_shift, int img_dim) {
+    const int g = (n_shift + 3) / 4;
+    const int cap = 2 * polar_lds_floats(img_dim, 8) * sizeof(float) <= 160 * 1024 - 4096 ? 8 : 16;
+    const int passes = (g + cap - 1) / cap;
+    return (g + passes - 1) / passes;
+}
 static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_ring) {
     const int g = (n_shift + 3) / 4, pairs = (n_ring + 1) / 2;
     const long long fill = 4096 / (n_img * g);
@@ -2417,9 +2544,7 @@ static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_r
         const int split = (int)std::min<long long>({fill, pairs, 16});
         return {split, split, g};
     }
-    const int cap = 2 * polar_lds_floats(img_dim, 8) * sizeof(float) <= 160 * 1024 - 4096 ? 8 : 16;
-    const int passes = (g + cap - 1) / cap;
-    return {(g + passes - 1) / passes, 1, 1};
+    return {polar_waves(n_shift, img_dim), 1, 1};
 }
 
 hipError_t prepare_launches() {
@@ -2428,6 +2553,8 @@ hipError_t prepare_launches() {
         const int lds = (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float));
         hipError_t e = hipFuncSetAttribute((const void *)k_ref_spectra, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float)));
+        if (e != hipSuccess) return e;
+        e = hipFuncSetAttribute((const void *)k_polar_single, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute((const void *)k_polar_spectra<false>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -2590,6 +2717,29 @@ hipError_t launch_ccf_single(const float2 *spec, const float2 *norm, const float
     hipLaunchKernelGGL(k_ccf_single, dim3((n_img + 3) / 4), dim3(256), 0, st, spec, norm, rspec, rsum0,
                        ref_of, ref_stride, n_img, n_shift, n_ring, n_ref, twiddle, rec);
     return hipGetLastError();
+}
+
+hipError_t launch_polar_single(const float *imgs, int n_img, int img_dim, ShiftView acc, const int2 *shift_i,
+                               int n_shift, const float2 *tmpl, int n_ring, const float2 *twiddle,
+                               const float2 *rspec, const float *rsum0, const int *ref_of, int ref_stride, int n_ref,
+                               PeakRec *rec, hipStream_t st) {
+    if (n_img <= 0 || n_shift <= 0) return hipSuccess;
+    if (hipError_t e = prepare_launches()) return e;
+    const int nw = polar_waves(n_shift, img_dim);
+    hipLaunchKernelGGL(k_polar_single, dim3(n_img), dim3(64 * nw), polar_lds_floats(img_dim, nw) * sizeof(float), st,
+                       imgs, img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, rspec, rsum0, ref_of,
+                       ref_stride, n_ref, rec);
+    return hipGetLastError();
+}
+
+// One pass does a group of four shifts in one wavefront; two passes split the rings of few
+// groups over wavefronts.  Pre-alignment of 76 x 76 images, 34 rings, three iterations, one
+// pass / two (us): 49 shifts, 5 images 512 / 585, 155 images 662 / 1145, 5000 images 12700 /
+// 18900; 9 shifts, 30 images 340 / 292, 150 images 455 / 457, 600 images 776 / 898; 1 shift,
+// 600 images 759 / 634.  128 x 128, 61 rings, 9 shifts: 150 images 650 / 594, 600 images
+// 1598 / 1674.
+bool polar_single_fills(int n_img, int n_shift) {
+    return n_shift > 12 || (n_shift >= 4 && (long long)n_img * ((n_shift + 3) / 4) >= 1024);
 }
 
 hipError_t launch_ccf_candidates(const float2 *spec, const float2 *norm, const float2 *rspec,
