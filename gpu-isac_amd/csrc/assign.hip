@@ -23,6 +23,7 @@
 
 #include <cfloat>
 #include <climits>
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <vector>
@@ -390,13 +391,34 @@ __global__ void k_assign_init(int *status, int *last_n, float *last_v, int P, in
     }
 }
 
+// One device allocation cut into arrays (256-byte aligned).
 struct Buf {
     void *p = nullptr;
-    ~Buf() {
-        if (p) (void)hipFree(p);
-    }
+    size_t bytes = 0;
     template <class T>
     T *as() { return static_cast<T *>(p); }
+};
+struct Arena {
+    std::vector<Buf *> parts;
+    void *base = nullptr;
+    ~Arena() {
+        if (base) (void)hipFree(base);
+    }
+    void add(Buf &b, size_t bytes) {
+        b.bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
+        parts.push_back(&b);
+    }
+    hipError_t allocate() {
+        size_t total = 0;
+        for (Buf *b : parts) total += b->bytes;
+        const hipError_t e = hipMalloc(&base, total);
+        char *at = static_cast<char *>(base);
+        for (Buf *b : parts) {
+            b->p = at;
+            at += b->bytes;
+        }
+        return e;
+    }
 };
 
 int err(int code, const char *msg) {
@@ -413,20 +435,17 @@ int assign_groups(const float *d_d, int N, int P, int pitch, int *d_out, hipStre
     if (cap > kMaxCap)
         return err(4, "assign_groups: classes of more than 2048 particles are not supported");
     Buf status, last_n, last_v, cnt, props, holders, hold_v, hold_cnt, left;
-    hipError_t e = hipSuccess;
-    auto alloc = [&](Buf &b, size_t bytes) {
-        if (e == hipSuccess) e = hipMalloc(&b.p, bytes > 0 ? bytes : 4);
-    };
-    alloc(status, (size_t)P * 4);
-    alloc(last_n, (size_t)P * 4);
-    alloc(last_v, (size_t)P * 4);
-    alloc(cnt, (size_t)N * 4);
-    alloc(props, (size_t)N * P * 4);
-    alloc(holders, (size_t)N * cap * 4);
-    alloc(hold_cnt, (size_t)N * 4);
-    alloc(hold_v, (size_t)N * cap * 4);
-    alloc(left, 4);
-    if (e != hipSuccess) return err(1, "assign_groups: device allocation failed");
+    Arena arena;
+    arena.add(status, (size_t)P * 4);
+    arena.add(last_n, (size_t)P * 4);
+    arena.add(last_v, (size_t)P * 4);
+    arena.add(cnt, (size_t)N * 4);
+    arena.add(props, (size_t)N * P * 4);
+    arena.add(holders, (size_t)N * cap * 4);
+    arena.add(hold_cnt, (size_t)N * 4);
+    arena.add(hold_v, (size_t)N * cap * 4);
+    arena.add(left, 4);
+    if (arena.allocate() != hipSuccess) return err(1, "assign_groups: device allocation failed");
     const int mx = P > N ? P : N;
     hipLaunchKernelGGL(k_assign_init, dim3((mx + 255) / 256), dim3(256), 0, st, status.as<int>(),
                        last_n.as<int>(), last_v.as<float>(), P, hold_cnt.as<int>(), cnt.as<int>(), N);

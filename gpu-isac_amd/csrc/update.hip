@@ -22,19 +22,41 @@
 #include "isac_internal.h"
 #include "../../include/gpu_aln_pack.h"
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
 namespace isac {
 namespace {
 
+// One device allocation cut into arrays (256-byte aligned).
 struct Buf {
     void *p = nullptr;
-    ~Buf() {
-        if (p) (void)hipFree(p);
-    }
+    size_t bytes = 0;
     template <class T>
     T *as() { return static_cast<T *>(p); }
+};
+struct Arena {
+    std::vector<Buf *> parts;
+    void *base = nullptr;
+    ~Arena() {
+        if (base) (void)hipFree(base);
+    }
+    void add(Buf &b, size_t bytes) {
+        b.bytes = (std::max<size_t>(bytes, 4) + 255) & ~(size_t)255;
+        parts.push_back(&b);
+    }
+    hipError_t allocate() {
+        size_t total = 0;
+        for (Buf *b : parts) total += b->bytes;
+        const hipError_t e = hipMalloc(&base, total);
+        char *at = static_cast<char *>(base);
+        for (Buf *b : parts) {
+            b->p = at;
+            at += b->bytes;
+        }
+        return e;
+    }
 };
 
 int err(int code, const char *msg) {
@@ -54,23 +76,20 @@ int update_references(const float *imgs, int P, int D, const float *peak, const 
         return err(2, "isac_update_references_device: cutoff and falloff must be positive");
     const int Dh = D / 2 + 1;
     Buf tp, mir, post, raw, cnt, off, mem, avg, neg, work, tw, bad;
-    hipError_t e = hipSuccess;
-    auto alloc = [&](Buf &b, size_t bytes) {
-        if (e == hipSuccess) e = hipMalloc(&b.p, bytes);
-    };
-    alloc(tp, (size_t)P * sizeof(float4));
-    alloc(mir, (size_t)P * sizeof(int));
-    alloc(post, (size_t)P * sizeof(float2));
-    alloc(raw, (size_t)P * sizeof(float4));
-    alloc(cnt, (size_t)N * sizeof(int));
-    alloc(off, ((size_t)N + 1) * sizeof(int));
-    alloc(mem, (size_t)P * sizeof(int));
-    alloc(avg, (size_t)N * sizeof(double2));
-    alloc(neg, (size_t)N * sizeof(float2));
-    alloc(work, (size_t)N * D * Dh * sizeof(float2));
-    alloc(tw, (size_t)D * sizeof(float2));
-    alloc(bad, sizeof(int));
-    if (e != hipSuccess) return err(1, "isac_update_references_device: device allocation failed");
+    Arena arena;
+    arena.add(tp, (size_t)P * sizeof(float4));
+    arena.add(mir, (size_t)P * sizeof(int));
+    arena.add(post, (size_t)P * sizeof(float2));
+    arena.add(raw, (size_t)P * sizeof(float4));
+    arena.add(cnt, (size_t)N * sizeof(int));
+    arena.add(off, ((size_t)N + 1) * sizeof(int));
+    arena.add(mem, (size_t)P * sizeof(int));
+    arena.add(avg, (size_t)N * sizeof(double2));
+    arena.add(neg, (size_t)N * sizeof(float2));
+    arena.add(work, (size_t)N * D * Dh * sizeof(float2));
+    arena.add(tw, (size_t)D * sizeof(float2));
+    arena.add(bad, sizeof(int));
+    if (arena.allocate() != hipSuccess) return err(1, "isac_update_references_device: device allocation failed");
     std::vector<float2> twh(D);
     for (int m = 0; m < D; ++m) {
         const double a = -2.0 * M_PI * (double)m / (double)D;
@@ -83,7 +102,7 @@ int update_references(const float *imgs, int P, int D, const float *peak, const 
                     cnt.as<int>(), off.as<int>(), mem.as<int>(), avg.as<double2>(),
                     neg.as<float2>(), work.as<float2>(), tw.as<float2>(), bad.as<int>(),
                     reinterpret_cast<float2 *>(shift_avg_out), members_out};
-    e = launch_update_references(imgs, P, D, peak, cls, N, cutoff, falloff, w, refs,
+    const hipError_t e = launch_update_references(imgs, P, D, peak, cls, N, cutoff, falloff, w, refs,
                                  reinterpret_cast<float4 *>(params), st);
     if (e != hipSuccess) return err(1, "isac_update_references_device: launch failed");
     int flag = 0;

@@ -195,13 +195,35 @@ def check(lib=None):
 
 
 def get_c_ptr_array(images: Sequence[np.ndarray]):
-    """C array of float* to C-contiguous float32 images (bin/sp_isac2_gpu.py:166-174)."""
+    """C array of float* to C-contiguous float32 images (bin/sp_isac2_gpu.py:166-174).
+
+    Of a stack (one float32 C-contiguous array [n, ...]) the addresses are computed in one go."""
+    if type(images) is np.ndarray and images.ndim > 1 and images.size and images.dtype == np.float32 \
+            and images.flags["C_CONTIGUOUS"]:
+        n = images.shape[0]
+        addr = images.ctypes.data + images.strides[0] * np.arange(n, dtype=np.uintp)
+        out = (float_ptr * n).from_buffer(addr)
+        out._images = images   # lives as long as the pointers
+        return out
     ptrs = []
     for img in images:
         assert img.flags["C_CONTIGUOUS"]
         assert img.dtype == np.float32
         ptrs.append(img.ctypes.data_as(float_ptr))
     return (float_ptr * len(ptrs))(*ptrs)
+
+
+def _param_records(prm, n: int) -> np.ndarray:
+    """The library's n AlignParam records as a structured array (a view)."""
+    if n == 0:
+        return np.empty(0, np.dtype(AlignParam))
+    return np.frombuffer((AlignParam * n).from_address(ctypes.addressof(prm.contents)), np.dtype(AlignParam))
+
+
+def _set_shifts(prm, acc: np.ndarray):
+    rec = _param_records(prm, len(acc))
+    rec["shift_x"] = acc[:, 0]
+    rec["shift_y"] = acc[:, 1]
 
 
 def make_config(sbj_num, ref_num, img_dim, ring_num, shift_step, shift_rng_x, shift_rng_y,
@@ -234,17 +256,10 @@ def multi_ref_align(sbj: np.ndarray, ref: np.ndarray, ring_num: int, shift_step:
     try:
         check(lib)
         if acc_xy is not None:
-            acc = np.asarray(acc_xy, dtype=np.float64).reshape(P, 2)
-            for i in range(P):
-                prm[i].shift_x = float(acc[i, 0])
-                prm[i].shift_y = float(acc[i, 1])
+            _set_shifts(prm, np.asarray(acc_xy, dtype=np.float64).reshape(P, 2))
         else:
-            for i in range(P):
-                prm[i].shift_x = 0.0
-                prm[i].shift_y = 0.0
-        imgs_s = [sbj[i] for i in range(P)]
-        imgs_r = [ref[i] for i in range(N)]
-        lib.multi_ref_align(get_c_ptr_array(imgs_s), get_c_ptr_array(imgs_r),
+            _set_shifts(prm, np.zeros((P, 2)))
+        lib.multi_ref_align(get_c_ptr_array(sbj), get_c_ptr_array(ref),
                             peak_list.ctypes.data_as(float_ptr), d.ctypes.data_as(float_ptr),
                             ctypes.c_uint(pitch), ctypes.c_float(mem_request))
         check(lib)
@@ -267,11 +282,10 @@ def post_rotate(peak_list: np.ndarray) -> np.ndarray:
 
 
 def params_to_numpy(prm, n: int) -> dict:
-    return {"shift_x": np.array([prm[i].shift_x for i in range(n)], np.float32),
-            "shift_y": np.array([prm[i].shift_y for i in range(n)], np.float32),
-            "angle": np.array([prm[i].angle for i in range(n)], np.float32),
-            "mirror": np.array([int(prm[i].mirror) for i in range(n)], np.int32),
-            "ref_id": np.array([prm[i].ref_id for i in range(n)], np.int32)}
+    rec = _param_records(prm, n)
+    return {"shift_x": rec["shift_x"].astype(np.float32), "shift_y": rec["shift_y"].astype(np.float32),
+            "angle": rec["angle"].astype(np.float32), "mirror": rec["mirror"].astype(np.int32),
+            "ref_id": rec["ref_id"].astype(np.int32)}
 
 
 def pre_align(data: np.ndarray, ref: np.ndarray, ring_num: int, shift_rng: float,
@@ -298,14 +312,11 @@ def pre_align(data: np.ndarray, ref: np.ndarray, ring_num: int, shift_rng: float
     try:
         check(lib)
         if acc_xy is not None:
-            acc = np.asarray(acc_xy, dtype=np.float64).reshape(n, 2)
-            for i in range(n):
-                prm[i].shift_x = float(acc[i, 0])
-                prm[i].shift_y = float(acc[i, 1])
+            _set_shifts(prm, np.asarray(acc_xy, dtype=np.float64).reshape(n, 2))
         n_batch = (n + batch - 1) // batch
         ref_img = np.ascontiguousarray(ref, dtype=np.float32).reshape(1, D, D)[0]
         if n_batch == 1:
-            lib.pre_align_fetch(get_c_ptr_array([data[i] for i in range(n)]), ctypes.c_uint(n),
+            lib.pre_align_fetch(get_c_ptr_array(data), ctypes.c_uint(n),
                                 b"sbj_batch")
             check(lib)
         for _ in range(iterations):
@@ -314,7 +325,7 @@ def pre_align(data: np.ndarray, ref: np.ndarray, ring_num: int, shift_rng: float
             for b in range(n_batch):
                 s0, s1 = b * batch, min(n, (b + 1) * batch)
                 if n_batch > 1:
-                    lib.pre_align_fetch(get_c_ptr_array([data[i] for i in range(s0, s1)]),
+                    lib.pre_align_fetch(get_c_ptr_array(data[s0:s1]),
                                         ctypes.c_uint(s1 - s0), b"sbj_batch")
                     check(lib)
                 lib.pre_align_run(ctypes.c_int(s0), ctypes.c_int(s1))
@@ -336,17 +347,13 @@ def ref_free_align(sbj: np.ndarray, cid: np.ndarray, avg: np.ndarray, ring_num: 
     cid = np.asarray(cid, dtype=np.int32)
     avg = np.ascontiguousarray(avg, dtype=np.float32)
     cfg = make_config(P, int(cid[-1]) + 1, D, ring_num, 1.0, shift_rng, shift_rng, "multigroup_aln")
-    cid_c = (ctypes.c_int * P)(*[int(c) for c in cid])
-    prm = lib.ref_free_alignment_2D_init(ctypes.byref(cfg), get_c_ptr_array([sbj[i] for i in range(P)]),
-                                         get_c_ptr_array([avg[k] for k in range(avg.shape[0])]),
+    cid_c = (ctypes.c_int * P)(*cid.tolist())
+    prm = lib.ref_free_alignment_2D_init(ctypes.byref(cfg), get_c_ptr_array(sbj), get_c_ptr_array(avg),
                                          cid_c, ctypes.c_uint(device))
     try:
         check(lib)
         if acc_xy is not None:
-            acc = np.asarray(acc_xy, dtype=np.float64).reshape(P, 2)
-            for i in range(P):
-                prm[i].shift_x = float(acc[i, 0])
-                prm[i].shift_y = float(acc[i, 1])
+            _set_shifts(prm, np.asarray(acc_xy, dtype=np.float64).reshape(P, 2))
         for i in range(num_iter):
             if cutoff_freq > 0.0:
                 freq = 0.1 + (cutoff_freq - 0.1) * i / float(max(num_iter - 1, 1))
@@ -665,10 +672,8 @@ def classes_from_assignment(groups, n_ref):
     if cap < 1:
         raise ValueError(f"{P} particles cannot fill {n_ref} classes (the driver divides by n_img // n_ref)")
     cls = np.zeros(P, np.int32)
-    for i in range(cap * n_ref):
-        cls[g[i]] = i // cap
-    for i in range(P % cap):
-        cls[g[cap * n_ref + i]] = g[-1]
+    cls[g[:cap * n_ref]] = np.repeat(np.arange(n_ref, dtype=np.int32), cap)
+    cls[g[cap * n_ref:cap * n_ref + P % cap]] = g[-1]
     return cls
 
 
