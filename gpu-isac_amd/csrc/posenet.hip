@@ -331,6 +331,69 @@ __global__ __launch_bounds__(256) void k_conv_mfma(const unsigned short *__restr
     }
 }
 
+// ------------------------------------------------------------ dense layer of few rows
+// k_conv_mfma<1> for few pixels (the dense layers at a training batch): its 64 x 64 tiles
+// are then a handful of wavefronts, each waiting for the loads of one k-step after the
+// other.  Here a wavefront owns 16 rows x 16 output channels and keeps the loads of
+// kDenseAhead k-steps in flight.  The chain over the k-steps is the same, so the outputs
+// are bit-identical.
+// What bounds it: the latency of Cin / (16 kDenseAhead) rounds of loads.  256
+// rows, 2592 -> 384: 29 us (k_conv_mfma 103), 384 -> 304: 10 (25), 304 -> 384: 7 (19).
+constexpr int kDenseAhead = 12;
+constexpr size_t kDenseTiles = 32;
+
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void k_dense(const unsigned short *__restrict__ x, long long rows, int Cin,
+                                               const unsigned short *__restrict__ w,
+                                               const float *__restrict__ bias, int bias_stride, int Cout,
+                                               int relu, void *__restrict__ yv) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lk = (lane >> 4) * 4;
+    const long long P = ((long long)blockIdx.x * 4 + wave) * 16 + li;
+    if (P - li >= rows) return;   // uniform over the wavefront; no barriers below
+    const bool pval = P < rows;
+    const int cb0 = blockIdx.y * 16, NK = Cin / 16;
+    const unsigned short *xr = x + (size_t)(pval ? P : 0) * Cin + lk;
+    const unsigned short *wr = w + (size_t)(cb0 + li) * Cin + lk;   // Cout is a multiple of 16
+    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint2 a0[kDenseAhead], b0[kDenseAhead], a1[kDenseAhead], b1[kDenseAhead];
+    auto load = [&](int ks, uint2 (&a)[kDenseAhead], uint2 (&b)[kDenseAhead]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDenseAhead; ++j) {
+            const int k = min(ks + j, NK - 1);   // past the end: loaded, not used
+            a[j] = *reinterpret_cast<const uint2 *>(wr + 16 * k);
+            b[j] = *reinterpret_cast<const uint2 *>(xr + 16 * k);
+        }
+    };
+    auto mma = [&](int ks, const uint2 (&a)[kDenseAhead], const uint2 (&b)[kDenseAhead])
+        __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDenseAhead; ++j)
+            if (ks + j < NK) acc = mfma_bf16(a[j], pval ? b[j] : make_uint2(0u, 0u), acc);
+    };
+    load(0, a0, b0);
+    for (int ks = 0; ks < NK; ks += 2 * kDenseAhead) {
+        load(ks + kDenseAhead, a1, b1);
+        mma(ks, a0, b0);
+        load(ks + 2 * kDenseAhead, a0, b0);
+        mma(ks + kDenseAhead, a1, b1);
+    }
+    if (!pval) return;
+    const int co = cb0 + lk;
+    float o[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        o[v] = acc[v] + (bias ? bias[(size_t)(co + v) * bias_stride] : 0.0f);
+        if (relu) o[v] = fmaxf(o[v], 0.0f);
+    }
+    if (OUT_F32)
+        *reinterpret_cast<float4 *>(static_cast<float *>(yv) + (size_t)P * Cout + co) =
+            make_float4(o[0], o[1], o[2], o[3]);
+    else
+        *reinterpret_cast<uint2 *>(static_cast<unsigned short *>(yv) + (size_t)P * Cout + co) =
+            pack4(o[0], o[1], o[2], o[3]);
+}
+
 // ------------------------------------------------------------ banded pooled convolution
 // Inference form of k_conv_mfma<3, false, true> for Cout in {64, 128, 256}:
 // workgroup = (image, band of P pooled rows).  The band's input rows
@@ -1241,6 +1304,20 @@ int isac_nn_conv_fwd(const uint16_t *x, int n, int H, int W, int Cin, const uint
         }
     }
     dim3 grid(blocks_for(np, 256), (unsigned)((Cout + 63) / 64));
+    // few rows: k_conv_mfma would have at most kDenseTiles workgroups.  Its time hardly
+    // changes up to 256 of them, k_dense's grows by its 16-row tiles' repeated loads: 24
+    // workgroups 57 us against 103 (2592 -> 384) and 18 against 25 (384 -> 304), 41
+    // workgroups 26 against 27 (384 -> 2592), 96 workgroups 166 against 114
+    if (ks == 1 && (size_t)grid.x * grid.y <= kDenseTiles) {
+        const dim3 dg(blocks_for(np, 64), (unsigned)(Cout / 16));
+        if (out_f32)
+            hipLaunchKernelGGL(k_dense<true>, dg, dim3(256), 0, st, x, (long long)np, Cin, w, bias, bias_stride,
+                               Cout, relu, y);
+        else
+            hipLaunchKernelGGL(k_dense<false>, dg, dim3(256), 0, st, x, (long long)np, Cin, w, bias, bias_stride,
+                               Cout, relu, y);
+        return launched("isac_nn_conv_fwd");
+    }
     if (ks == 3 && !out_f32)
         hipLaunchKernelGGL((k_conv_mfma<3, false>), grid, dim3(256), 0, st, x, n, H, W, Cin, w, bias,
                            bias_stride, Cout, relu, y);
