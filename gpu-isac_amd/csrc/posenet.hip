@@ -10,7 +10,7 @@
 // A wavefront owns 64 output channels x 64 pixels (16 accumulator blocks); a
 // workgroup is 4 wavefronts along the pixels.  The same kernel computes the
 // input gradient of a layer from the flipped weights.  The weight gradient is
-// a reduction over pixels and runs on the vector ALUs from LDS tiles, split
+// a reduction over pixels and runs on the matrix cores from LDS tiles, split
 // over pixel ranges into partial sums that a second kernel adds in a fixed
 // order.  No reference counterpart: the reference has no learned component.
 #include "isac_internal.h"
@@ -842,10 +842,19 @@ __global__ void k_relu_bwd(const unsigned short *__restrict__ y, const unsigned 
 // consecutive pixels are one 16-byte read (A: co = l % 32, pixels 16 s + 8 (l / 32)
 // ..; B: k = l % 32, the same pixels).  Products of bf16 values are exact in FP32.
 // Blocks along z take pixel ranges [z chunk, (z + 1) chunk) and write partial
-// sums part[z][Cout][K + 1], added in a fixed order by k_sum_parts.
+// sums part[z][Cout][K + 1], added in a fixed order by k_sum_parts (one range: the
+// gradient itself).
+// What bounds it: the latency of a stage's loads, so the next stage's are in flight over
+// the products, and workgroups are made until eight share a CU;
+// then vector instructions and LDS writes of the staging.  Batch 256: 370 k pixels,
+// 32 -> 64: 68 us (87 with loads waited for, 64-bit divisions and 482 ranges), 92 k, 64 ->
+// 128: 63 (82), 1.5 M, 1 -> 32: 61 (130).
 constexpr int kWgPix = 64;              // pixels per stage
 constexpr int kWgRow = kWgPix + 8;      // bf16 per LDS row: rows 8 apart fall 32 banks apart
 
+// DV: Cout is a multiple of 8.  XV: so is Cin, and a column group is 8 channels of one tap
+// or the bias.
+template <bool DV, bool XV>
 __global__ __launch_bounds__(256) void k_wgrad(const unsigned short *__restrict__ x,
                                                const unsigned short *__restrict__ dz, int n, int H,
                                                int W, int Cin, int Cout, int KS, long long chunk,
@@ -855,76 +864,102 @@ __global__ __launch_bounds__(256) void k_wgrad(const unsigned short *__restrict_
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int K = KS * KS * Cin, K1 = K + 1;
     const int k0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
-    const long long NP = (long long)n * H * W;
+    const unsigned HW = (unsigned)H * W;
+    const long long NP = (long long)n * HW;
     const long long p0 = (long long)blockIdx.z * chunk;
-    const long long p1 = min(NP, p0 + chunk);
+    const long long p1 = min(NP, p0 + chunk);   // > p0
     const int wm = wave >> 1, wn = wave & 1;
     // staging: pixel pair pp (stage pixels 2 pp, 2 pp + 1), column group cg (8 columns)
     const int pp = tid & 31, cg = tid >> 5;
     const int cb = c0 + 8 * cg, kb = k0 + 8 * cg;
-    const bool dvec = (Cout % 8 == 0) && cb + 8 <= Cout;
-    const bool xvec = (Cin % 8 == 0) && kb + 8 <= K;   // 8 channels of one tap
-    float16_t acc = {};
-    for (long long pc = p0; pc < p1; pc += kWgPix) {
-        unsigned dw[8], xw[8];   // (pixel 2 pp, pixel 2 pp + 1) per column
+    // tap offsets and element offset of the group's columns
+    constexpr int NE = XV ? 1 : 8;
+    int kdy[NE], kdx[NE], kof[NE];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dw[e] = xw[e] = 0u;
+    for (int e = 0; e < NE; ++e) {
+        const int k = min(kb + e, K - 1), t = k / Cin, ci = k - t * Cin;
+        kdy[e] = t / KS - KS / 2;
+        kdx[e] = t % KS - KS / 2;
+        kof[e] = (kdy[e] * W + kdx[e]) * Cin + ci;
+    }
+    const unsigned inv_hw = 0xffffffffu / HW, inv_w = 0xffffffffu / (unsigned)W;
+    // quotient of a < 2^31 by d from floor((2^32 - 1) / d): at most one too small
+    auto divide = [](unsigned a, unsigned d, unsigned inv, unsigned &rem) __attribute__((always_inline)) {
+        unsigned q = __umulhi(a, inv);
+        rem = a - q * d;
+        if (rem >= d) {
+            rem -= d;
+            ++q;
+        }
+        return q;
+    };
+    unsigned rem0 = (unsigned)(p0 % HW);   // the stage's first pixel within its image
+    long long left = p1 - p0 - 2 * pp;     // pixels from this lane's first to the range's end
+    const unsigned short *xp = x + (size_t)(p0 + 2 * pp) * Cin;
+    const unsigned short *dp = dz + (size_t)(p0 + 2 * pp) * Cout + cb;
+    // per pixel four words of two columns, or a word per column
+    unsigned dr[2][DV ? 4 : 8], xr[2][XV ? 4 : 8];
+    auto load = [&]() __attribute__((always_inline)) {
+        unsigned rem, px, py;
+        divide(rem0 + 2 * pp, HW, inv_hw, rem);
+        py = divide(rem, W, inv_w, px);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const long long P = pc + 2 * pp + h;
-            if (P >= p1) continue;
-            unsigned short d8[8], x8[8];
-            if (dvec) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(dz + (size_t)P * Cout + cb);
-                const unsigned vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) d8[e] = (unsigned short)(vv[e / 2] >> (16 * (e & 1)));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    d8[e] = (cb + e < Cout) ? dz[(size_t)P * Cout + cb + e] : (unsigned short)0;
-            }
-            const int img = (int)(P / ((long long)H * W));
-            const int rem = (int)(P - (long long)img * H * W);
-            const int py = rem / W, px = rem - py * W;
-            if (xvec) {
-                const int t = kb / Cin, ci = kb - t * Cin;
-                const int sy = py + t / KS - KS / 2, sx2 = px + t % KS - KS / 2;
+            const bool in = h < left;
+            auto inside = [&](int e) __attribute__((always_inline)) {
+                return (unsigned)((int)py + kdy[e]) < (unsigned)H && (unsigned)((int)px + kdx[e]) < (unsigned)W;
+            };
+            if constexpr (DV) {
                 uint4 v = make_uint4(0u, 0u, 0u, 0u);
-                if (sy >= 0 && sy < H && sx2 >= 0 && sx2 < W)
-                    v = *reinterpret_cast<const uint4 *>(x + (((size_t)img * H + sy) * W + sx2) * Cin + ci);
-                const unsigned vv[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x8[e] = (unsigned short)(vv[e / 2] >> (16 * (e & 1)));
+                if (in && cb < Cout) v = *reinterpret_cast<const uint4 *>(dp + h * Cout);
+                dr[h][0] = v.x, dr[h][1] = v.y, dr[h][2] = v.z, dr[h][3] = v.w;
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const int k = kb + e;
-                    unsigned short xv = 0;
-                    if (k == K) {
-                        xv = 0x3f80;   // bf16 1.0: the bias column
-                    } else if (k < K) {
-                        const int t = k / Cin, ci = k - t * Cin;
-                        const int sy = py + t / KS - KS / 2, sx2 = px + t % KS - KS / 2;
-                        if (sy >= 0 && sy < H && sx2 >= 0 && sx2 < W)
-                            xv = x[(((size_t)img * H + sy) * W + sx2) * Cin + ci];
-                    }
-                    x8[e] = xv;
+                    dr[h][e] = 0u;
+                    if (in && cb + e < Cout) dr[h][e] = dp[h * Cout + e];
                 }
             }
+            if constexpr (XV) {
+                uint4 u = make_uint4(0u, 0u, 0u, 0u);
+                if (in && kb == K) u.x = 0x3f80u;   // bf16 1.0: the bias column
+                if (in && kb < K && inside(0)) u = *reinterpret_cast<const uint4 *>(xp + h * Cin + kof[0]);
+                xr[h][0] = u.x, xr[h][1] = u.y, xr[h][2] = u.z, xr[h][3] = u.w;
+            } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                dw[e] |= (unsigned)d8[e] << (16 * h);
-                xw[e] |= (unsigned)x8[e] << (16 * h);
+                for (int e = 0; e < 8; ++e) {
+                    xr[h][e] = (in && kb + e == K) ? 0x3f80u : 0u;
+                    if (in && kb + e < K && inside(e)) xr[h][e] = xp[h * Cin + kof[e]];
+                }
+            }
+            if (++px == (unsigned)W) {
+                px = 0;
+                if (++py == (unsigned)H) py = 0;
             }
         }
+        divide(rem0 + kWgPix, HW, inv_hw, rem);
+        rem0 = rem;
+        left -= kWgPix;
+        xp += (size_t)kWgPix * Cin;
+        dp += (size_t)kWgPix * Cout;
+    };
+    // column e of the stage: pixels 2 pp and 2 pp + 1 in one word
+    auto pair = [](const auto &r, int e) __attribute__((always_inline)) {
+        if constexpr (sizeof(r[0]) == 32) return r[0][e] | (r[1][e] << 16);
+        const unsigned a = r[0][e / 2], b = r[1][e / 2];
+        return (e & 1) ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
+    };
+    float16_t acc = {};
+    load();
+    for (long long pc = p0; pc < p1; pc += kWgPix) {
         __syncthreads();   // the previous stage's operand reads are done
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            *reinterpret_cast<unsigned *>(sd + (8 * cg + e) * kWgRow + 2 * pp) = dw[e];
-            *reinterpret_cast<unsigned *>(sx + (8 * cg + e) * kWgRow + 2 * pp) = xw[e];
+            *reinterpret_cast<unsigned *>(sd + (8 * cg + e) * kWgRow + 2 * pp) = pair(dr, e);
+            *reinterpret_cast<unsigned *>(sx + (8 * cg + e) * kWgRow + 2 * pp) = pair(xr, e);
         }
         __syncthreads();
+        if (pc + kWgPix < p1) load();
 #pragma unroll
         for (int s = 0; s < kWgPix / 16; ++s) {
             const int off = 16 * s + 8 * (lane >> 5);
@@ -943,12 +978,23 @@ __global__ __launch_bounds__(256) void k_wgrad(const unsigned short *__restrict_
     }
 }
 
-__global__ void k_sum_parts(const float *__restrict__ part, int nparts, size_t count,
-                            float *__restrict__ g) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
+// Workgroup = 64 elements; wavefront w adds the parts w, w + 16, ..., and the first one
+// the sixteen sums in order.  A thread for an element and all its parts left 320 elements
+// of 503 parts waiting for one load after the other (117 us, now 8).
+__global__ __launch_bounds__(1024) void k_sum_parts(const float *__restrict__ part, int nparts, size_t count,
+                                                    float *__restrict__ g) {
+    __shared__ float red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t i = (size_t)blockIdx.x * 64 + lane;
     float s = 0.0f;
-    for (int z = 0; z < nparts; ++z) s += part[(size_t)z * count + i];
+    if (i < count) {
+#pragma unroll 8
+        for (int z = wave; z < nparts; z += 16) s += part[(size_t)z * count + i];
+    }
+    red[wave][lane] = s;
+    __syncthreads();
+    if (wave > 0 || i >= count) return;
+    for (int w = 1; w < 16; ++w) s += red[w][lane];
     g[i] = s;
 }
 
@@ -1450,18 +1496,27 @@ int isac_nn_conv_wgrad(const uint16_t *x, const uint16_t *dz, int n, int H, int 
     const int K1 = ks * ks * Cin + 1;
     const size_t per = (size_t)Cout * K1 * sizeof(float);
     const long long NP = (long long)n * H * W;
+    // pixel ranges of at least 512, until eight workgroups share a CU
+    const unsigned gx = (unsigned)((K1 + 63) / 64), gy = (unsigned)((Cout + 63) / 64);
     long long nparts = (long long)(part_bytes / per);
-    nparts = std::min<long long>(nparts, std::max<long long>(1, NP / 512));
-    nparts = std::min<long long>(nparts, 512);
     if (nparts < 1) return fail(2, "isac_nn_conv_wgrad: scratch smaller than one partial sum");
+    nparts = std::min<long long>(nparts, std::max<long long>(1, NP / 512));
+    nparts = std::min<long long>(nparts, std::max<long long>(1, 2048 / ((long long)gx * gy)));
     const long long chunk = ((NP + nparts - 1) / nparts + kWgPix - 1) / kWgPix * kWgPix;
     nparts = (NP + chunk - 1) / chunk;
     hipStream_t st = (hipStream_t)stream;
-    dim3 grid((unsigned)((K1 + 63) / 64), (unsigned)((Cout + 63) / 64), (unsigned)nparts);
-    hipLaunchKernelGGL(k_wgrad, grid, dim3(256), 0, st, x, dz, n, H, W, Cin, Cout, ks, chunk, part);
+    float *out = nparts == 1 ? g : part;
+    const dim3 grid(gx, gy, (unsigned)nparts);
+    if (Cout % 8 == 0 && Cin % 8 == 0)
+        hipLaunchKernelGGL((k_wgrad<true, true>), grid, dim3(256), 0, st, x, dz, n, H, W, Cin, Cout, ks, chunk, out);
+    else if (Cout % 8 == 0)
+        hipLaunchKernelGGL((k_wgrad<true, false>), grid, dim3(256), 0, st, x, dz, n, H, W, Cin, Cout, ks, chunk, out);
+    else
+        hipLaunchKernelGGL((k_wgrad<false, false>), grid, dim3(256), 0, st, x, dz, n, H, W, Cin, Cout, ks, chunk, out);
     if (int e = launched("isac_nn_conv_wgrad")) return e;
+    if (nparts == 1) return 0;
     const size_t cnt = (size_t)Cout * K1;
-    hipLaunchKernelGGL(k_sum_parts, dim3(blocks_for(cnt, 256)), dim3(256), 0, st, part, (int)nparts, cnt, g);
+    hipLaunchKernelGGL(k_sum_parts, dim3(blocks_for(cnt, 64)), dim3(1024), 0, st, part, (int)nparts, cnt, g);
     return launched("isac_nn_conv_wgrad (sum)");
 }
 

@@ -37,3 +37,33 @@ def test_dense_rows_equal_the_large_batch(gpu, n, cin, cout, relu, f32):
     # sums of cin products in FP32, and the output's rounding
     np.testing.assert_allclose(got.double().cpu().numpy(), ref, rtol=2.0 ** -23 if f32 else 2.0 ** -8,
                                atol=cin * 2.0 ** -22)
+
+
+@pytest.mark.parametrize("n,H,W,cin,cout,ks,parts", [
+    (1, 1, 1, 16, 16, 1, 4),        # one pixel, one part
+    (129, 1, 1, 24, 40, 1, 4),      # images of one pixel, several to a stage
+    (70, 7, 5, 1, 32, 3, 3),        # one channel, images across stages, a short last range
+    (3, 61, 67, 1, 32, 3, 40),      # more parts than a workgroup of the sum has wavefronts
+    (2, 33, 32, 24, 72, 3, 2),      # partial column and channel tiles, ranges that end in a stage
+    (5, 2, 300, 64, 20, 3, 1),      # channels not a multiple of 8
+    (700, 2, 1, 16, 136, 1, 17),
+])
+def test_weight_gradient_edges(gpu, n, H, W, cin, cout, ks, parts):
+    """Against 64-bit sums over the pixels; a product is exact in FP32, so a sum of m of
+    them is within m 2^-24 of the sum of their magnitudes."""
+    import torch
+    rng = np.random.default_rng(n + cin + H)
+    x, dz = _bf16(rng, n, H, W, cin), _bf16(rng, n, H, W, cout)
+    K1 = ks * ks * cin + 1
+    g = torch.full((cout, K1), float("nan"), device="cuda")
+    part = torch.empty(parts * cout * K1, device="cuda")
+    _call("isac_nn_conv_wgrad", x, dz, n, H, W, cin, cout, ks, g, part, part.numel() * 4)
+    torch.cuda.synchronize()
+    r = ks // 2
+    xp = torch.nn.functional.pad(x.double().cpu(), (0, 0, r, r, r, r))
+    cols = torch.cat([xp[:, i:i + H, j:j + W] for i in range(ks) for j in range(ks)], -1).reshape(n * H * W, -1)
+    cols = torch.cat([cols, torch.ones(n * H * W, 1, dtype=torch.float64)], 1)
+    d = dz.double().cpu().reshape(n * H * W, cout)
+    want, mag = d.T @ cols, d.abs().T @ cols.abs()
+    err = (g.double().cpu() - want).abs()
+    assert bool((err <= n * H * W * 2.0 ** -24 * mag + 1e-30).all()), float((err / (mag + 1e-30)).max())
