@@ -579,6 +579,7 @@ __device__ __forceinline__ float16_t mfma32_bf16(uint4 a, uint4 b, float16_t c) 
 
 constexpr int kResidentLdsMax = 63 * 1024;   // dynamic band; with the static bias copy <= 64 KB
 constexpr int kResidentCoutMax = 128;
+constexpr int kConvBandMax = 31 * 1024;      // band of k_conv_resident<32> and <64>: see their launch
 
 // First maximum (in lane order) of the four lanes of a quad, valid in lane 4k:
 // the pairs (4k, 4k+1) and (4k+2, 4k+3) keep their first maximum, then the pair
@@ -671,12 +672,18 @@ __global__ __launch_bounds__(256, CIN == 32 ? 4 : 2) void k_conv_pool_resident(
 
 // ------------------------------------------------------------ 3x3 convolution, resident weights
 // Unpooled 3x3 convolution (pad 1, bias, optional ReLU, bf16 output) for Cin 32 /
-// 64 / 128 and Cout 16 / 32 / 64: persistent workgroups; each wavefront keeps
+// 64 / 128 and Cout 16 / 32 / 64, or tiles of 64 (blockIdx.y): persistent workgroups; each wavefront keeps
 // the A operands of its 16 output channels for all NK = 9 Cin / 16 k-steps in
 // registers (NK x 2 VGPRs) and streams 16-pixel blocks (row-major over a band
 // of rows, input band with halo staged in LDS as in the pooled forms) through
 // the fully unrolled k-steps on v_mfma_f32_16x16x16_bf16, in the order of
 // k_conv_mfma: the output is bit-identical to it.
+// What bounds it: a chain of NK dependent products and the LDS reads that feed them, so a
+// wavefront takes kResChains blocks at a time (four are no better), and the staging
+// between items.  Batch 256, 19 x 19, 64 -> 128: 54 us, 250 TFLOP/s (k_conv_mfma 106);
+// 38 x 38, 32 -> 64: 47 (71).
+constexpr int kResChains = 2;
+
 template <int CIN>
 __global__ __launch_bounds__(256, 2) void k_conv_resident(
     const unsigned short *__restrict__ x, int H, int W, const unsigned short *__restrict__ w,
@@ -686,14 +693,15 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
     extern __shared__ __align__(16) unsigned short band[];
     __shared__ __align__(16) float sbias[kResidentCoutMax];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < Cout; i += 256) sbias[i] = bias ? bias[(size_t)i * bias_stride] : 0.0f;
-    const int ncb = Cout / 16, wpc = 4 / ncb;   // co blocks of 16, wavefronts per co block
+    const int cy = blockIdx.y * 64, nco = min(Cout - cy, 64);
+    for (int i = tid; i < nco; i += 256) sbias[i] = bias ? bias[(size_t)(cy + i) * bias_stride] : 0.0f;
+    const int ncb = nco / 16, wpc = 4 / ncb;   // co blocks of 16, wavefronts per co block
     const int co0 = (wave / wpc) * 16, wi = wave % wpc;
     const int li = lane & 15, lk = (lane >> 4) * 4;
     uint2 wa[NK];
 #pragma unroll
     for (int s = 0; s < NK; ++s)
-        wa[s] = *reinterpret_cast<const uint2 *>(w + (size_t)(co0 + li) * K + 16 * s + lk);
+        wa[s] = *reinterpret_cast<const uint2 *>(w + (size_t)(cy + co0 + li) * K + 16 * s + lk);
     const int Wl = W + 2;
     for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
         const int img = item / nband, bnd = item - img * nband;
@@ -712,28 +720,40 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
         __syncthreads();
         const int npx = (r1 - r0) * W, nblk = (npx + 15) / 16;
         const size_t px0 = ((size_t)img * H + r0) * W;
-        for (int b = wi; b < nblk; b += wpc) {
-            const int px = 16 * b + li;
-            const bool pv = px < npx;
-            const int pc = pv ? px : 0;
-            const int pr = pc / W, pcl = pc - pr * W;
-            // top-left tap of the lane's pixel (band row / column of input pixel - 1)
-            const unsigned short *pb = band + pr * RS + pcl * Cs + lk;
-            float4_t acc = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int b = wi; b < nblk; b += kResChains * wpc) {
+            const unsigned short *pb[kResChains];
+            int px[kResChains];
+            float4_t acc[kResChains];
+#pragma unroll
+            for (int j = 0; j < kResChains; ++j) {
+                px[j] = 16 * (b + j * wpc) + li;
+                const int pc = px[j] < npx ? px[j] : 0;
+                const int pr = pc / W, pcl = pc - pr * W;
+                // top-left tap of the lane's pixel (band row / column of input pixel - 1)
+                pb[j] = band + pr * RS + pcl * Cs + lk;
+                acc[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
 #pragma unroll
             for (int s = 0; s < NK; ++s) {
                 const int t = s / CPT, c = (s % CPT) * 16;
-                const uint2 bv = *reinterpret_cast<const uint2 *>(pb + (t / 3) * RS + (t % 3) * Cs + c);
-                acc = mfma_bf16(wa[s], bv, acc);
+#pragma unroll
+                for (int j = 0; j < kResChains; ++j) {
+                    const uint2 bv = *reinterpret_cast<const uint2 *>(pb[j] + (t / 3) * RS + (t % 3) * Cs + c);
+                    acc[j] = mfma_bf16(wa[s], bv, acc[j]);
+                }
             }
             const int co = co0 + lk;
             const float4 bb = *reinterpret_cast<const float4 *>(sbias + co);
-            float o[4] = {acc[0] + bb.x, acc[1] + bb.y, acc[2] + bb.z, acc[3] + bb.w};
-            if (relu) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) o[v] = fmaxf(o[v], 0.0f);
+            for (int j = 0; j < kResChains; ++j) {
+                float o[4] = {acc[j][0] + bb.x, acc[j][1] + bb.y, acc[j][2] + bb.z, acc[j][3] + bb.w};
+                if (relu) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) o[v] = fmaxf(o[v], 0.0f);
+                }
+                if (px[j] < npx)
+                    *reinterpret_cast<uint2 *>(y + (px0 + px[j]) * Cout + cy + co) = pack4(o[0], o[1], o[2], o[3]);
             }
-            if (pv) *reinterpret_cast<uint2 *>(y + (px0 + px) * Cout + co) = pack4(o[0], o[1], o[2], o[3]);
         }
     }
 }
@@ -1300,14 +1320,18 @@ int isac_nn_conv_fwd(const uint16_t *x, int n, int H, int W, int Cin, const uint
     if (np == 0) return 0;
     hipStream_t st = (hipStream_t)stream;
     if (ks == 3 && !out_f32 && (Cin == 32 || Cin == 64 || Cin == 128) &&
-        (Cout == 16 || Cout == 32 || Cout == 64)) {
+        (Cout == 16 || Cout == 32 || Cout % 64 == 0)) {
         // resident-weight form: band height with the fewest wavefront rounds of
         // 16 pixels, plus half a round per band for its staging
         const int Cs = Cin + 8, Wl = W + 2;
         const int RS = Wl * Cs + ((64 - Wl * Cs % 128) + 128) % 128;
-        const int rmax = kResidentLdsMax / (RS * 2) - 2;
+        // Bands of 31 KB let four workgroups share a CU, one staging while others compute:
+        // 47 us against 68 with 63 KB (38 x 38, 32 -> 64, batch 256), 54 against 75 (19 x 19,
+        // 64 -> 128).  At 128 input channels the weights' registers leave two, and the
+        // larger band is the better one (9 x 9, 128 -> 32: 19 against 27)
+        const int rmax = (Cin == 128 ? kResidentLdsMax : kConvBandMax) / (RS * 2) - 2;
         if (rmax >= 1) {
-            const int wpc = 4 / (Cout / 16);
+            const int wpc = 4 / (std::min(Cout, 64) / 16);
             int TH = 1;
             double best = 1e30;
             for (int t = 1; t <= std::min(rmax, H); ++t) {
@@ -1334,17 +1358,18 @@ int isac_nn_conv_fwd(const uint16_t *x, int n, int H, int W, int Cin, const uint
                 hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, lds) != hipSuccess ||
                 per_cu < 1)
                 return fail(3, "isac_nn_conv_fwd: occupancy query failed");
-            const unsigned grid = (unsigned)std::min<long long>(items, (long long)cus * per_cu);
+            const unsigned gy = (unsigned)((Cout + 63) / 64);
+            const dim3 grid((unsigned)std::min<long long>(items, std::max(1ll, (long long)cus * per_cu / gy)), gy);
             const unsigned short *xw = x;
             unsigned short *yw = static_cast<unsigned short *>(y);
             if (Cin == 32)
-                hipLaunchKernelGGL(k_conv_resident<32>, dim3(grid), dim3(256), lds, st, xw, H, W, w, bias,
+                hipLaunchKernelGGL(k_conv_resident<32>, grid, dim3(256), lds, st, xw, H, W, w, bias,
                                    bias_stride, Cout, relu, TH, nband, (int)items, RS, yw);
             else if (Cin == 64)
-                hipLaunchKernelGGL(k_conv_resident<64>, dim3(grid), dim3(256), lds, st, xw, H, W, w, bias,
+                hipLaunchKernelGGL(k_conv_resident<64>, grid, dim3(256), lds, st, xw, H, W, w, bias,
                                    bias_stride, Cout, relu, TH, nband, (int)items, RS, yw);
             else
-                hipLaunchKernelGGL(k_conv_resident<128>, dim3(grid), dim3(256), lds, st, xw, H, W, w, bias,
+                hipLaunchKernelGGL(k_conv_resident<128>, grid, dim3(256), lds, st, xw, H, W, w, bias,
                                    bias_stride, Cout, relu, TH, nband, (int)items, RS, yw);
             return launched("isac_nn_conv_fwd");
         }

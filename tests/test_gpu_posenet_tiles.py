@@ -67,3 +67,19 @@ def test_weight_gradient_edges(gpu, n, H, W, cin, cout, ks, parts):
     want, mag = d.T @ cols, d.abs().T @ cols.abs()
     err = (g.double().cpu() - want).abs()
     assert bool((err <= n * H * W * 2.0 ** -24 * mag + 1e-30).all()), float((err / (mag + 1e-30)).max())
+
+
+@pytest.mark.parametrize("H,W,cin,cout", [(19, 19, 64, 128), (9, 9, 32, 192), (5, 3, 128, 64), (1, 1, 32, 16),
+                                          (38, 37, 32, 32), (2, 65, 128, 128)])
+def test_resident_conv_channel_tiles(gpu, H, W, cin, cout):
+    """Tiles of 64 output channels and several pixel blocks at a time, bit for bit the
+    unbanded kernel's (run at 208 channels, which is no multiple of 64)."""
+    import torch
+    rng = np.random.default_rng(H + W + cin)
+    x, w = _bf16(rng, 3, H, W, cin), _bf16(rng, 208, 9 * cin)
+    b = torch.from_numpy(rng.standard_normal(208).astype(np.float32)).cuda()
+    got, want = (torch.empty((3, H, W, c), dtype=torch.bfloat16, device="cuda") for c in (cout, 208))
+    _call("isac_nn_conv_fwd", x, 3, H, W, cin, w, b, 1, cout, 3, 1, 0, got)
+    _call("isac_nn_conv_fwd", x, 3, H, W, cin, w, b, 1, 208, 3, 1, 0, want)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want[..., :cout].contiguous())
