@@ -68,7 +68,7 @@ int isac_nn_relu_bwd(const uint16_t *y, const uint16_t *dy, size_t count, uint16
 /* Weight and bias gradient of a ks x ks layer (Cin >= 1, any Cout):
  * g [Cout][K+1] fp32 = sum over pixels of dz[p][co] * x-patch[p][k] (the last
  * column sums dz: the bias gradient).  part is scratch of part_bytes; the
- * pixel range is split into as many partial sums as fit (fixed order, so the
+ * pixel range is split into at most as many partial sums as fit (fixed order, so the
  * result is deterministic). */
 int isac_nn_conv_wgrad(const uint16_t *x, const uint16_t *dz, int n, int H, int W, int Cin,
                        int Cout, int ks, float *g, float *part, size_t part_bytes, void *stream);
