@@ -340,9 +340,11 @@ __device__ __forceinline__ float2 ring_norm(double a, double q, int R) {
     return f2((float)(mu * kRingLen), (float)(1.0 / (sd + 1e-7)));
 }
 
-// LDS floats of a polar kernel with nw wavefronts: lane twiddles, exchange buffers, image.
-__host__ __device__ constexpr int polar_lds_floats(int D, int nw) {
-    return 2 * kIfftTw + nw * 4 * kXchLd + (D + 2) * (D + 2);
+// LDS floats of a polar kernel with nw wavefronts: lane twiddles, parts of the sums of ring
+// pairs split over `split` wavefronts, exchange buffers, image.
+__host__ __device__ constexpr int polar_part_floats(int split) { return split > 1 ? split * kWave * 4 : 0; }
+__host__ __device__ constexpr int polar_lds_floats(int D, int nw, int split = 1) {
+    return 2 * kIfftTw + polar_part_floats(split) + nw * 4 * kXchLd + (D + 2) * (D + 2);
 }
 
 // Bordered copy of an image (see tap), all threads; the caller synchronises.
@@ -355,10 +357,13 @@ __device__ __forceinline__ void load_bordered(float *img, const float *src, int 
 }
 
 // Samples and transform of ring pair (i, i + 1) of one row about (cx, cy): lane u takes
-// angles u + 16 m; sums (FP64) into sA, sQ; spectra of both rings out (b = 0 past R).
-__device__ __forceinline__ void ring_pair(const float *img1, float Wf, float lim, int W, const float2 *tmpl, int i,
-                                          int R, float cx, float cy, int u, float *xb, const float2 *tw, double &sA,
-                                          double &sQ, float2 (&a)[8], float2 (&b)[8]) {
+// angles u + 16 m; spectra of both rings out (b = 0 past R).  Returns the lane's part of the
+// pair's sums (FP64).  A lane's parts are added in ring order from 0, then its row's lanes,
+// whichever wavefronts took the pairs: a row's sums do not depend on the launch's shape.  (A
+// variance far below the mean's square shows any other order.)
+__device__ __forceinline__ double2 ring_pair(const float *img1, float Wf, float lim, int W, const float2 *tmpl, int i,
+                                             int R, float cx, float cy, int u, float *xb, const float2 *tw,
+                                             float2 (&a)[8], float2 (&b)[8]) {
     float2 x[16];
     const float2 *ta = tmpl + (size_t)i * kRingLen + u;
     double a1 = 0.0, a2 = 0.0, b1 = 0.0, b2 = 0.0;
@@ -378,10 +383,10 @@ __device__ __forceinline__ void ring_pair(const float *img1, float Wf, float lim
         b2 = fma(db, db, b2);
     }
     const double wa = (double)(i + 1), wb = (double)(i + 2);
-    sA += wa * a1 + wb * b1;
-    sQ += wa * a2 + wb * b2;
+    const double2 sum = make_double2(fma(wa, a1, wb * b1), fma(wa, a2, wb * b2));
     fft256_rows4(x, xb, tw, u);
     unpack_rings(x, a, b, xb, u);
+    return sum;
 }
 
 // A lane's slots u + 16 m of one ring row: four 16-byte accesses (slot_re).
@@ -411,7 +416,6 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     float2 *__restrict__ spec, float2 *__restrict__ norm,
     const unsigned long long *__restrict__ smask, int split) {
     extern __shared__ float4 smem4[];
-    __shared__ double red[2][4 * 16];
     __shared__ int slist[64];
     __shared__ int scnt;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -419,8 +423,9 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     const int p = blockIdx.x;
     if (MASKED && smask[p] == 0ull) return;   // uniform over the workgroup
     float2 *tw = reinterpret_cast<float2 *>(smem4);
-    float *xb = reinterpret_cast<float *>(tw + kIfftTw) + (wave * 4 + f) * kXchLd;
-    float *img = reinterpret_cast<float *>(tw + kIfftTw) + nw * 4 * kXchLd;
+    double2 *part = reinterpret_cast<double2 *>(tw + kIfftTw);   // [wavefront][lane], where split
+    float *xb0 = reinterpret_cast<float *>(tw + kIfftTw) + polar_part_floats(split);
+    float *xb = xb0 + (wave * 4 + f) * kXchLd, *img = xb0 + nw * 4 * kXchLd;
     const int W = D + 2;
     load_bordered(img, imgs + (size_t)p * D * D, D);
     fill_ifft_twiddles(tw, twg, tid, blockDim.x);
@@ -450,28 +455,36 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
         const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
         double sA = 0.0, sQ = 0.0;
         float2 *row = spec + ((size_t)p * S + s) * (size_t)R * kSlots;
-        for (int i = 2 * q0; i < R; i += 2 * split) {
-            float2 a[8], b[8];
-            ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, sA, sQ, a, b);
-            if (live) {
-                store_slots(row + (size_t)i * kSlots, a, u);
-                if (i + 1 < R) store_slots(row + (size_t)(i + 1) * kSlots, b, u);
+        for (int i0 = 0; i0 < R; i0 += 2 * split) {
+            const int i = i0 + 2 * q0;   // uniform over the wavefront
+            double2 t = make_double2(0.0, 0.0);
+            if (i < R) {
+                float2 a[8], b[8];
+                t = ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, a, b);
+                if (live) {
+                    store_slots(row + (size_t)i * kSlots, a, u);
+                    if (i + 1 < R) store_slots(row + (size_t)(i + 1) * kSlots, b, u);
+                }
             }
+            if (split == 1) {
+                sA += t.x;
+                sQ += t.y;
+                continue;
+            }
+            // one group per workgroup: all wavefronts come here as often
+            part[wave * kWave + lane] = t;
+            __syncthreads();
+            if (wave == 0)
+                for (int w = 0; w < split; ++w) {
+                    const double2 v = part[w * kWave + lane];
+                    sA += v.x;
+                    sQ += v.y;
+                }
+            __syncthreads();
         }
+        if (split > 1 && wave > 0) break;
         sA = row_sum(sA);
         sQ = row_sum(sQ);
-        if (split > 1) {   // one group per workgroup: all wavefronts arrive here once
-            if (u == 0) {
-                red[0][4 * wave + f] = sA;
-                red[1][4 * wave + f] = sQ;
-            }
-            __syncthreads();
-            if (wave > 0) break;
-            for (int w = 1; w < split; ++w) {
-                sA += red[0][4 * w + f];
-                sQ += red[1][4 * w + f];
-            }
-        }
         if (live && u == 0) norm[(size_t)p * S + s] = ring_norm(sA, sQ, R);
     }
 }
@@ -501,12 +514,10 @@ __global__ __launch_bounds__(1024) void k_ref_spectra(const float *__restrict__ 
     __syncthreads();
     const int i = 2 * (4 * wave + f);
     const bool live = i < R;
-    double sA = 0.0, sQ = 0.0;
     float2 a[8], b[8];
     const float c = (float)(D / 2);
-    ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, live ? i : 0, R, c, c, u, xb, tw, sA, sQ, a, b);
-    sA = row_sum(sA);
-    sQ = row_sum(sQ);
+    const double2 t = ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, live ? i : 0, R, c, c, u, xb, tw, a, b);
+    const double sA = row_sum(t.x), sQ = row_sum(t.y);
     if (u == 0) {
         red[0][4 * wave + f] = live ? sA : 0.0;
         red[1][4 * wave + f] = live ? sQ : 0.0;
@@ -1172,7 +1183,9 @@ __global__ __launch_bounds__(1024, 4) void k_polar_single(
         };
         for (int i = 0; i < R; i += 2) {
             float2 a[8], b[8];
-            ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, i, R, cx, cy, u, xb, tw, sA, sQ, a, b);
+            const double2 t = ring_pair(img + W + 1, (float)W, (float)(D - 1), W, tmpl, i, R, cx, cy, u, xb, tw, a, b);
+            sA += t.x;
+            sQ += t.y;
             contract(a, i);
             if (i + 1 < R) contract(b, i + 1);
         }
@@ -2553,7 +2566,7 @@ static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_r
 hipError_t prepare_launches() {
     static bool lds_raised = false;
     if (!lds_raised) {
-        const int lds = (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float));
+        const int lds = (int)(polar_lds_floats(kMaxImgDim, 16, 16) * sizeof(float));
         hipError_t e = hipFuncSetAttribute((const void *)k_ref_spectra, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float)));
         if (e != hipSuccess) return e;
@@ -2586,7 +2599,7 @@ hipError_t launch_polar_spectra(const float *imgs, int n_img, int img_dim, Shift
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
     if (hipError_t e = prepare_launches()) return e;
     const PolarShape ps = polar_shape(n_img, n_shift, img_dim, n_ring);
-    const size_t lds = polar_lds_floats(img_dim, ps.waves) * sizeof(float);
+    const size_t lds = polar_lds_floats(img_dim, ps.waves, ps.split) * sizeof(float);
     hipLaunchKernelGGL(k_polar_spectra<false>, dim3(n_img, ps.groups_y), dim3(64 * ps.waves), lds, st, imgs,
                        img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, nullptr, ps.split);
     return hipGetLastError();
