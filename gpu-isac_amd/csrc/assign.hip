@@ -10,9 +10,12 @@
 // assignment, and particle-proposing deferred acceptance finds it in parallel:
 // every free particle proposes to its best class not yet tried; every class
 // keeps its cap best proposers (score descending, particle ascending) and
-// releases the rest; repeat until no free particle has a class left.  The order of
-// the proposals does not change the result, so a few rounds over all particles place
-// most of them and one workgroup then follows the chains of the last (k_chains).
+// releases the rest; repeat until no free particle has a class left.  The last of a full
+// class's holders only ever gets better, so a class whose last holder is before a particle
+// refuses it for good, and the particle passes it over.  Without those proposals a particle
+// that no class takes ends at once instead of trying every class: scores of 20000 x 100 need
+// 9 rounds instead of 95 (0.36 ms), 890 x 149, 145 left over, 4 instead of 170 (0.17 ms; 4.1
+// when one workgroup made the proposals past the eighth round, 2.9 in rounds).
 //
 // Output (n_img + 1 ints): class k's particles (ascending) at [k*cap, (k+1)*cap),
 // then the r = n_img - n_ref*cap particles no class took (ascending), then one
@@ -34,9 +37,10 @@ namespace {
 constexpr int kWave = 64;
 constexpr int kSortN = 4096;          // LDS sort capacity of one class step
 constexpr int kMaxCap = 2048;         // largest class size supported
-constexpr int kChainFree = 1024;      // most free particles k_chains starts from
-constexpr int kChainSteps = 4096;     // most proposals of one of its wavefronts
-constexpr int kRounds = 8;            // rounds before k_chains (4: 0.1 ms slower, 20000 x 100)
+// Rounds queued before a read-back.  Scores of classes that resemble each other need 4 to
+// 10; an empty round costs 8 us, a read-back 25.  5 / 10 / 16 rounds: 20000 x 100 407 / 362 /
+// 412 us, 930 x 120 256 / 178 / 209, 890 x 149 156 / 171 / 206.
+constexpr int kRounds = 10;
 
 __device__ __forceinline__ float score(const float *d, int pitch, int n, int p) {
     const float v = d[(size_t)n * pitch + p];
@@ -48,21 +52,32 @@ __device__ __forceinline__ bool before(float v1, int a1, float v2, int a2) {
     return v1 > v2 || (v1 == v2 && a1 < a2);
 }
 
+// The last holder of a full class, or what everything is before.
+struct __align__(8) Last {
+    float v;
+    int p;
+};
+
 // The wavefront's best class for particle p strictly after (lv, ln) in the order (value
-// desc, class asc), or (.., INT_MAX) if every class has been tried; in all lanes.
-__device__ __forceinline__ void next_class(const float *d, int pitch, int N, int p, int ln, float lv, int lane,
-                                           float &bv, int &bn) {
+// desc, class asc) among those that would take it, or (.., INT_MAX) if there is none; in
+// all lanes.
+__device__ __forceinline__ void next_class(const float *d, int pitch, int N, int p, int ln, float lv,
+                                           const Last *last, int lane, float &bv, int &bn) {
     bv = -INFINITY;
     bn = INT_MAX;
     for (int n0 = lane; n0 < N; n0 += 4 * kWave) {   // four loads in flight
         float v[4];
+        Last l[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = score(d, pitch, min(n0 + r * kWave, N - 1), p);
+        for (int r = 0; r < 4; ++r) {
+            v[r] = score(d, pitch, min(n0 + r * kWave, N - 1), p);
+            l[r] = last[min(n0 + r * kWave, N - 1)];
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int n = n0 + r * kWave;
             const bool after = n < N && (ln < 0 || before(lv, ln, v[r], n));   // strictly after the last try
-            if (after && (bn == INT_MAX || before(v[r], n, bv, bn))) {
+            if (after && before(v[r], p, l[r].v, l[r].p) && (bn == INT_MAX || before(v[r], n, bv, bn))) {
                 bv = v[r];
                 bn = n;
             }
@@ -79,24 +94,26 @@ __device__ __forceinline__ void next_class(const float *d, int pitch, int N, int
     }
 }
 
-// One wavefront per particle: a free particle proposes to its best class after
-// the last one it tried.
+// One wavefront per particle: a free particle proposes to its best class after the last
+// one it tried.  *made = round if any particle does.
 __global__ __launch_bounds__(256) void k_propose(const float *__restrict__ d, int pitch, int N,
                                                  int P, int *__restrict__ status,
                                                  int *__restrict__ last_n, float *__restrict__ last_v,
-                                                 int *__restrict__ cnt, int *__restrict__ props) {
+                                                 const Last *__restrict__ last, int *__restrict__ cnt,
+                                                 int *__restrict__ props, int round, int *__restrict__ made) {
     const int lane = threadIdx.x & 63;
     const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (p >= P) return;
     if (status[p] != 0) return;   // held or exhausted (uniform over the wavefront)
     float bv;
     int bn;
-    next_class(d, pitch, N, p, last_n[p], last_v[p], lane, bv, bn);
+    next_class(d, pitch, N, p, last_n[p], last_v[p], last, lane, bv, bn);
     if (lane != 0) return;
     if (bn == INT_MAX) {
-        status[p] = 2;   // every class has been tried
+        status[p] = 2;   // no class takes it
         return;
     }
+    *made = round;
     last_n[p] = bn;
     last_v[p] = bv;
     status[p] = 1;
@@ -141,8 +158,8 @@ __device__ void lds_sort(float *v, int *a, int n, int tid, int nthreads) {
 __global__ __launch_bounds__(256) void k_accept(const float *__restrict__ d, int pitch, int P,
                                                 int cap, int *__restrict__ cnt,
                                                 const int *__restrict__ props,
-                                                int *__restrict__ holders, float *__restrict__ hold_v,
-                                                int *__restrict__ hold_cnt, int *__restrict__ status) {
+                                                int *__restrict__ holders, int *__restrict__ hold_cnt,
+                                                Last *__restrict__ last, int *__restrict__ status) {
     __shared__ float sv[kSortN];
     __shared__ int sa[kSortN];
     const int c = blockIdx.x, tid = threadIdx.x;
@@ -172,126 +189,12 @@ __global__ __launch_bounds__(256) void k_accept(const float *__restrict__ d, int
         h = min(cap, h + (q1 - q0));
         __syncthreads();
     }
-    for (int i = tid; i < h; i += 256) {
-        holders[(size_t)c * cap + i] = sa[i];
-        hold_v[(size_t)c * cap + i] = sv[i];
-    }
+    for (int i = tid; i < h; i += 256) holders[(size_t)c * cap + i] = sa[i];
     if (tid == 0) {
         hold_cnt[c] = h;
         cnt[c] = 0;
+        if (h == cap) last[c] = Last{sv[cap - 1], sa[cap - 1]};
     }
-}
-
-// The last rounds, one workgroup: each wavefront takes a free particle, proposes for it,
-// goes on with the particle that its class releases, and so on until one finds room, then
-// takes the next free one.  A class is locked while its holders change; a wavefront holds
-// one lock at a time and never waits with it, so every wait ends.  More than kChainFree
-// free particles: nothing is done.  A wavefront that has made kChainSteps proposals frees
-// its particle and ends.  left[0] = 1 if free particles may be left.
-// A round of the two kernels above costs 19 us however few propose, and there are as many
-// as the longest chain has proposals: of 20000 particles and 100 classes 112 rounds, the last
-// 95 with 2300 proposals in all.  Here those take 0.53 ms, 2 us of latency a proposal and 16
-// proposals at once; as rounds, with a read-back every eighth, the whole took 3.4 ms, now 0.77.
-__global__ __launch_bounds__(1024) void k_chains(const float *__restrict__ d, int pitch, int N, int P, int cap,
-                                                 int *__restrict__ last_n, float *__restrict__ last_v,
-                                                 int *holders, float *hold_v, int *hold_cnt, int *status, int *left) {
-    __shared__ int list[kChainFree], lock[1024];
-    __shared__ int n_free, head, more;
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (tid == 0) n_free = head = more = 0;
-    lock[tid] = 0;
-    __syncthreads();
-    for (int p = tid; p < P; p += 1024)
-        if (status[p] == 0) {
-            const int i = atomicAdd(&n_free, 1);
-            if (i < kChainFree) list[i] = p;
-        }
-    __syncthreads();
-    const int nf = n_free;
-    if (nf > kChainFree) {   // uniform
-        if (tid == 0) left[0] = 1;
-        return;
-    }
-    int steps = 0;
-    while (steps < kChainSteps) {
-        int q = 0;
-        if (lane == 0) q = atomicAdd(&head, 1);
-        q = __shfl(q, 0, kWave);
-        if (q >= nf) break;
-        int p = list[q];
-        for (; p >= 0 && steps < kChainSteps; ++steps) {   // p is free and this wavefront's own
-            float bv;
-            int bn;
-            next_class(d, pitch, N, p, last_n[p], last_v[p], lane, bv, bn);
-            if (bn == INT_MAX) {
-                if (lane == 0) status[p] = 2;
-                p = -1;
-                break;
-            }
-            if (lane == 0) {
-                last_n[p] = bn;
-                last_v[p] = bv;
-                while (atomicCAS(&lock[bn & 1023], 0, 1) != 0) __builtin_amdgcn_s_sleep(1);
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            int *hp = holders + (size_t)bn * cap;
-            float *hv = hold_v + (size_t)bn * cap;
-            const int h = hold_cnt[bn];
-            int slot = h, out = -1;   // a free place, nobody released
-            if (h >= cap) {           // the last of the holders in the class's order
-                float wv = INFINITY;
-                int wp = -1, ws = 0;
-                for (int i0 = lane; i0 < cap; i0 += 4 * kWave) {
-                    float v[4];
-                    int a[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int i = min(i0 + r * kWave, cap - 1);   // a repeated entry changes nothing
-                        v[r] = hv[i];
-                        a[r] = hp[i];
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (wp < 0 || before(wv, wp, v[r], a[r])) {
-                            wv = v[r];
-                            wp = a[r];
-                            ws = min(i0 + r * kWave, cap - 1);
-                        }
-                }
-#pragma unroll
-                for (int off = 32; off >= 1; off >>= 1) {
-                    const float ov = __shfl_xor(wv, off, kWave);
-                    const int op = __shfl_xor(wp, off, kWave), os = __shfl_xor(ws, off, kWave);
-                    if (op >= 0 && (wp < 0 || before(wv, wp, ov, op))) {
-                        wv = ov;
-                        wp = op;
-                        ws = os;
-                    }
-                }
-                const bool in = before(bv, p, wv, wp);
-                slot = in ? ws : -1;
-                out = in ? wp : p;
-            }
-            if (lane == 0 && slot >= 0) {
-                hp[slot] = p;
-                hv[slot] = bv;
-                status[p] = 1;
-                if (out >= 0)
-                    status[out] = 0;
-                else
-                    hold_cnt[bn] = h + 1;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __builtin_amdgcn_wave_barrier();
-            if (lane == 0) atomicExch(&lock[bn & 1023], 0);
-            p = out;
-        }
-        if (p >= 0 && lane == 0) more = 1;   // out of steps
-    }
-    if (lane == 0 && steps >= kChainSteps) more = 1;
-    __syncthreads();
-    if (tid == 0) left[0] = more;
 }
 
 // Output, part 1: block c writes class c's holders ascending at out[c*cap ...].
@@ -378,7 +281,7 @@ __global__ __launch_bounds__(1024) void k_assign_output(const float *__restrict_
 }
 
 __global__ void k_assign_init(int *status, int *last_n, float *last_v, int P, int *hold_cnt,
-                              int *cnt, int N) {
+                              Last *last, int *cnt, int N, int *made) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < P) {
         status[i] = 0;
@@ -387,8 +290,10 @@ __global__ void k_assign_init(int *status, int *last_n, float *last_v, int P, in
     }
     if (i < N) {
         hold_cnt[i] = 0;
+        last[i] = Last{-INFINITY, INT_MAX};
         cnt[i] = 0;
     }
+    if (i == 0) *made = 0;
 }
 
 // One device allocation cut into arrays (256-byte aligned).
@@ -434,7 +339,7 @@ int assign_groups(const float *d_d, int N, int P, int pitch, int *d_out, hipStre
     const int cap = P / N;
     if (cap > kMaxCap)
         return err(4, "assign_groups: classes of more than 2048 particles are not supported");
-    Buf status, last_n, last_v, cnt, props, holders, hold_v, hold_cnt, left;
+    Buf status, last_n, last_v, cnt, props, holders, hold_cnt, last, made;
     Arena arena;
     arena.add(status, (size_t)P * 4);
     arena.add(last_n, (size_t)P * 4);
@@ -443,32 +348,32 @@ int assign_groups(const float *d_d, int N, int P, int pitch, int *d_out, hipStre
     arena.add(props, (size_t)N * P * 4);
     arena.add(holders, (size_t)N * cap * 4);
     arena.add(hold_cnt, (size_t)N * 4);
-    arena.add(hold_v, (size_t)N * cap * 4);
-    arena.add(left, 4);
+    arena.add(last, (size_t)N * sizeof(Last));
+    arena.add(made, 4);
     if (arena.allocate() != hipSuccess) return err(1, "assign_groups: device allocation failed");
     const int mx = P > N ? P : N;
     hipLaunchKernelGGL(k_assign_init, dim3((mx + 255) / 256), dim3(256), 0, st, status.as<int>(),
-                       last_n.as<int>(), last_v.as<float>(), P, hold_cnt.as<int>(), cnt.as<int>(), N);
-    // every pass makes at least one proposal until no particle is free; a particle
-    // proposes to each class at most once, so N * P + 1 passes bound the loop.
-    const long long max_passes = (long long)N * P + 1;
-    for (long long pass = 0; pass < max_passes; ++pass) {
+                       last_n.as<int>(), last_v.as<float>(), P, hold_cnt.as<int>(), last.as<Last>(), cnt.as<int>(), N,
+                       made.as<int>());
+    // every round makes at least one proposal until no particle is free (a round without one
+    // changes nothing); a particle proposes to each class at most once, so N * P + 1 rounds
+    // bound the loop.
+    const long long max_rounds = (long long)N * P + 1;
+    for (long long first = 0; first < max_rounds; first += kRounds) {
+        int round = (int)first, proposed = 0;
         for (int r = 0; r < kRounds; ++r) {
+            ++round;
             hipLaunchKernelGGL(k_propose, dim3((P + 3) / 4), dim3(256), 0, st, d_d, pitch, N, P,
-                               status.as<int>(), last_n.as<int>(), last_v.as<float>(),
-                               cnt.as<int>(), props.as<int>());
+                               status.as<int>(), last_n.as<int>(), last_v.as<float>(), last.as<Last>(),
+                               cnt.as<int>(), props.as<int>(), round, made.as<int>());
             hipLaunchKernelGGL(k_accept, dim3(N), dim3(256), 0, st, d_d, pitch, P, cap,
-                               cnt.as<int>(), props.as<int>(), holders.as<int>(), hold_v.as<float>(),
-                               hold_cnt.as<int>(), status.as<int>());
+                               cnt.as<int>(), props.as<int>(), holders.as<int>(), hold_cnt.as<int>(),
+                               last.as<Last>(), status.as<int>());
         }
-        hipLaunchKernelGGL(k_chains, dim3(1), dim3(1024), 0, st, d_d, pitch, N, P, cap, last_n.as<int>(),
-                           last_v.as<float>(), holders.as<int>(), hold_v.as<float>(), hold_cnt.as<int>(),
-                           status.as<int>(), left.as<int>());
-        int more = 0;
-        if (hipMemcpyAsync(&more, left.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        if (hipMemcpyAsync(&proposed, made.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
             hipStreamSynchronize(st) != hipSuccess)
             return err(1, "assign_groups: proposal round failed");
-        if (more == 0) break;
+        if (proposed != round) break;   // none in the last one
     }
     hipLaunchKernelGGL(k_class_out, dim3(N), dim3(256), 0, st, cap, holders.as<int>(),
                        hold_cnt.as<int>(), d_out);
