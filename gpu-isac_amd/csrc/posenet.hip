@@ -579,7 +579,6 @@ __device__ __forceinline__ float16_t mfma32_bf16(uint4 a, uint4 b, float16_t c) 
 
 constexpr int kResidentLdsMax = 63 * 1024;   // dynamic band; with the static bias copy <= 64 KB
 constexpr int kResidentCoutMax = 128;
-constexpr int kConvBandMax = 31 * 1024;      // band of k_conv_resident<32> and <64>: see their launch
 
 // First maximum (in lane order) of the four lanes of a quad, valid in lane 4k:
 // the pairs (4k, 4k+1) and (4k+2, 4k+3) keep their first maximum, then the pair
@@ -1290,6 +1289,28 @@ unsigned blocks_for(size_t count, int threads) { return (unsigned)((count + thre
 
 using namespace isac;
 
+// Most output rows of a band of k_conv_resident, row_bytes of LDS a row (0: it cannot run).
+// Small bands let more workgroups share a CU, one staging while others compute, but each
+// stages two rows more than it computes.  At 128 input channels the weights' registers
+// leave two workgroups, and the largest band is the best one (9 x 9, 128 -> 32: 19 us, 27
+// with 31 KB).  Else, batches of 370 k pixels, us with bands of 31 / 39 / 52 / 63 KB:
+//   38 x 38, 32 -> 64     44 /  40 /  42 /  65     a few rows or more: 31 KB
+//   126 x 126, 32 -> 64   38 /  39 /  46 /  54     one row of 32 channels: 31 KB
+//   64 x 64, 64 -> 16     46 /  36 /  39 /  38     one of 64: the smallest with two
+//   72 x 72, 64 -> 16    (123)/ (123)/  - /  43    none (k_conv_mfma): the smallest with any
+//   14 x 14, 64 -> 64    125 /  95 /  95 /  95     whole images of up to 52 KB are not cut
+//   19 x 19, 32 -> 64     58 /  64 /  43 /  43
+//   24 x 24, 32 -> 64     42 /  50 /  68 /  56     (whole: 55 KB)
+static int conv_band_rows(int Cin, int H, int row_bytes) {
+    auto rows = [&](int kb) { return kb * 1024 / row_bytes - 2; };
+    if (Cin != 128) {
+        if (H <= rows(52)) return H;
+        for (const int kb : {31, 39, 52})
+            if (rows(kb) >= Cin / 32) return rows(kb);
+    }
+    return kResidentLdsMax / row_bytes - 2;
+}
+
 extern "C" {
 
 int isac_nn_standardize(const float *img, int n, int D, uint16_t *x0, void *stream) {
@@ -1325,11 +1346,7 @@ int isac_nn_conv_fwd(const uint16_t *x, int n, int H, int W, int Cin, const uint
         // 16 pixels, plus half a round per band for its staging
         const int Cs = Cin + 8, Wl = W + 2;
         const int RS = Wl * Cs + ((64 - Wl * Cs % 128) + 128) % 128;
-        // Bands of 31 KB let four workgroups share a CU, one staging while others compute:
-        // 47 us against 68 with 63 KB (38 x 38, 32 -> 64, batch 256), 54 against 75 (19 x 19,
-        // 64 -> 128).  At 128 input channels the weights' registers leave two, and the
-        // larger band is the better one (9 x 9, 128 -> 32: 19 against 27)
-        const int rmax = (Cin == 128 ? kResidentLdsMax : kConvBandMax) / (RS * 2) - 2;
+        const int rmax = conv_band_rows(Cin, H, RS * 2);
         if (rmax >= 1) {
             const int wpc = 4 / (std::min(Cout, 64) / 16);
             int TH = 1;
