@@ -21,6 +21,7 @@
 #include <cmath>
 #include <climits>
 #include <cstdio>
+#include <type_traits>
 
 namespace isac {
 namespace {
@@ -678,11 +679,10 @@ __global__ __launch_bounds__(256, CIN == 32 ? 4 : 2) void k_conv_pool_resident(
 // the fully unrolled k-steps on v_mfma_f32_16x16x16_bf16, in the order of
 // k_conv_mfma: the output is bit-identical to it.
 // What bounds it: a chain of NK dependent products and the LDS reads that feed them, so a
-// wavefront takes kResChains blocks at a time (four are no better), and the staging
+// wavefront takes two blocks at a time (four are no better), one where none is left for the
+// second (9 x 9, 128 -> 32: 124 us, 132 with a second chain of nothing), and the staging
 // between items.  Batch 256, 19 x 19, 64 -> 128: 54 us, 250 TFLOP/s (k_conv_mfma 106);
 // 38 x 38, 32 -> 64: 47 (71).
-constexpr int kResChains = 2;
-
 template <int CIN>
 __global__ __launch_bounds__(256, 2) void k_conv_resident(
     const unsigned short *__restrict__ x, int H, int W, const unsigned short *__restrict__ w,
@@ -719,12 +719,14 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
         __syncthreads();
         const int npx = (r1 - r0) * W, nblk = (npx + 15) / 16;
         const size_t px0 = ((size_t)img * H + r0) * W;
-        for (int b = wi; b < nblk; b += kResChains * wpc) {
-            const unsigned short *pb[kResChains];
-            int px[kResChains];
-            float4_t acc[kResChains];
+        // CH blocks from b on, wpc apart
+        auto blocks = [&](auto chains, int b) __attribute__((always_inline)) {
+            constexpr int CH = decltype(chains)::value;
+            const unsigned short *pb[CH];
+            int px[CH];
+            float4_t acc[CH];
 #pragma unroll
-            for (int j = 0; j < kResChains; ++j) {
+            for (int j = 0; j < CH; ++j) {
                 px[j] = 16 * (b + j * wpc) + li;
                 const int pc = px[j] < npx ? px[j] : 0;
                 const int pr = pc / W, pcl = pc - pr * W;
@@ -736,7 +738,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
             for (int s = 0; s < NK; ++s) {
                 const int t = s / CPT, c = (s % CPT) * 16;
 #pragma unroll
-                for (int j = 0; j < kResChains; ++j) {
+                for (int j = 0; j < CH; ++j) {
                     const uint2 bv = *reinterpret_cast<const uint2 *>(pb[j] + (t / 3) * RS + (t % 3) * Cs + c);
                     acc[j] = mfma_bf16(wa[s], bv, acc[j]);
                 }
@@ -744,7 +746,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
             const int co = co0 + lk;
             const float4 bb = *reinterpret_cast<const float4 *>(sbias + co);
 #pragma unroll
-            for (int j = 0; j < kResChains; ++j) {
+            for (int j = 0; j < CH; ++j) {
                 float o[4] = {acc[j][0] + bb.x, acc[j][1] + bb.y, acc[j][2] + bb.z, acc[j][3] + bb.w};
                 if (relu) {
 #pragma unroll
@@ -753,7 +755,10 @@ __global__ __launch_bounds__(256, 2) void k_conv_resident(
                 if (px[j] < npx)
                     *reinterpret_cast<uint2 *>(y + (px0 + px[j]) * Cout + cy + co) = pack4(o[0], o[1], o[2], o[3]);
             }
-        }
+        };
+        int b = wi;
+        for (; b + wpc < nblk; b += 2 * wpc) blocks(std::integral_constant<int, 2>{}, b);
+        if (b < nblk) blocks(std::integral_constant<int, 1>{}, b);
     }
 }
 
