@@ -338,8 +338,10 @@ __global__ __launch_bounds__(256) void k_conv_mfma(const unsigned short *__restr
 // other.  Here a wavefront owns 16 rows x 16 output channels and keeps the loads of
 // kDenseAhead k-steps in flight.  The chain over the k-steps is the same, so the outputs
 // are bit-identical.
-// What bounds it: the latency of Cin / (16 kDenseAhead) rounds of loads.  256
-// rows, 2592 -> 384: 29 us (k_conv_mfma 103), 384 -> 304: 10 (25), 304 -> 384: 7 (19).
+// What bounds it: the latency of Cin / (16 kDenseAhead) rounds of loads,
+// and with few of them the loads themselves: none is made past the end (4096 rows, 64 ->
+// 128: 4.4 us; 18 with the last k-step loaded again, k_conv_mfma 9.7).  256 rows, 2592 ->
+// 384: 27 us (k_conv_mfma 103), 384 -> 384: 8 (27).
 constexpr int kDenseAhead = 12;
 constexpr size_t kDenseTiles = 32;
 
@@ -361,9 +363,9 @@ __global__ __launch_bounds__(256) void k_dense(const unsigned short *__restrict_
     auto load = [&](int ks, uint2 (&a)[kDenseAhead], uint2 (&b)[kDenseAhead]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kDenseAhead; ++j) {
-            const int k = min(ks + j, NK - 1);   // past the end: loaded, not used
-            a[j] = *reinterpret_cast<const uint2 *>(wr + 16 * k);
-            b[j] = *reinterpret_cast<const uint2 *>(xr + 16 * k);
+            if (ks + j >= NK) break;   // uniform
+            a[j] = *reinterpret_cast<const uint2 *>(wr + 16 * (ks + j));
+            b[j] = *reinterpret_cast<const uint2 *>(xr + 16 * (ks + j));
         }
     };
     auto mma = [&](int ks, const uint2 (&a)[kDenseAhead], const uint2 (&b)[kDenseAhead])
@@ -1399,7 +1401,7 @@ int isac_nn_conv_fwd(const uint16_t *x, int n, int H, int W, int Cin, const uint
     dim3 grid(blocks_for(np, 256), (unsigned)((Cout + 63) / 64));
     // few rows: k_conv_mfma would have at most kDenseTiles workgroups.  Its time hardly
     // changes up to 256 of them, k_dense's grows by its 16-row tiles' repeated loads: 24
-    // workgroups 57 us against 103 (2592 -> 384) and 18 against 25 (384 -> 304), 41
+    // workgroups 51 us against 103 (2592 -> 384) and 13 against 27 (384 -> 384), 41
     // workgroups 26 against 27 (384 -> 2592), 96 workgroups 166 against 114
     if (ks == 1 && (size_t)grid.x * grid.y <= kDenseTiles) {
         const dim3 dg(blocks_for(np, 64), (unsigned)(Cout / 16));
