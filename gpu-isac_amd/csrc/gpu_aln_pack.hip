@@ -292,6 +292,7 @@ int batch_for(size_t per_item, size_t fixed_bytes, float mem_frac, int total) {
     size_t budget = std::min(have > fixed_bytes ? have - fixed_bytes : 0, cap);
     size_t b = per_item ? budget / per_item : (size_t)total;
     b = std::max<size_t>(b, 1);
+    b = std::min<size_t>(b, isac::kGridItems / 1024);   // the kernels take up to 1024 work-items a particle
     return (int)std::min<size_t>(b, (size_t)total);
 }
 

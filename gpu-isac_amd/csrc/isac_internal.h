@@ -20,6 +20,9 @@ constexpr int kSlots = 128;     // packed spectrum slots per ring: slot 0 = (X[0
 constexpr int kPartOff = 4;
 __host__ __device__ constexpr int slot_re(int k) { return (k >> 6) * 128 + (k & 15) * 8 + ((k >> 4) & 3); }
 constexpr int kMaxImgDim = 128; // image staged whole in LDS by the polar kernel
+// Work-items that a launch can have in its grid's first dimension; past them HIP refuses it
+// or runs the count modulo 2^32.
+constexpr long long kGridItems = (1ll << 32) - 1;
 constexpr int kMaxRings = 127;  // rings must fit inside a 256-sample ring FFT budget
 
 // Same memory layout as the reference's AlignParam (cuda/gpu_aln_common.h:78-85).

@@ -2682,13 +2682,21 @@ hipError_t launch_ccf_mref(const float2 *spec, const float2 *norm, const float2 
                            const float *rsum0, int n_img, int n_shift, int n_ring, int n_ref,
                            const float2 *twiddle, PeakRec *rec, hipStream_t st) {
     if (n_img <= 0 || n_ref <= 0) return hipSuccess;
-    const MrefJob j = mref_job(spec, norm, rspec, rsum0, rec, n_img, n_shift, n_ring, n_ref);
     const int cp = particles_per_workgroup(n_img, n_shift, n_ref);
-    const long long blocks = (long long)((n_img + cp - 1) / cp) * ((n_ref + kMrefRefs - 1) / kMrefRefs);
-    const dim3 grid((unsigned)blocks), wg(kMrefWaves * 64);
-    if (n_ring >= kMrefKeep) hipLaunchKernelGGL(k_ccf_mref<kMrefKeep>, grid, wg, 0, st, j, cp, twiddle);
-    else hipLaunchKernelGGL(k_ccf_mref<0>, grid, wg, 0, st, j, cp, twiddle);
-    return hipGetLastError();
+    const long long ng = (n_ref + kMrefRefs - 1) / kMrefRefs;
+    const dim3 wg(kMrefWaves * 64);
+    const long long step = std::max(1ll, kGridItems / wg.x / ng) * cp;
+    for (long long p = 0; p < n_img; p += step) {
+        const int n = (int)std::min(step, n_img - p);
+        const size_t row = (size_t)p * n_shift;
+        const MrefJob j = mref_job(spec + row * n_ring * kSlots, norm + row, rspec, rsum0, rec + (size_t)p * n_ref, n,
+                                   n_shift, n_ring, n_ref);
+        const dim3 grid((unsigned)((n + cp - 1) / cp * ng));
+        if (n_ring >= kMrefKeep) hipLaunchKernelGGL(k_ccf_mref<kMrefKeep>, grid, wg, 0, st, j, cp, twiddle);
+        else hipLaunchKernelGGL(k_ccf_mref<0>, grid, wg, 0, st, j, cp, twiddle);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 MrefJob mref_job(const float2 *spec, const float2 *norm, const float2 *rspec, const float *rsum0,
@@ -2744,10 +2752,17 @@ hipError_t launch_polar_single(const float *imgs, int n_img, int img_dim, ShiftV
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
     if (hipError_t e = prepare_launches()) return e;
     const int nw = polar_waves(n_shift, img_dim);
-    hipLaunchKernelGGL(k_polar_single, dim3(n_img), dim3(64 * nw), polar_lds_floats(img_dim, nw) * sizeof(float), st,
-                       imgs, img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, rspec, rsum0, ref_of,
-                       ref_stride, n_ref, rec);
-    return hipGetLastError();
+    const size_t lds = polar_lds_floats(img_dim, nw) * sizeof(float);
+    const long long step = kGridItems / (64 * nw);
+    for (long long p = 0; p < n_img; p += step) {
+        const ShiftView a{acc.base + (size_t)p * acc.stride, acc.stride};
+        const dim3 grid((unsigned)std::min(step, n_img - p));
+        hipLaunchKernelGGL(k_polar_single, grid, dim3(64 * nw), lds, st, imgs + (size_t)p * img_dim * img_dim, img_dim,
+                           a, shift_i, n_shift, tmpl, n_ring, twiddle, rspec, rsum0, ref_of + (size_t)p * ref_stride,
+                           ref_stride, n_ref, rec + p);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 // One pass does a group of four shifts in one wavefront; two passes split the rings of few
