@@ -1135,9 +1135,11 @@ int alloc_params(size_t n, int ref_id) {
 }
 
 // Host image list checks and the pinned staging buffer of the host-pointer entries: two
-// halves of at most kStageHalf bytes (or one image).  The host gathers images into one
-// while the copy engine moves the other; pinning a buffer for all 3000 images of 76 x 76 cost
-// more (4 ms) than their copy (1.5 ms).
+// halves of at most kStageHalf bytes and half the images (or one image).  The host gathers
+// images into one while the copy engine moves the other.  New pinned pages cost 0.38 ms a
+// MB at their first touch: pinning all 3000 images of 76 x 76 took more (4 ms) than their
+// copy (1.5), and two halves of 8 MB for 225 images of 96 x 96 (8 MB) 2.6 ms a call, now
+// 0.9.
 constexpr size_t kStageHalf = (size_t)8 << 20;
 int check_image_list(const float **imgs, unsigned n) {
     if (n == 0) return 0;
@@ -1155,7 +1157,7 @@ int check_image_list(const float **imgs, unsigned n) {
 
 // Halves for images of img_bytes each, at most n of them.
 int reserve_stage(size_t img_bytes, size_t n) {
-    const size_t half = std::max<size_t>(1, std::min(n, kStageHalf / img_bytes)) * img_bytes;
+    const size_t half = std::max<size_t>(1, std::min((n + 1) / 2, kStageHalf / img_bytes)) * img_bytes;
     for (hipEvent_t &e : g.stage_free)
         if (!e) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (g.h_stage_half < half) {

@@ -26,6 +26,8 @@ def _images(kind, n, D, seed):
     (1500, 2, 40, 17, 1.0),   # whole: not split, quarters: 3
     (300, 3, 100, 47, 1.0),   # whole: 4, quarters: 16, three batches of the static scratch: 9
     (90, 2, 128, 61, 4.0),    # whole: 2, quarters: 8, batches of 12 and 6: 16
+    (3, 1, 32, 4, 0.0),       # one image a quarter, a reference alone
+    (229, 5, 32, 3, 1.0),     # odd counts through the halves of the host's staging
 ])
 def test_entries_give_the_same_bits(gpu, P, N, D, R, rng, kind):
     import torch
