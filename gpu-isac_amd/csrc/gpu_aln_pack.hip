@@ -528,6 +528,9 @@ int run_proposal(const float *d_sbj, const float *d_ref, ShiftView acc, int P, i
     HIP_OK(ws.fb_idx.reserve((size_t)P * sizeof(int)));
     HIP_OK(ws.fb_count.reserve(sizeof(int)));
     unsigned n_l2 = 0;
+    // shifts that K windows cover, if they fall anywhere
+    const double window = std::min(1.0, (double)(std::min(nx, 2 * hw + 1) * std::min(ny, 2 * hw + 1)) / S);
+    const int n_window = std::max(1, (int)std::lround(S * (1.0 - std::pow(1.0 - window, K))));
     // level 1
     for (int p0 = 0; p0 < P; p0 += pb) {
         const int n = std::min(pb, P - p0);
@@ -540,7 +543,7 @@ int run_proposal(const float *d_sbj, const float *d_ref, ShiftView acc, int P, i
                                                  ws.shifts_i.as<int2>(), S, ws.tmpl.as<float2>(), R,
                                                  ws.twiddle.as<float2>(), ws.spec.as<float2>(),
                                                  ws.norm.as<float2>(),
-                                                 ws.smask.as<unsigned long long>(), st));
+                                                 ws.smask.as<unsigned long long>(), n_window, st));
         {
             ProfScope ps(g.prof, st);
             HIP_OK(isac::launch_ccf_prop(ws.spec.as<float2>(), ws.norm.as<float2>(),
@@ -572,7 +575,7 @@ int run_proposal(const float *d_sbj, const float *d_ref, ShiftView acc, int P, i
                                                  ws.shifts_i.as<int2>(), S, ws.tmpl.as<float2>(), R,
                                                  ws.twiddle.as<float2>(), ws.spec.as<float2>(),
                                                  ws.norm.as<float2>(),
-                                                 ws.smask2.as<unsigned long long>(), st));
+                                                 ws.smask2.as<unsigned long long>(), S, st));
         HIP_OK(isac::launch_ccf_candidates(ws.spec.as<float2>(), ws.norm.as<float2>(),
                                            ws.rspec.as<float2>(), ws.rsum0.as<float>(),
                                            ws.cand.as<int>(), K, n2, S, R, N, ws.twiddle.as<float2>(),

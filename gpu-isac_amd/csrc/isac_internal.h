@@ -98,12 +98,12 @@ hipError_t launch_ccf_mref_queue(const MrefJob *jobs, const int4 *items, const i
                                  hipStream_t st);
 int mref_queue_blocks_per_cu();   // occupancy of the queue kernel (0 on error)
 
-// Polar spectra of the shifts marked in smask[img] only (n_shift <= 64).
+// Polar spectra of the shifts marked in smask[img] only (n_shift <= 64), about n_rows of them.
 hipError_t launch_polar_spectra_masked(const float *imgs, int n_img, int img_dim, ShiftView acc,
                                        const int2 *shift_i, int n_shift, const float2 *tmpl,
                                        int n_ring, const float2 *twiddle, float2 *spec,
                                        float2 *norm, const unsigned long long *smask,
-                                       hipStream_t st);
+                                       int n_rows, hipStream_t st);
 
 // Narrowed search: prop [n_img][K] int4 (ref, mirror, psi bin, shift) -> items
 // [n_img][K] and shift masks; shift grid nx x ny (x-major), window +-hw shifts.

@@ -340,11 +340,9 @@ __device__ __forceinline__ float2 ring_norm(double a, double q, int R) {
     return f2((float)(mu * kRingLen), (float)(1.0 / (sd + 1e-7)));
 }
 
-// LDS floats of a polar kernel with nw wavefronts: lane twiddles, parts of the sums of ring
-// pairs split over `split` wavefronts, exchange buffers, image.
-__host__ __device__ constexpr int polar_part_floats(int split) { return split > 1 ? split * kWave * 4 : 0; }
-__host__ __device__ constexpr int polar_lds_floats(int D, int nw, int split = 1) {
-    return 2 * kIfftTw + polar_part_floats(split) + nw * 4 * kXchLd + (D + 2) * (D + 2);
+// LDS floats of a polar kernel with nw wavefronts: lane twiddles, exchange buffers, image.
+__host__ __device__ constexpr int polar_lds_floats(int D, int nw) {
+    return 2 * kIfftTw + nw * 4 * kXchLd + (D + 2) * (D + 2);
 }
 
 // Bordered copy of an image (see tap), all threads; the caller synchronises.
@@ -399,22 +397,28 @@ __device__ __forceinline__ void store_slots(float2 *row, const float2 (&a)[8], i
     }
 }
 
-// Raw ring spectra of an image at every grid shift.  Workgroup = one image (staged once
-// in LDS); a wavefront takes four rows (shifts) at a time, one per 16 lanes, and their
-// rings in pairs.  split > 1: the ring pairs of a group of rows go round over `split`
-// wavefronts, and blockIdx.y names the group.  MASKED: only the shifts whose bit is set
-// in smask[p] (S <= 64) are computed; the other rows of spec / norm are left as they were.
+// Raw ring spectra of an image at every grid shift.  Workgroup = one image (staged once in
+// LDS) and `rows` of its rows (shifts) from blockIdx.y * rows on.  MASKED: only the shifts
+// whose bit is set in smask[p] (S <= 64) are computed, all by one workgroup; the other rows
+// of spec / norm are left as they were.
+// Unspread, a wavefront takes four rows at a time, one per 16 lanes, and their ring pairs in
+// turn.  SPREAD, the pairs of all rows go round over the 16-lane groups, and a lane's parts
+// of a row's sums come together in LDS after each round: no lanes without a row and no
+// wavefronts without a group of four, for two barriers a round.
 // What bounds it: vector instructions (about 25 a sample with its FP64 sums, 20 a point
 // of the transform) and the writes; 6000 images of 76 x 76, 49 shifts, 34 rings, 10.2 GB:
 // 3.5 ms, 2.7 without the stores, 2.7 with stores but no transforms.  A transform over 64
 // lanes with an exchange at each stage made it 3.9.  Four wavefronts per SIMD (128
-// registers) are needed to hide the taps.
-template <bool MASKED>
+// registers) are needed to hide the taps.  Unspread / spread: 8000 images of 100 x 100, 1
+// shift 1.93 / 0.39 ms, 5000 of 128 x 128, 9 shifts 3.23 / 1.36, 3000 of 128 x 128, 25 shifts
+// 2.51 / 1.94, 10000 of 76 x 76, 9 shifts 1.55 / 1.36, 25 shifts of 5000 1.61 / 1.69, 49 shifts
+// of 5000 3.05 / 3.28.
+template <bool MASKED, bool SPREAD>
 __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     const float *__restrict__ imgs, int D, ShiftView acc, const int2 *__restrict__ shift_i,
     int S, const float2 *__restrict__ tmpl, int R, const float2 *__restrict__ twg,
     float2 *__restrict__ spec, float2 *__restrict__ norm,
-    const unsigned long long *__restrict__ smask, int split) {
+    const unsigned long long *__restrict__ smask, int rows) {
     extern __shared__ float4 smem4[];
     __shared__ int slist[64];
     __shared__ int scnt;
@@ -423,8 +427,7 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     const int p = blockIdx.x;
     if (MASKED && smask[p] == 0ull) return;   // uniform over the workgroup
     float2 *tw = reinterpret_cast<float2 *>(smem4);
-    double2 *part = reinterpret_cast<double2 *>(tw + kIfftTw);   // [wavefront][lane], where split
-    float *xb0 = reinterpret_cast<float *>(tw + kIfftTw) + polar_part_floats(split);
+    float *xb0 = reinterpret_cast<float *>(tw + kIfftTw);
     float *xb = xb0 + (wave * 4 + f) * kXchLd, *img = xb0 + nw * 4 * kXchLd;
     const int W = D + 2;
     load_bordered(img, imgs + (size_t)p * D * D, D);
@@ -437,7 +440,9 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
         scnt = c;
     }
     __syncthreads();
-    const int n_rows = MASKED ? scnt : S;
+    const int row0 = MASKED ? 0 : blockIdx.y * rows;
+    const int n_rows = MASKED ? scnt : min(rows, S - row0);
+    const int pairs = (R + 1) / 2, slots = 4 * nw;
     float ax = 0.0f, ay = 0.0f;
     if (acc.base) {
         ax = acc.base[(size_t)p * acc.stride];
@@ -445,47 +450,84 @@ __global__ __launch_bounds__(1024, 4) void k_polar_spectra(
     }
     const float *img1 = img + W + 1;
     const float Wf = (float)W, lim = (float)(D - 1);
-    const int q0 = split > 1 ? wave : 0;          // first ring pair of this wavefront
-    const int jw = split > 1 ? blockIdx.y : wave, jn = split > 1 ? gridDim.y : nw;
-    for (int j0 = 4 * jw; j0 < n_rows; j0 += 4 * jn) {
-        const bool live = j0 + f < n_rows;   // lanes past the last row repeat it, without its stores
-        const int j = min(j0 + f, n_rows - 1);
-        const int s = MASKED ? slist[j] : j;
-        const int2 si = shift_i[s];
-        const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
-        double sA = 0.0, sQ = 0.0;
-        float2 *row = spec + ((size_t)p * S + s) * (size_t)R * kSlots;
-        for (int i0 = 0; i0 < R; i0 += 2 * split) {
-            const int i = i0 + 2 * q0;   // uniform over the wavefront
-            double2 t = make_double2(0.0, 0.0);
-            if (i < R) {
+    auto shift_of = [&](int j) { return MASKED ? slist[j] : row0 + j; };
+    if (!SPREAD) {
+        for (int j0 = 4 * wave; j0 < n_rows; j0 += slots) {
+            const bool live = j0 + f < n_rows;   // lanes past the last row repeat it, without its stores
+            const int s = shift_of(min(j0 + f, n_rows - 1));
+            const int2 si = shift_i[s];
+            const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
+            double sA = 0.0, sQ = 0.0;
+            float2 *row = spec + ((size_t)p * S + s) * (size_t)R * kSlots;
+            for (int i = 0; i < R; i += 2) {
                 float2 a[8], b[8];
-                t = ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, a, b);
+                const double2 t = ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, a, b);
+                sA += t.x;
+                sQ += t.y;
                 if (live) {
                     store_slots(row + (size_t)i * kSlots, a, u);
                     if (i + 1 < R) store_slots(row + (size_t)(i + 1) * kSlots, b, u);
                 }
             }
-            if (split == 1) {
-                sA += t.x;
-                sQ += t.y;
-                continue;
-            }
-            // one group per workgroup: all wavefronts come here as often
-            part[wave * kWave + lane] = t;
-            __syncthreads();
-            if (wave == 0)
-                for (int w = 0; w < split; ++w) {
-                    const double2 v = part[w * kWave + lane];
-                    sA += v.x;
-                    sQ += v.y;
-                }
-            __syncthreads();
+            sA = row_sum(sA);
+            sQ = row_sum(sQ);
+            if (live && u == 0) norm[(size_t)p * S + s] = ring_norm(sA, sQ, R);
         }
-        if (split > 1 && wave > 0) break;
-        sA = row_sum(sA);
-        sQ = row_sum(sQ);
-        if (live && u == 0) norm[(size_t)p * S + s] = ring_norm(sA, sQ, R);
+        return;
+    }
+    // task t: ring pair t % pairs of row t / pairs, on slot t % slots
+    const int slot = 4 * wave + f, n_task = n_rows * pairs;
+    double sA = 0.0, sQ = 0.0;   // of the row that this slot adds up: rows slot, slot + slots, ..
+    for (int t0 = 0; t0 < n_task; t0 += slots) {
+        const int t1 = min(t0 + slots, n_task);
+        if (t0 + 4 * wave < t1) {   // uniform over the wavefront
+            const int t = min(t0 + slot, t1 - 1);   // lanes past the last task repeat it, without its stores
+            const bool live = t0 + slot < t1;
+            const int j = t / pairs, i = 2 * (t - j * pairs);
+            const int s = shift_of(j);
+            const int2 si = shift_i[s];
+            const float cx = (float)(D / 2 + si.x) + ax, cy = (float)(D / 2 + si.y) + ay;
+            float2 a[8], b[8];
+            const double2 part = ring_pair(img1, Wf, lim, W, tmpl, i, R, cx, cy, u, xb, tw, a, b);
+            if (live) {
+                float2 *row = spec + (((size_t)p * S + s) * (size_t)R + i) * kSlots;
+                store_slots(row, a, u);
+                if (i + 1 < R) store_slots(row + kSlots, b, u);
+            }
+            wave_lds_sync();
+            reinterpret_cast<double2 *>(xb)[u] = part;   // the exchange buffer is free until the next round
+        }
+        __syncthreads();
+        // the row of this slot that has tasks in this round, if any: they are in ring order
+        const int ja = t0 / pairs, jb = (t1 - 1) / pairs;
+        const int j = ja + (slot + slots - ja % slots) % slots;
+        if (j <= jb) {
+            const int ta = max(j * pairs, t0), tb = min((j + 1) * pairs, t1);
+            const float *q = xb0 + (ta - t0) * kXchLd + 4 * u;
+            int n = tb - ta;
+            for (; n >= 4; n -= 4, q += 4 * kXchLd) {   // four loads in flight
+                double2 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const double2 *>(q + k * kXchLd);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    sA += v[k].x;
+                    sQ += v[k].y;
+                }
+            }
+            for (; n > 0; --n, q += kXchLd) {
+                const double2 v = *reinterpret_cast<const double2 *>(q);
+                sA += v.x;
+                sQ += v.y;
+            }
+            if (tb == (j + 1) * pairs) {
+                sA = row_sum(sA);
+                sQ = row_sum(sQ);
+                if (u == 0) norm[(size_t)p * S + shift_of(j)] = ring_norm(sA, sQ, R);
+                sA = sQ = 0.0;
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -2538,11 +2580,11 @@ __global__ void k_row_c2r(float *__restrict__ refs, int D, const float2 *__restr
 // Launch shape of the polar pass.  A workgroup's wavefronts take the row groups (four
 // shifts each) in equal passes: 13 groups run as 2 x 7, not 8 + 5.  Up to 8 wavefronts
 // where two workgroups fit in a CU's LDS, up to 16 where only one does.  With fewer
-// groups than the chip has wavefront slots (16 per CU), the ring pairs of a group are
-// split over wavefronts, one group per workgroup: 24 images of 64 x 64, 9 shifts, 29
-// rings take 21 us instead of 77.
+// groups than the chip has wavefront slots (16 per CU), a workgroup takes one group, its
+// ring pairs spread over the wavefronts: 24 images of 64 x 64, 9 shifts, 29 rings take 21 us
+// instead of 77.
 struct PolarShape {
-    int waves, split, groups_y;
+    int waves, rows, spread;
 };
 static int polar_wave_cap(int img_dim) {
     return 2 * polar_lds_floats(img_dim, 8) * sizeof(float) <= 160 * 1024 - 4096 ? 8 : 16;
@@ -2553,31 +2595,51 @@ static int polar_waves(int n_shift, int img_dim) {
     const int passes = (g + cap - 1) / cap;
     return (g + passes - 1) / passes;
 }
+// Cost of an image's n ring pairs of wavefronts by workgroups of nw wavefronts of which busy
+// have any: the vector unit's time, and more where fewer than nine of a CU's are busy (seven
+// of 128 x 128, 25 shifts: 11.6 ns a pair, nine to sixteen 9.4 to 9.9, three 21).
+static double polar_cost(int img_dim, int nw, int busy, double n) {
+    const int fit = (int)(160 * 1024 / (polar_lds_floats(img_dim, nw) * sizeof(float) + 512));
+    return n / std::min(1.0, busy * std::max(1, std::min(fit, 16 / nw)) / 9.0);
+}
+// Wavefronts of the spread form of n_rows rows, or 0 where `plain` unspread ones are the better
+// form: a spread pair costs 6 to 12 % more, by 25 and 49 shifts of 76 x 76.
+static int polar_spread(int n_rows, int img_dim, int n_ring, int plain) {
+    const long long pairs = (n_ring + 1) / 2, g = (n_rows + 3) / 4, tasks = n_rows * pairs;
+    int nw = 4;   // the smallest workgroup of which a CU holds 16 wavefronts
+    while (nw < 16 && 16 / nw * (polar_lds_floats(img_dim, nw) * sizeof(float) + 512) > 160 * 1024) nw *= 2;
+    if (tasks < 4 * nw) nw = tasks <= 16 ? (int)(tasks + 3) / 4 : (int)(tasks + 15) / 16 * 4;
+    const double spread = 1.06 * ((tasks + 4 * nw - 1) / (4 * nw) * nw);
+    return polar_cost(img_dim, nw, nw, spread) <
+                   0.95 * polar_cost(img_dim, plain, (int)std::min<long long>(g, plain), (double)(g * pairs))
+               ? nw
+               : 0;
+}
 static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_ring) {
     const int g = (n_shift + 3) / 4, pairs = (n_ring + 1) / 2;
     const long long fill = 4096 / (n_img * g);
     if (fill >= 2 && pairs >= 2) {
-        const int split = (int)std::min<long long>({fill, pairs, 16});
-        return {split, split, g};
+        const int split = (int)std::min<long long>({fill, (std::min(n_shift, 4) * pairs + 3) / 4, 16});
+        return {split, 4, 1};
     }
-    return {polar_waves(n_shift, img_dim), 1, 1};
+    const int plain = polar_waves(n_shift, img_dim), nw = polar_spread(n_shift, img_dim, n_ring, plain);
+    return {nw ? nw : plain, n_shift, nw > 0};
 }
 
 hipError_t prepare_launches() {
     static bool lds_raised = false;
     if (!lds_raised) {
-        const int lds = (int)(polar_lds_floats(kMaxImgDim, 16, 16) * sizeof(float));
+        const int lds = (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float));
         hipError_t e = hipFuncSetAttribute((const void *)k_ref_spectra, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(polar_lds_floats(kMaxImgDim, 16) * sizeof(float)));
         if (e != hipSuccess) return e;
         e = hipFuncSetAttribute((const void *)k_polar_single, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute((const void *)k_polar_spectra<false>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute((const void *)k_polar_spectra<true>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
+        for (const void *fn : {(const void *)k_polar_spectra<false, false>, (const void *)k_polar_spectra<false, true>,
+                               (const void *)k_polar_spectra<true, false>, (const void *)k_polar_spectra<true, true>}) {
+            e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+        }
         const int lds_frag = (int)((256 + 4 * 512) * sizeof(float2) +
                                    (kMaxImgDim + 2 * kFragBorder) * (kMaxImgDim + 2 * kFragBorder) *
                                        sizeof(float));
@@ -2599,9 +2661,10 @@ hipError_t launch_polar_spectra(const float *imgs, int n_img, int img_dim, Shift
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
     if (hipError_t e = prepare_launches()) return e;
     const PolarShape ps = polar_shape(n_img, n_shift, img_dim, n_ring);
-    const size_t lds = polar_lds_floats(img_dim, ps.waves, ps.split) * sizeof(float);
-    hipLaunchKernelGGL(k_polar_spectra<false>, dim3(n_img, ps.groups_y), dim3(64 * ps.waves), lds, st, imgs,
-                       img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, nullptr, ps.split);
+    const size_t lds = polar_lds_floats(img_dim, ps.waves) * sizeof(float);
+    const auto kernel = ps.spread ? k_polar_spectra<false, true> : k_polar_spectra<false, false>;
+    hipLaunchKernelGGL(kernel, dim3(n_img, (n_shift + ps.rows - 1) / ps.rows), dim3(64 * ps.waves), lds, st, imgs,
+                       img_dim, acc, shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, nullptr, ps.rows);
     return hipGetLastError();
 }
 
@@ -2633,17 +2696,20 @@ hipError_t launch_polar_spectra_masked(const float *imgs, int n_img, int img_dim
                                        const int2 *shift_i, int n_shift, const float2 *tmpl,
                                        int n_ring, const float2 *twiddle, float2 *spec,
                                        float2 *norm, const unsigned long long *smask,
-                                       hipStream_t st) {
+                                       int n_rows, hipStream_t st) {
     if (n_img <= 0 || n_shift <= 0) return hipSuccess;
     if (n_shift > 64) return hipErrorInvalidValue;
     if (hipError_t e = prepare_launches()) return e;
-    // unsplit, and as many wavefronts as fit: how many of a particle's shifts are set is
-    // not known here, and about 30 of 49 (8 windows) are one pass of 8 wavefronts but two
-    // of 7 (10 000 images of 76 x 76: 3.9 ms against 4.1)
-    const int waves = std::min((n_shift + 3) / 4, polar_wave_cap(img_dim));
-    const size_t lds = polar_lds_floats(img_dim, waves) * sizeof(float);
-    hipLaunchKernelGGL(k_polar_spectra<true>, dim3(n_img), dim3(64 * waves), lds, st, imgs, img_dim, acc,
-                       shift_i, n_shift, tmpl, n_ring, twiddle, spec, norm, smask, 1);
+    // as many wavefronts as fit: how many of a particle's shifts are set is not known here,
+    // and about 30 of 49 (8 windows) are one pass of 8 wavefronts but two of 7 (10 000 images
+    // of 76 x 76: 3.9 ms against 4.1).  About 9 (one window) spread: 1.20 ms, unspread 1.73
+    const int plain = std::min((n_shift + 3) / 4, polar_wave_cap(img_dim));
+    const int nw = polar_spread(n_rows, img_dim, n_ring, plain);
+    const PolarShape ps{nw ? nw : plain, n_shift, nw > 0};
+    const size_t lds = polar_lds_floats(img_dim, ps.waves) * sizeof(float);
+    const auto kernel = ps.spread ? k_polar_spectra<true, true> : k_polar_spectra<true, false>;
+    hipLaunchKernelGGL(kernel, dim3(n_img), dim3(64 * ps.waves), lds, st, imgs, img_dim, acc, shift_i, n_shift, tmpl,
+                       n_ring, twiddle, spec, norm, smask, n_shift);
     return hipGetLastError();
 }
 
