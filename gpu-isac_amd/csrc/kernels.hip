@@ -1044,52 +1044,51 @@ __device__ __forceinline__ void write_rec(PeakRec *o, const PeakState &st, const
 
 constexpr float kNoPeak = -3.40282e+38f;
 
-// A lane's two slots of a ring row: k = u + 16 (4 mh + 2 jp) and k + 16, with
-// (mh, jp) = lane row; two 8-byte loads per row.
-__device__ __forceinline__ int lane_slot(int lane) { return (lane & 15) + 64 * (lane >> 5) + 32 * ((lane >> 4) & 1); }
-__device__ __forceinline__ void load_pair(const float2 *row, int lane, float2 &re, float2 &im) {
-    const float2 *q = row + (lane >> 5) * 64 + (lane & 15) * 4 + ((lane >> 4) & 1);
-    re = q[0];
-    im = q[kPartOff / 2];
+// value of the neighbouring lane (lane ^ 1)
+__device__ __forceinline__ float dpp_xor1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
 }
 
-// Products of one reference's lane slots (br, bi) with a row's: P1..P4 = rr sr, ri si,
-// rr si, ri sr of both slots, summed over rings
-__device__ __forceinline__ void pair_fma(float (&acc)[2][4], float2 br, float2 bi, float2 ar, float2 ai) {
-    acc[0][0] += br.x * ar.x;
-    acc[0][1] += bi.x * ai.x;
-    acc[0][2] += br.x * ai.x;
-    acc[0][3] += bi.x * ar.x;
-    acc[1][0] += br.y * ar.y;
-    acc[1][1] += bi.y * ai.y;
-    acc[1][2] += br.y * ai.y;
-    acc[1][3] += bi.y * ar.y;
+// A lane's 16 bytes of a ring row: one part (real in even lanes) of the four slots
+// (lane >> 1 & 15) + 64 (lane >> 5) + 16 j.
+__device__ __forceinline__ float4 load_part(const float2 *row, int lane) {
+    return reinterpret_cast<const float4 *>(row)[lane];
+}
+
+// Products of one reference's lane part b with a row's a, summed over rings: own part in
+// acc[0], the other one in acc[1].  Even lanes have P1 = rr sr and P3 = rr si of the four
+// slots, odd lanes P2 = ri si and P4 = ri sr.
+__device__ __forceinline__ void part_fma(float (&acc)[2][4], const float4 &b, const float4 &a) {
+    const float bv[4] = {b.x, b.y, b.z, b.w}, av[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        acc[0][j] = fmaf(bv[j], av[j], acc[0][j]);
+        acc[1][j] = fmaf(bv[j], dpp_xor1(av[j]), acc[1][j]);
+    }
 }
 
 // Z of one (shift row, reference) from the ring products, into LDS at the transform's
 // positions: C0 = R conj S = (P1 + P2, P4 - P3), C1 = conj(R S) = (P1 - P2, -(P3 + P4));
-// Z[k] = C0 + i C1, Z[256 - k] its Hermitian partner; slot 0 packs the real bins 0
-// (with the mean correction) and 128.  nm = (mu L, 1 / sd) scales the row, but for
-// Z[64..127], which ifft256_lane16 scales.
-__device__ __forceinline__ void store_pair_z(float2 *xb, const float (&acc)[2][4], float2 nm, float rs0, int lane) {
-    const int k0 = lane_slot(lane);
+// Z[k] = C0 + i C1 from even lanes, Z[256 - k] its Hermitian partner from odd ones; slot 0
+// packs the real bins 0 (with the mean correction) and 128.  nm = (mu L, 1 / sd) scales the
+// row, but for Z[64..127], which ifft256_head scales.
+__device__ __forceinline__ void store_part_z(float2 *xb, const float (&acc)[2][4], float2 nm, float rs0, int lane) {
+    const bool odd = lane & 1;
+    const int k0 = ((lane >> 1) & 15) + 64 * (lane >> 5);
+    const float gz = odd || lane < 32 ? nm.y : 1.0f;
+    float2 *o = xb + (odd ? kMirOff : 0) + k0;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int k = k0 + 16 * h;
-        const float a = acc[h][0] + acc[h][1], e = acc[h][2] + acc[h][3];
-        const float c = acc[h][0] - acc[h][1], b = acc[h][3] - acc[h][2];
-        const float gz = lane < 32 ? nm.y : 1.0f;   // lane rows 2, 3: slots 64..127
-        float2 z = f2(gz * (a + e), gz * (b + c)), y = f2(nm.y * (a - e), nm.y * (c - b));
-        int ky = kMirOff + k;
-        if (h == 0 && lane == 0) {
-            const float c0 = nm.y * fmaf(-nm.x, rs0, acc[0][0]);
-            const float cn = nm.y * acc[0][1];
-            z = f2(c0, c0);
-            y = f2(cn, cn);
-            ky = kMirOff + 128;
+    for (int j = 0; j < 4; ++j) {
+        const float o0 = dpp_xor1(acc[0][j]), o1 = dpp_xor1(acc[1][j]);
+        const float a = acc[0][j] + o0, e = acc[1][j] + o1;
+        const float c = odd ? o0 - acc[0][j] : acc[0][j] - o0, b = odd ? acc[1][j] - o1 : o1 - acc[1][j];
+        float2 z = odd ? f2(gz * (a - e), gz * (c - b)) : f2(gz * (a + e), gz * (b + c));
+        if (j == 0 && lane < 2) {
+            const float v = nm.y * (odd ? acc[0][0] : fmaf(-nm.x, rs0, acc[0][0]));
+            xb[odd ? kMirOff + 128 : 0] = f2(v, v);
+            continue;
         }
-        xb[k] = z;
-        xb[ky] = y;
+        o[16 * j] = z;
     }
 }
 
@@ -1136,20 +1135,20 @@ __global__ __launch_bounds__(256) void k_ccf_single(
         for (int r = 0; r < 4; ++r)
             arow[r] = spec + (size_t)p * img_stride + (size_t)min(s0 + r, S - 1) * R * kSlots;
         for (int i = 0; i < R; ++i) {
-            float2 br, bi, ar[4], ai[4];
-            load_pair(rb0 + i * kSlots, lane, br, bi);
+            const float4 b = load_part(rb0 + i * kSlots, lane);
+            float4 a[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) load_pair(arow[r] + i * kSlots, lane, ar[r], ai[r]);
+            for (int r = 0; r < 4; ++r) a[r] = load_part(arow[r] + i * kSlots, lane);
             __builtin_amdgcn_sched_barrier(0);   // all of the ring's loads in flight before the FMAs
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pair_fma(acc[r], br, bi, ar[r], ai[r]);
+            for (int r = 0; r < 4; ++r) part_fma(acc[r], b, a[r]);
         }
         wave_lds_sync();
         float2 nm[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             nm[r] = norm[(size_t)p * S + min(s0 + r, S - 1)];
-            store_pair_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
+            store_part_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
         }
         wave_lds_sync();
         float2 x[16];
@@ -1478,11 +1477,6 @@ struct MrefLds {
     float nb[kMrefRefs][2][8];        // seven samples around the running maxima
 };
 
-// value of the neighbouring lane (lane ^ 1)
-__device__ __forceinline__ float dpp_xor1(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
-}
-
 // f(0), f(1), .., f(N - 1) with compile-time arguments
 template <class F, int... I>
 __device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
@@ -1798,18 +1792,24 @@ __global__ void k_prop_items(const int4 *__restrict__ prop, int n_img, int K, in
 }
 
 // One wavefront per item: the shifts of the item's (2 hw + 1)^2 window (in
-// increasing grid order) three at a time against its reference, with exactly
+// increasing grid order) NROW at a time against its reference, with exactly
 // the arithmetic of the exhaustive kernels (ring contraction, psi FFT), the
 // maximum taken over the item's (mirror, psi) mask only.  Workgroup = one
 // particle's K <= 8 items (K wavefronts), so the spectrum rows its windows share
 // are read through one CU and one L2.
+// What bounds it: the loads of the contraction, one 16-byte load a row and ring (10 000 x 8
+// items of 76 x 76, 9 shifts, 34 rings: 2.97 ms; two 8-byte loads 3.22), and the vector work
+// of the psi transforms; LDS for K items only lets more workgroups share a CU where they are
+// few (10 000 x 1 item of one shift: 0.46 -> 0.11 ms, with NROW = 1 for windows of one shift).
+template <int NROW>
 __global__ __launch_bounds__(512) void k_ccf_prop(
     const float2 *__restrict__ spec, const float2 *__restrict__ norm,
     const float2 *__restrict__ rspec, const float *__restrict__ rsum0,
     const PropItem *__restrict__ items, int K, int n_items, int S, int R, int N, int nx, int ny,
     int hw, const float2 *__restrict__ twg, PeakRec *__restrict__ rec) {
+    extern __shared__ float4 smem4[];
+    float2 (*fbuf)[4 * kFftLd] = reinterpret_cast<float2 (*)[4 * kFftLd]>(smem4);   // [K]
     __shared__ float2 tw[kIfftTw];
-    __shared__ float2 fbuf[kMaxProposals][4 * kFftLd];
     __shared__ float nbuf[kMaxProposals][2][8];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     fill_ifft_twiddles(tw, twg, tid, blockDim.x);
@@ -1839,40 +1839,43 @@ __global__ __launch_bounds__(512) void k_ccf_prop(
         const float2 *rb0 = rspec + (size_t)n * R * kSlots;
         const size_t img_stride = (size_t)S * R * kSlots;
         float2 *xb = fbuf[wave] + (lane >> 4) * kFftLd;
-        for (int r0 = 0; r0 < nr; r0 += 3) {
-            float acc[3][2][4];
+        for (int r0 = 0; r0 < nr; r0 += NROW) {
+            float acc[NROW][2][4];
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
+            for (int r = 0; r < NROW; ++r)
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[r][h][e] = 0.0f;
-            const float2 *arow[3];
+            const float2 *arow[NROW];
 #pragma unroll
-            for (int r = 0; r < 3; ++r)
+            for (int r = 0; r < NROW; ++r)
                 arow[r] = spec + (size_t)p * img_stride + (size_t)row(min(r0 + r, nr - 1)) * R * kSlots;
             for (int i = 0; i < R; ++i) {
-                float2 br, bi, ar[3], ai[3];
-                load_pair(rb0 + i * kSlots, lane, br, bi);
+                const float4 b = load_part(rb0 + i * kSlots, lane);
+                float4 a[NROW];
 #pragma unroll
-                for (int r = 0; r < 3; ++r) load_pair(arow[r] + i * kSlots, lane, ar[r], ai[r]);
+                for (int r = 0; r < NROW; ++r) a[r] = load_part(arow[r] + i * kSlots, lane);
                 __builtin_amdgcn_sched_barrier(0);   // all of the ring's loads in flight before the FMAs
 #pragma unroll
-                for (int r = 0; r < 3; ++r) pair_fma(acc[r], br, bi, ar[r], ai[r]);
+                for (int r = 0; r < NROW; ++r) part_fma(acc[r], b, a[r]);
             }
             wave_lds_sync();
-            float2 nm[3];
+            float2 nm[NROW];
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
+            for (int r = 0; r < NROW; ++r) {
                 nm[r] = norm[(size_t)p * S + row(min(r0 + r, nr - 1))];
-                store_pair_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
+                store_part_z(fbuf[wave] + r * kFftLd, acc[r], nm[r], rs0, lane);
             }
             wave_lds_sync();
             float2 x[16];
-            ifft256_rows4(x, lane_row_of(nm[0].y, nm[1].y, nm[2].y, 0.0f, lane), xb, tw, u);
-            // window rows are not consecutive shifts: one at a time
-            for (int r = 0; r < min(3, nr - r0); ++r)
-                peak_update<false, true>(st, x, r, 1, row(r0 + r), lane, xb, nbuf[wave], allow);
+            ifft256_rows4(x, lane_row_of(nm[0].y, nm[NROW / 2].y, nm[NROW - 1].y, 0.0f, lane), xb, tw, u);
+            // a window's rows are consecutive shifts up to the end of its column
+            for (int r = 0; r < min(NROW, nr - r0);) {
+                const int cnt = min(min(NROW, nr - r0) - r, wy - (r0 + r) % wy);
+                peak_update<false, true>(st, x, r, cnt, row(r0 + r), lane, xb, nbuf[wave], allow);
+                r += cnt;
+            }
         }
     }
     write_rec(rec + item, st, nbuf[wave], lane);
@@ -2626,6 +2629,8 @@ static PolarShape polar_shape(long long n_img, int n_shift, int img_dim, int n_r
     return {nw ? nw : plain, n_shift, nw > 0};
 }
 
+constexpr int kPropLds = 4 * kFftLd * sizeof(float2);   // of k_ccf_prop, a proposal
+
 hipError_t prepare_launches() {
     static bool lds_raised = false;
     if (!lds_raised) {
@@ -2638,6 +2643,10 @@ hipError_t prepare_launches() {
         for (const void *fn : {(const void *)k_polar_spectra<false, false>, (const void *)k_polar_spectra<false, true>,
                                (const void *)k_polar_spectra<true, false>, (const void *)k_polar_spectra<true, true>}) {
             e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+            if (e != hipSuccess) return e;
+        }
+        for (const void *fn : {(const void *)k_ccf_prop<1>, (const void *)k_ccf_prop<3>}) {
+            e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxProposals * kPropLds);
             if (e != hipSuccess) return e;
         }
         const int lds_frag = (int)((256 + 4 * 512) * sizeof(float2) +
@@ -3017,8 +3026,9 @@ hipError_t launch_ccf_prop(const float2 *spec, const float2 *norm, const float2 
     const int n_items = n_img * K;
     if (n_items <= 0) return hipSuccess;
     if (K < 1 || K > kMaxProposals) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_ccf_prop, dim3(n_img), dim3(64 * K), 0, st, spec, norm, rspec, rsum0,
-                       items, K, n_items, n_shift, n_ring, n_ref, nx, ny, hw, twiddle, rec);
+    if (hipError_t e = prepare_launches()) return e;
+    hipLaunchKernelGGL(hw > 0 ? k_ccf_prop<3> : k_ccf_prop<1>, dim3(n_img), dim3(64 * K), K * kPropLds, st, spec, norm,
+                       rspec, rsum0, items, K, n_items, n_shift, n_ring, n_ref, nx, ny, hw, twiddle, rec);
     return hipGetLastError();
 }
 
