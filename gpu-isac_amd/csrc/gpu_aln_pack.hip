@@ -668,7 +668,7 @@ int run_single(const float *d_sbj, DevParam *prm, const int *ref_of, int ref_str
     if (int e = ensure_template(R)) return e;
     if (int e = ensure_shifts(shifts)) return e;
     if (int e = ref_spectra(d_ref, N, D, R, st)) return e;
-    if (isac::polar_single_fills(cnt, S)) {
+    if (isac::polar_single_fills(cnt, S, D)) {
         HIP_OK(ws.rec.reserve((size_t)cnt * sizeof(PeakRec)));
         HIP_OK(isac::launch_polar_single(d_sbj, cnt, D, {&prm[0].shift_x, (int)(sizeof(DevParam) / sizeof(float))},
                                          ws.shifts_i.as<int2>(), S, ws.tmpl.as<float2>(), R,

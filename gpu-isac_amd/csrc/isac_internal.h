@@ -180,7 +180,7 @@ hipError_t launch_polar_single(const float *imgs, int n_img, int img_dim, ShiftV
                                int n_shift, const float2 *tmpl, int n_ring, const float2 *twiddle,
                                const float2 *rspec, const float *rsum0, const int *ref_of, int ref_stride, int n_ref,
                                PeakRec *rec, hipStream_t st);
-bool polar_single_fills(int n_img, int n_shift);
+bool polar_single_fills(int n_img, int n_shift, int img_dim);
 
 // Exact FP32 re-scoring of K candidate references per particle (ref cand[p*K+k];
 // a negative entry gives an empty record), same arithmetic as launch_ccf_mref;

@@ -2840,14 +2840,19 @@ hipError_t launch_polar_single(const float *imgs, int n_img, int img_dim, ShiftV
     return hipSuccess;
 }
 
-// One pass does a group of four shifts in one wavefront; two passes split the rings of few
+// One pass does a group of four shifts in one wavefront; two passes spread the rings of few
 // groups over wavefronts.  Pre-alignment of 76 x 76 images, 34 rings, three iterations, one
 // pass / two (us): 49 shifts, 5 images 512 / 585, 155 images 662 / 1145, 5000 images 12700 /
 // 18900; 9 shifts, 30 images 340 / 292, 150 images 455 / 457, 600 images 776 / 898; 1 shift,
-// 600 images 759 / 634.  128 x 128, 61 rings, 9 shifts: 150 images 650 / 594, 600 images
-// 1598 / 1674.
-bool polar_single_fills(int n_img, int n_shift) {
-    return n_shift > 12 || (n_shift >= 4 && (long long)n_img * ((n_shift + 3) / 4) >= 1024);
+// 600 images 759 / 634.  Two iterations of 25 shifts: 600 images of 76 x 76 1494 / 1985, 3000
+// of 128 x 128 8729 / 8952.  Where a CU holds one workgroup of the few wavefronts of 4 to 12
+// shifts, the spread form is the better one for all but few images: 128 x 128, 9 shifts, 500
+// images 2064 / 2310, 600 2581 / 2557, 800 3160 / 2250, 2000 5764 / 3855; with two a CU they
+// are within 7 % (118 x 118, 1500 images 2843 / 2853).
+bool polar_single_fills(int n_img, int n_shift, int img_dim) {
+    const long long groups = (long long)n_img * ((n_shift + 3) / 4);
+    const bool two = 2 * (polar_lds_floats(img_dim, polar_waves(n_shift, img_dim)) * sizeof(float) + 4096) <= 160 * 1024;
+    return n_shift > 12 || (n_shift >= 4 && groups >= 1024 && (two || groups < 2048));
 }
 
 hipError_t launch_ccf_candidates(const float2 *spec, const float2 *norm, const float2 *rspec,

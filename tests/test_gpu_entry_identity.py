@@ -56,7 +56,7 @@ def test_entries_give_the_same_bits(gpu, P, N, D, R, rng, kind):
 
 
 @pytest.mark.parametrize("kind", ["offset", "constant"])
-@pytest.mark.parametrize("P,D,R", [(700, 40, 9), (350, 96, 44)])
+@pytest.mark.parametrize("P,D,R", [(700, 40, 9), (350, 96, 44), (490, 128, 61)])
 def test_single_routes_give_the_same_bits(gpu, P, D, R, kind):
     """All images in one pass from the pixels, sevenths of them through ring spectra in memory."""
     x, ref = _images(kind, P, D, P + R), _images("offset", 3, D, R)
