@@ -1468,8 +1468,22 @@ constexpr int kRefPre = 2;        // and of the references' rings past the resid
 // with none, 13.5 with 4, 14.3 with 6, 15.0 with 8 (a wavefront has 128 registers)
 constexpr int kMrefKeep = 4;
 
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// Loads through a job's pointers.  The queue kernel reads them from memory, where nothing
+// says that they are global, and a flat load also holds the LDS counter.
+#define GLOBAL_AS __attribute__((address_space(1)))
+typedef GLOBAL_AS char global_char;
+template <class T>
+__device__ __forceinline__ T load_global(const T *p) {
+    return *(const GLOBAL_AS T *)p;
+}
+__device__ __forceinline__ float2 load_global2(const float2 *p) {
+    const f32x2_t v = *(const GLOBAL_AS f32x2_t *)p;
+    return f2(v.x, v.y);
+}
 
 struct MrefLds {
     float2 z[64 * kFftLd];            // transform (reference n, row r) at n + 8 r
@@ -1498,9 +1512,9 @@ __device__ __forceinline__ int mref_ref_at(const MrefJob &j, int p0, int g, int 
 // Contraction wavefront w of a run.  KR: rings of the references kept in registers (at
 // most R).
 template <bool LIST, int KR>
-__device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, int np, int g, MrefLds &sh) {
+__device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int lane, int p0, int np, int g,
+                                              MrefLds &sh) {
     const int S = j.S, R = j.R, N = j.N;
-    const int lane = threadIdx.x & 63;
     const int f = lane >> 4, u = lane & 15;
     const int ps = (LIST && j.pidx) ? j.pidx[p0] : p0;   // spectra row of the first particle
     const int n_rows = np * S;
@@ -1516,8 +1530,8 @@ __device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, i
     const float sgn = part ? -1.0f : 1.0f;
     // the host validates candidate ids; the clamp keeps every read in bounds
     const int ref = min(max(mref_ref_at<LIST>(j, p0, g, t), 0), N - 1);
-    const char *bp = reinterpret_cast<const char *>(j.rspec) + (size_t)ref * row_bytes + ring_off;
-    const float rs0 = j.rsum0[ref];
+    const global_char *bp = (const global_char *)j.rspec + (size_t)ref * row_bytes + ring_off;
+    const float rs0 = load_global<float>(j.rsum0 + ref);
 
     // LDS positions: this lane's Z values (reference t, row f or 4 + f; even lanes Z[k],
     // odd lanes Z[256 - k]) of its wavefront's slots 16 (4 mh + jj) + 4 uq + b, w = 4 mh + uq
@@ -1527,7 +1541,7 @@ __device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, i
     unsigned aoff = (unsigned)min(ar, n_rows - 1) * row_bytes + ring_off;
     f32x4_t keep[KR > 0 ? KR : 1], rb[kRefPre], ra[kMrefPre];
     auto load_b = [&](int i) {
-        return *reinterpret_cast<const f32x4_t *>(bp + (size_t)(unsigned)min(i, R - 1) * (kSlots * 8));
+        return *(const GLOBAL_AS f32x4_t *)(bp + (size_t)(unsigned)min(i, R - 1) * (kSlots * 8));
     };
     auto load_a = [&](int i) {
         const __amdgpu_buffer_rsrc_t rs =
@@ -1541,7 +1555,7 @@ __device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, i
         float2 nm[2];
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
-            nm[hh] = j.norm[(size_t)ps * S + 8 * (size_t)blk + min(4 * hh + f, n_rows - 1 - 8 * blk)];
+            nm[hh] = load_global2(j.norm + ((size_t)ps * S + 8 * (size_t)blk + min(4 * hh + f, n_rows - 1 - 8 * blk)));
         static_for<kRefPre>([&](auto dc) { rb[decltype(dc)::value] = load_b(KR + decltype(dc)::value); });
 
         f32x16_t acc[4] = {};
@@ -1609,9 +1623,8 @@ __device__ __forceinline__ void mref_contract(const MrefJob &j, int w, int p0, i
 
 // Psi wavefront c of a run: column c of the tile.
 template <bool LIST>
-__device__ __forceinline__ void mref_psi(const MrefJob &j, int c, int p0, int np, int g, MrefLds &sh) {
+__device__ __forceinline__ void mref_psi(const MrefJob &j, int c, int lane, int p0, int np, int g, MrefLds &sh) {
     const int S = j.S;
-    const int lane = threadIdx.x & 63;
     const int f = lane >> 4, u = lane & 15;
     const int ps = (LIST && j.pidx) ? j.pidx[p0] : p0;
     const int n_rows = np * S;
@@ -1623,7 +1636,8 @@ __device__ __forceinline__ void mref_psi(const MrefJob &j, int c, int p0, int np
     for (int blk = 0; blk < n_blk; ++blk) {
         const int rows = min(8, n_rows - 8 * blk);
         const size_t row0 = (size_t)ps * S + 8 * (size_t)blk;
-        const float gs0 = j.norm[row0 + min(f, rows - 1)].y, gs1 = j.norm[row0 + min(4 + f, rows - 1)].y;
+        const float gs0 = load_global2(j.norm + (row0 + min(f, rows - 1))).y;
+        const float gs1 = load_global2(j.norm + (row0 + min(4 + f, rows - 1))).y;
         __syncthreads();   // the contraction of this block is done
         __syncthreads();   // and its cross-spectra are in LDS
         if (ref < 0) continue;   // uniform over the wavefront
@@ -1658,10 +1672,10 @@ __device__ __forceinline__ void mref_psi(const MrefJob &j, int c, int p0, int np
 // references against its particle; every slot of the list gets a record, and each listed
 // reference's record is the one the exhaustive form computes for it.
 template <bool LIST, int KR>
-__device__ __forceinline__ void mref_run(const MrefJob &j, int p0, int np, int g, MrefLds &sh) {
-    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if (w < 8) mref_contract<LIST, KR>(j, w, p0, np, g, sh);
-    else mref_psi<LIST>(j, w - 8, p0, np, g, sh);
+__device__ __forceinline__ void mref_run(const MrefJob &j, int tid, int p0, int np, int g, MrefLds &sh) {
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    if (w < 8) mref_contract<LIST, KR>(j, w, lane, p0, np, g, sh);
+    else mref_psi<LIST>(j, w - 8, lane, p0, np, g, sh);
 }
 
 // Logical block = run of cp particles x reference tile (fastest).
@@ -1674,7 +1688,7 @@ __global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_mref(MrefJob j, int 
     const int ng = (j.N + kMrefRefs - 1) / kMrefRefs;
     const int p0 = lb / ng * cp;
     if (p0 >= j.n_img) return;  // uniform over the workgroup
-    mref_run<false, KR>(j, p0, min(cp, j.n_img - p0), lb % ng, sh);
+    mref_run<false, KR>(j, threadIdx.x, p0, min(cp, j.n_img - p0), lb % ng, sh);
 }
 
 // Candidate re-scoring (the candidate form of MrefJob) by the exhaustive kernel's
@@ -1683,7 +1697,7 @@ template <int KR>
 __global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_cand(MrefJob j, const float2 *__restrict__ twg) {
     __shared__ MrefLds sh;
     fill_ifft_twiddles(sh.tw, twg, threadIdx.x, kMrefWaves * 64);
-    mref_run<true, KR>(j, blockIdx.x, 1, 0, sh);
+    mref_run<true, KR>(j, threadIdx.x, blockIdx.x, 1, 0, sh);
 }
 
 // Persistent form over many jobs (batched subsets): work items (job, first particle,
@@ -1705,10 +1719,15 @@ __global__ __launch_bounds__(kMrefWaves * 64, 4) void k_ccf_mref_queue(
         __syncthreads();
         if (threadIdx.x == 0) claim = atomicAdd(&counters[q], 1);
         __syncthreads();
-        const int idx = q0 + claim;
+        const int idx = q0 + __builtin_amdgcn_readfirstlane(claim);   // scalar, and what follows from it
         if (idx >= q1) break;
         const int4 it = items[idx];
-        mref_run<false, KR>(jobs[it.x], it.y, it.w, it.z, sh);
+        const MrefJob j = jobs[it.x];
+        // what follows from the lane is computed again for each item: kept over the loop it
+        // takes the registers of the resident rings
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        mref_run<false, KR>(j, tid, it.y, it.w, it.z, sh);
     }
 }
 
