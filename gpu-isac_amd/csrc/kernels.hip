@@ -1167,11 +1167,13 @@ __device__ __forceinline__ float mul_rn(float a, float b) {
 // Each image against its own reference ref_of[p * ref_stride], from the pixels: k_polar_spectra's
 // workgroup and wavefronts (one image, four shift rows at a time, a ring pair at a time), but
 // the spectra of a pair are contracted with the reference's at once, in the ring order and
-// operation order of k_ccf_single, and never leave the registers; then the psi transforms of
-// the four rows.  The wavefronts' first maxima are merged: larger value, then smaller shift.
-// What bounds it: vector instructions, as k_polar_spectra without its stores.  5000 images
+// operation order of k_ccf_single, and are never written out; then the psi transforms of the
+// four rows.  The wavefronts' first maxima are merged: larger value, then smaller shift.
+// What bounds it: vector instructions, as k_polar_spectra without its stores, and scratch: 61
+// of a lane's values do not fit the 128 registers of four wavefronts per SIMD.  5000 images
 // of 76 x 76, 34 rings, 49 and 9 shifts in turn: 2.1 ms a search; the two passes, with 8.6 GB
-// of spectra written and read at 49 shifts, took 3.3.
+// of spectra written and read at 49 shifts, took 3.3.  With the sums of a ring pair over
+// its lanes at once 9 values spill, and pre-alignment of these images took 13.3 ms for 12.7.
 __global__ __launch_bounds__(1024, 4) void k_polar_single(
     const float *__restrict__ imgs, int D, ShiftView acc, const int2 *__restrict__ shift_i, int S,
     const float2 *__restrict__ tmpl, int R, const float2 *__restrict__ twg, const float2 *__restrict__ rspec,

@@ -179,6 +179,15 @@ __device__ __forceinline__ void write_operand(unsigned char *row_base, int k, in
     }
 }
 
+// x gs as an FP32 value: rounded before it becomes an operand, not in one step with it (the
+// compiler makes v_fma_mixlo_f16 of a product and its conversion in some forms of the code and
+// not in others, and a peak between two equal samples then moves).
+__device__ __forceinline__ float scaled(float x, float gs) {
+    float v = x * gs;
+    asm("" : "+v"(v));
+    return v;
+}
+
 // Particle operands from the raw FP32 spectra.  Operand row p * S_pad + s holds spectra
 // row p * S + s; rows with s >= S or p >= n_img (padding) are zero.  Workgroup = one row:
 // a thread turns 8 rings of four slots (two 16-byte loads a ring, slot_re) into 16-byte
@@ -230,8 +239,8 @@ __global__ __launch_bounds__(256) void k_frag_rows(const float2 *__restrict__ sp
                 const float y = e == 0 ? im[j].x : e == 1 ? im[j].y : e == 2 ? im[j].z : im[j].w;
                 const bool in = 8 * c + j < R;
                 // slot 0: S[0] - mu L, S[128]
-                a[j] = to16<BF16>(in ? (k == 0 ? x - nm.x : x + y) * gs : 0.0f);
-                b[j] = to16<BF16>(in ? (k == 0 ? y : x - y) * gs : 0.0f);
+                a[j] = to16<BF16>(in ? scaled(k == 0 ? x - nm.x : x + y, gs) : 0.0f);
+                b[j] = to16<BF16>(in ? scaled(k == 0 ? y : x - y, gs) : 0.0f);
             }
             auto pack = [](const unsigned short (&v)[8]) {
                 return make_uint4(v[0] | ((unsigned)v[1] << 16), v[2] | ((unsigned)v[3] << 16),
