@@ -633,7 +633,7 @@ def main():
         "value_protocol": "device-resident: images already in HBM when the timed region starts "
                           "(isac_mref_align_device); host_abi below is the same search behind "
                           "the reference's host-pointer ABI with PCIe both ways",
-        "roofline": {"bound": "valu_fp32", "kernel": "k_ccf_mref (ring contraction + psi IFFT + search)",
+        "roofline": {"bound": "fp32_matrix_and_vector_issue", "kernel": "k_ccf_mref (ring contraction + psi IFFT + search)",
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS,
                      "traffic": traffic_per_launch(pairs_per_launch),
